@@ -46,6 +46,19 @@ __device__ __forceinline__ float fp8e4m3_to_f32(uint8_t b) {
     return __uint_as_float(s | ((e + 120u) << 23) | (m << 20));
 }
 
+// s mod D and k mod 3 of a step or window index (>= 0) in 32-bit arithmetic: the 64-bit
+// remainder is a sequence of well over a hundred instructions, and every workgroup
+// needs these before its first load of a window.
+__device__ __forceinline__ int32_t mod_ring(int64_t s, int32_t D) {
+    const uint32_t hi = (uint32_t)((uint64_t)s >> 32), lo = (uint32_t)s, d = (uint32_t)D;
+    if (hi == 0u) return (int32_t)(lo % d);
+    const uint32_t r32 = (0xFFFFFFFFu % d + 1u) % d;       // 2^32 mod D (D <= 128: no overflow below)
+    return (int32_t)(((hi % d) * r32 + lo % d) % d);
+}
+__device__ __forceinline__ int mod3(int64_t k) {           // 2^32 = 1 mod 3
+    return (int)(((uint32_t)((uint64_t)k >> 32) % 3u + (uint32_t)k % 3u) % 3u);
+}
+
 enum : int { T_RAW = 0, T_LIF0 = 1, T_POISSON = 2, T_LIF = 3, T_LIFE = 4, T_LIFB = 5 };
 
 // Registers of one neuron across the steps of a window.
@@ -242,7 +255,7 @@ __global__ __launch_bounds__(kNeuBlock) void k_neurons(NeuArgs a, int32_t off, i
     NState st;
     if (active) neuron_load(a, i, type, MODE == kRingClass, st, a.last);
     const bool integ = integrates(type);
-    int32_t slot = (int32_t)(s0 % a.D);
+    int32_t slot = mod_ring(s0, a.D);
     for (int32_t w = 0; w < nsteps; ++w) {
         const int32_t s = (int32_t)(s0 + w);
         bool fired = false;
@@ -551,7 +564,10 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
 // the tile's region) in its flag, one 64-bit word per tile kBarStride words apart
 // (a cache line each), and waits until every workgroup's flag holds at least
 // `epoch`, one flag per thread; with `cnt`, the counts of tiles [ct0, ct1) land in
-// cnt[h] (0 for the others).  The wait is bounded: past `limit` clock ticks, or
+// cnt[h] (0 for the others).  A poll is one load, back to back with the next (each a
+// round trip past the L2, the pace of the loop); the error word and the clock, a round
+// trip of their own, are read every 16th poll only.  The wait is bounded: past `limit`
+// clock ticks (counted from the first look at the clock), or
 // once another workgroup has reported a timeout, it sets *err and returns false,
 // so every workgroup leaves the kernel (the host turns *err into an error).
 __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g, uint32_t epoch, uint32_t count,
@@ -563,19 +579,19 @@ __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g,
     if (threadIdx.x == 0) st_agent64(&flag[(size_t)g * kStride64], ((uint64_t)count << 32) | epoch);
     int bad = 0;
     for (uint32_t h = threadIdx.x; h < G && !bad; h += blockDim.x) {
-        const uint64_t c0 = (uint64_t)wall_clock64();
         uint64_t v = ld_agent64(&flag[(size_t)h * kStride64]);
-        while ((int32_t)((uint32_t)v - epoch) < 0) {
-            if (ld_agent(err) != 0u) {
-                bad = 1;
-                break;
+        uint64_t c0 = 0;
+        for (uint32_t polls = 0; (int32_t)((uint32_t)v - epoch) < 0; ++polls) {
+            if ((polls & 15u) == 15u) {
+                const uint64_t c = (uint64_t)wall_clock64();
+                if (polls == 15u) c0 = c;
+                const bool late = c - c0 > limit;
+                if (late) st_agent(err, 1u);
+                if (late || ld_agent(err) != 0u) {
+                    bad = 1;
+                    break;
+                }
             }
-            if ((uint64_t)wall_clock64() - c0 > limit) {
-                st_agent(err, 1u);
-                bad = 1;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
             v = ld_agent64(&flag[(size_t)h * kStride64]);
         }
         if (cnt) cnt[h] = (h >= ct0 && h < ct1) ? (uint32_t)(v >> 32) : 0u;
@@ -756,7 +772,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         if constexpr (PW) asm volatile("" : "+v"(tid));
         const int64_t s0 = sbase + (int64_t)kw * nsteps;
         const int64_t kwin = wbase + kw;
-        const int bcur = (int)(kwin % 3), bprev = (int)((kwin + 2) % 3), bnext = (int)((kwin + 1) % 3);
+        const int bcur = mod3(kwin), bnext = bcur == 2 ? 0 : bcur + 1, bprev = bcur == 0 ? 2 : bcur - 1;
         // The previous window's list: its start step, spike count and this thread's
         // first entry.  In a launch's first window the window's index comes from ctl,
         // and the words of all three lists load with it (one round trip instead of
@@ -846,7 +862,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         // 0 before the first window; at most D (a network without synapses has D = 1
         // and windows of up to kMaxWindow steps)
         const int32_t nprev = (int32_t)min(s0 - sprev, (int64_t)D);
-        const int32_t rprev = (int32_t)(sprev % D);
+        const int32_t rprev = mod_ring(sprev, D);
         // metadata of list entry e: first slot of its sub-row in this tile, length |
         // ring slot of its spike step << 26, BF16 / FP8 row scale bits or (STDP)
         // the source's last spike before the window; kTStdpB: row scale bits |
@@ -857,7 +873,9 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             uint32_t o0, o1;
             if (a.offs16) { o0 = a.offs16[ob]; o1 = a.offs16[ob + 1]; }
             else { o0 = a.offs32[ob]; o1 = a.offs32[ob + 1]; }
-            const int32_t sD = (int32_t)((sprev + (int64_t)(ent >> 26)) % D);
+            // (a window is shorter than the ring wherever a spike has synapses)
+            int32_t sD = rprev + (int32_t)(ent >> 26);
+            sD -= sD >= D ? D : 0;
             // padded sub-rows: starts are multiples of kSubAlign, the low bits of the next
             // entry hold the padding
             constexpr uint32_t am = (uint32_t)kSubAlign - 1u;
@@ -1179,7 +1197,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         uint32_t* lsp = sp_beg;
         uint32_t* wbuf = a.win_buf + (size_t)bcur * a.win_stride + lbase;
         uint32_t* rgw = a.win_buf + (size_t)bcur * a.win_stride + (size_t)t0 * (size_t)a.window;   // (rgp)
-        const int32_t slot0 = (int32_t)(s0 % D);
+        const int32_t slot0 = mod_ring(s0, D);
         unsigned long long se_local = 0ull;
         for (int32_t j0 = 0; j0 < tn; j0 += bd) {
             // a wave without neurons here skips the steps (its instructions would still
@@ -1392,7 +1410,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         // 4. LDS -> ring slice, except the slots this window consumed (cleared above,
         // or never read for neurons that do not integrate); meanwhile the list's
         // offset comes back from the atomic above
-        if (!PW || kw + 1 == nw) ring_slice_out(ring, gring, D, tn, (int32_t)(s0 % D), nsteps, RW);
+        if (!PW || kw + 1 == nw) ring_slice_out(ring, gring, D, tn, slot0, nsteps, RW);
         __syncthreads();
         for (uint32_t k = (uint32_t)tid; k < ((rgp && !a.rec) ? 0u : nl); k += (uint32_t)bd) {
             const uint32_t ent = lsp[k];
