@@ -118,7 +118,7 @@ struct mgb_sim {
     int64_t* prow = nullptr;           // first slot of each padded row of syn16 / syn_t / w_t
     float* tile_cc = nullptr;          // CLASS kinds: class cache of each tile
     uint32_t* tile_ccls = nullptr;
-    uint8_t* tile_lean = nullptr;      // every neuron of the tile an LIFB neuron of its two classes
+    uint8_t* tile_in = nullptr;        // [G] 1: a synapse targets the tile
     float* w_t = nullptr;              // kTF32 / kTStdp / kTStdpB weights in tile order
     uint32_t* row_aux = nullptr;       // kTStdpB: row scale bits | has-plastic << 31 per source
     uint8_t* tile_pl = nullptr;        // kTStdpB: 1 per tile with a plastic in-synapse
@@ -478,6 +478,12 @@ mgb_status choose_tiles(mgb_sim* s, const mgb_opts* o, int32_t n, int32_t D, con
     MGB_TRY(dalloc_n(s, &s->tile_of, (size_t)n));
     MGB_HIP_TRY(hipMemcpyAsync(s->tile_of, tof.data(), 4 * (size_t)n, hipMemcpyHostToDevice, st));
     MGB_TRY(dalloc_n(s, &s->tile_seg, tseg.size()));
+    std::vector<uint8_t> tin(tseg.size(), 0);
+    for (size_t g = 0; g + 1 < tlo.size(); ++g)
+        for (int32_t t = tlo[g]; t < tlo[g + 1] && !tin[g]; ++t)
+            tin[g] = (indeg[t] | indeg[(size_t)n + t]) != 0u ? 1 : 0;
+    MGB_TRY(dalloc_n(s, &s->tile_in, tin.size()));
+    MGB_HIP_TRY(hipMemcpyAsync(s->tile_in, tin.data(), tin.size(), hipMemcpyHostToDevice, st));
     MGB_TRY(dalloc_n(s, &s->seg_lo, lo.size()));
     MGB_TRY(dalloc_n(s, &s->seg_tile0, tile0.size()));
     MGB_TRY(dalloc_n(s, &s->seg_kbase, kbase.size()));
@@ -1062,11 +1068,6 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
     MGB_TRY(dalloc_n(s, &s->cnt, np));
     MGB_HIP_TRY(hipMemsetAsync(s->ctl, 0, sizeof(Ctl), st));
     MGB_HIP_TRY(hipMemcpyAsync(s->type, h.type.data(), (size_t)n, hipMemcpyHostToDevice, st));
-    if (s->tiled && s->tile_cc) {
-        // CLASS kinds: which tiles hold only LIFB neurons of their two cached classes
-        MGB_TRY(dalloc_n(s, &s->tile_lean, (size_t)s->G));
-        MGB_HIP_TRY(launch_tile_lean(s->tile_lo, s->G, s->type, s->tbl, s->tile_lean, st));
-    }
     MGB_HIP_TRY(hipMemcpyAsync(s->cset, h.cset.data(), (size_t)n, hipMemcpyHostToDevice, st));
     MGB_HIP_TRY(hipMemcpyAsync(s->stream_idx, h.stream.data(), 2 * (size_t)n, hipMemcpyHostToDevice, st));
     MGB_HIP_TRY(hipMemcpyAsync(s->rate, h.rate.data(), 4 * (size_t)n, hipMemcpyHostToDevice, st));
@@ -1248,7 +1249,7 @@ void update_persist(mgb_sim* s) {
     if (stdp_kind(s->tkind) || s->persist_req == MGB_PERSIST_OFF || !s->bar) return;
     // per-tile list regions (the kernel's variant with them) when asked for, or by
     // default in networks large enough for windows of many spikes (in small ones the
-    // variant without them, which preloads the neuron state, is the faster), when one
+    // variant without them was the faster), when one
     // thread per tile can scan their counts and the counts fit in LDS beside the tile's
     // data with every workgroup still resident
     const bool want = s->persist_req == MGB_PERSIST_REGIONS ||
@@ -1285,7 +1286,7 @@ TiledArgs tiled_args(const mgb_sim* s) {
     a.tbl_off = s->tbl_off; a.seq = s->seq; a.tbl_w = s->tbl_w;
     a.row_ptr = s->row_ptr; a.syn_t = s->syn_t; a.syn16 = s->syn16; a.offs16 = s->offs16; a.offs32 = s->offs32;
     a.prow = s->prow;
-    a.tile_cc = s->tile_cc; a.tile_ccls = s->tile_ccls; a.tile_lean = s->tile_lean;
+    a.tile_cc = s->tile_cc; a.tile_ccls = s->tile_ccls; a.tile_in = s->tile_in;
     a.ring_t = s->ring_t; a.ring_slab = s->ring_slab; a.rw = s->trw;
     a.ctl = s->ctl; a.win_buf = s->win_buf; a.win_stride = s->win_stride;
     a.rec = s->rec; a.rec_cap = (uint64_t)s->rec_cap;

@@ -205,7 +205,7 @@ struct TiledArgs {
     const int64_t* prow;    // first slot of each padded row of syn16 / syn_t / w_t
     const float* tile_cc;   // CLASS kinds: [G][2][2][kClassCache] class cache of each tile (k_tile_ccache)
     const uint32_t* tile_ccls;   // [G][2] its classes
-    const uint8_t* tile_lean;    // [G] 1: every neuron an LIFB neuron of one of those classes
+    const uint8_t* tile_in;      // [G] 1: a synapse targets the tile
     uint32_t* ring_t;
     size_t ring_slab;       // words per tile in ring_t: RW * D * B rounded up to 16 bytes
     Ctl* ctl;
@@ -300,10 +300,6 @@ size_t tiled_lds_bytes(int D, int B, int kind, int rw, int lut_lds = 0);
 // Class cache of every tile of the CLASS kinds (cc [G][2][2][kClassCache], cls [G][2]).
 hipError_t launch_tile_ccache(const int32_t* tile_lo, int32_t G, const uint16_t* tbl, const uint32_t* tbl_off,
                               const float* seq, float* cc, uint32_t* cls, hipStream_t st);
-// lean[g] = 1 when every neuron of tile g is an LIFB neuron of one of the tile's two
-// cached classes (needs the neuron types, uploaded after the tiles are built).
-hipError_t launch_tile_lean(const int32_t* tile_lo, int32_t G, const uint8_t* type, const uint16_t* tbl,
-                            uint8_t* lean, hipStream_t st);
 // Workgroups of `block` threads of the fused kernel for `a` that one CU holds at once.
 int tiled_blocks_per_cu(const TiledArgs& a, int block, bool persistent = false);
 hipError_t launch_tiled(const TiledArgs& a, int32_t off, int32_t wk, int32_t nsteps, int block,

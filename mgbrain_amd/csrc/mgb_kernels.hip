@@ -18,6 +18,8 @@
 // Floating-point expressions follow the reference's source with the
 // contraction nvcc applies by default written as explicit fmaf(); the library
 // is built with -ffp-contract=off so nothing else is fused.
+#include <type_traits>
+
 #include "mgb_internal.h"
 #include "mgb_rng.h"
 
@@ -599,6 +601,78 @@ __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g,
     return __syncthreads_or(bad) == 0;
 }
 
+template <int N>
+using Int = std::integral_constant<int, N>;
+
+// Registers of one neuron of a tile across the windows of a launch: the state, the
+// constants of its type's update that every step needs, and what its spikes add up to.
+struct TNeu {
+    float V, Ie, Ii, c3, c4;
+    int32_t refr, refr_steps;
+    int32_t last, dcnt;          // last spike step; spikes since the state was loaded
+    int32_t deg;                 // out-degree
+    int32_t csl;                 // CLASS kinds: which of the tile's two cached classes (-1: neither)
+};
+
+template <int T, class A>
+__device__ __forceinline__ void tneu_load(const A& a, int i, bool class_tables, const uint32_t* ccls, TNeu& st,
+                                          const int32_t* last) {
+    const uint32_t cs = a.cset[i];
+    const uint32_t cl = class_tables ? (uint32_t)a.tbl[i] : 0u;
+    const int64_t r0 = a.row_ptr[i], r1 = a.row_ptr[i + 1];
+    st.V = a.V[i];
+    st.refr = a.refr[i];
+    if (T != T_LIFB) {
+        st.Ie = a.Ie[i];
+        st.Ii = a.Ii[i];
+    }
+    if (last) st.last = last[i];
+    const CSet& C = a.csets[cs];
+    st.c3 = C.c[3];
+    st.c4 = C.c[4];
+    st.refr_steps = __float_as_int(C.c[30]);
+    st.deg = (int32_t)(r1 - r0);
+    if (class_tables) st.csl = cl == ccls[0] ? 0 : (cl == ccls[1] ? 1 : -1);
+}
+
+// Steps [w0, w0 + NB) of a window for one neuron per lane (type T, uniform over the
+// tile), given their inputs: selects instead of branches, bit w0 + u of the result set
+// where step w0 + u fired.  (LIF: c12..c17 in k.)
+template <int T, int NB>
+__device__ __forceinline__ uint32_t tneu_steps(TNeu& st, const float (&be)[NB], const float (&bi)[NB],
+                                               const float* k) {
+    uint32_t m = 0u;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const bool ref = st.refr > 0;
+        bool fire;
+        if (T == T_LIFB) {                                           // mgcore.cu:164-196
+            fire = !ref && st.V >= st.c4;
+            const float vn = st.V + fmaf(-0.005f, st.V, be[u]);
+            st.V = fire ? st.c3 : (ref ? st.V : vn);
+        } else if (T == T_LIFE) {                                    // :197-233
+            st.Ie = fmaf(st.Ie, 0.98f, be[u]);
+            st.Ii = fmaf(st.Ii, 0.99f, -bi[u]);
+            fire = !ref && st.V >= st.c4;
+            const float t0 = -0.06f - st.V;
+            const float t1 = fmaf(st.Ie, 0.0f - st.V, t0);
+            const float t2 = fmaf(st.Ii, -0.08f - st.V, t1);
+            const float vn = fmaf(t2 + 0.02f, 0.005f, st.V);
+            st.V = fire ? st.c3 : (ref ? st.V : vn);
+        } else {                                                     // LIF :132-163
+            const float vn = fmaf(st.Ii, k[1], fmaf(st.Ie, k[0], fmaf(k[5], st.V, k[2])));
+            const float en = st.Ie * k[3], in = st.Ii * k[4];
+            fire = !ref && vn >= st.c4;
+            st.V = ref ? st.V : (fire ? st.c3 : vn);
+            st.Ie = ref ? st.Ie : (fire ? en : en + be[u]);
+            st.Ii = ref ? st.Ii : (fire ? in : in + bi[u]);
+        }
+        st.refr = fire ? st.refr_steps : (ref ? st.refr - 1 : st.refr);
+        m |= (fire ? 1u : 0u) << u;
+    }
+    return m;
+}
+
 // One window of the fused tiled step (CLASS format).  Workgroup g (targets
 // [tile_lo[g], tile_lo[g+1]) of segment tile_seg[g]):
 //   1. loads its ring slice ring_t[g] (D x B words) into LDS;
@@ -742,8 +816,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     uint32_t* rg_pre = reinterpret_cast<uint32_t*>(itm + kItems) + (kAux ? kTiledBatch : 0);
     uint32_t* rg_off = rg_pre + (PW ? a.G : 0);
     // (a variant of the persistent form of the 16-bit CLASS words only: in the other
-    // kinds' persistent forms the code alone, never run, cost their windows 5 %, and
-    // it keeps the neuron-state preload out of the variant, which would spill)
+    // kinds' persistent forms the code alone, never run, cost their windows 5 %)
     constexpr bool kRg = RG;
     const bool rgn_on = kRg && a.region != 0;
     if (rgn_on)
@@ -756,13 +829,42 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     // (thread 0) synaptic events and spikes of the windows that wrote regions, added
     // to the run's counters by the launch's last window
     unsigned long long se_acc = 0ull, spk_acc = 0ull;
-    // a tile of at most one neuron per thread: the neuron's state and out-degree are
-    // loaded at the start of each window (after the ring copy, which they would
-    // delay), their latency hidden by the propagation phase
-    // (not where registers would spill: with STDP at 16 synapses a work item or with
-    // BF16 static weights, in the persistent form of the 32-bit CLASS words and in the
-    // list-region variant)
-    const bool pre = !(kRg || (PW && WK == kTClass)) && tn <= bd && full && !(kPl && (CH >= 16 || kMix));
+    // the tile's neuron type (tiles never mix types) and whether any synapse targets it
+    const int ttype = (int)a.type[t0];
+    const bool integ = integrates(ttype);
+    const bool fed = a.tile_in[g] != 0;
+    // a tile of at most one neuron per thread: its state and constants stay in registers
+    // from the launch's first window to its last (TNeu: 11 registers at most), loaded
+    // once behind the ring copy and stored at the end.  Loading them in every window
+    // cost its neuron steps a chain of two loads (with the batched reads of the steps
+    // below: 80,000 conductance neurons 13.9 -> 10.3 us per window of 8 steps).
+    const bool own = tn <= bd && full;
+    TNeu own_st = {};
+    own_st.c4 = __int_as_float(0x7F800000);               // lanes without a neuron never fire
+    own_st.csl = 0;
+    auto load_neuron = [&](int32_t i, TNeu& st, const int32_t* last) {
+        if (ttype == T_LIFB) tneu_load<T_LIFB>(a, i, kCls, ccls, st, last);
+        else if (integ) tneu_load<T_LIF>(a, i, kCls, ccls, st, last);
+        else {
+            st.deg = (int32_t)(a.row_ptr[i + 1] - a.row_ptr[i]);
+            if (last) st.last = last[i];
+        }
+    };
+    // what a launch (or, for tiles of several neurons per thread, a window) leaves
+    auto store_neuron = [&](int32_t i, const TNeu& st) {
+        if (integ) {
+            a.V[i] = st.V;
+            a.refr[i] = st.refr;
+            if (ttype != T_LIFB) {
+                a.Ie[i] = st.Ie;
+                a.Ii[i] = st.Ii;
+            }
+        }
+        if (st.dcnt) {
+            a.cnt[i] += st.dcnt;
+            if (!kPl) a.last[i] = st.last;
+        }
+    };
     uint32_t* gring = a.ring_t + (size_t)g * a.ring_slab;
     for (int32_t kw = 0; kw < nw; ++kw) {
         // (persistent form: the thread index is opaque to the compiler in each window,
@@ -809,6 +911,11 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             sprev = bprev == 0 ? tb0 : (bprev == 1 ? tb1 : tb2);
             E = bprev == 0 ? n0 : (bprev == 1 ? n1 : n2);
             ent0 = bprev == 0 ? l0 : (bprev == 1 ? l1 : l2);
+            if (!fed) E = 0u;
+        } else if (!fed) {
+            sprev = s0 - nsteps;                        // no synapse targets the tile: no spike matters
+            E = 0u;
+            ent0 = 0u;
         } else if (rgc) {
             // the counts came with the wait (rg_pre); the list is laid out by their prefix
             sprev = s0 - nsteps;
@@ -898,17 +1005,15 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         constexpr bool kAhead = !kPl;
         uint32_t ent1 = 0u;
         if (kAhead && E > (uint32_t)bd && (uint32_t)tid < E - (uint32_t)bd) ent1 = lent((uint32_t)bd + (uint32_t)tid);
-        if (full && kw == 0) ring_slice_in(ring, gring, D, tn, rprev, nprev, RW);
-        NState pst;
-        int ptype = T_RAW;
-        int32_t pdeg = 0;
-        // CLASS kinds: every neuron of the tile (one per thread) an LIFB neuron of one of
-        // the tile's two cached classes (precomputed per tile)
-        const bool tile_lean = kCls && pre && a.tile_lean && a.tile_lean[g] != 0;
-        if (pre && tid < tn) {
-            ptype = (int)a.type[t0 + tid];
-            neuron_load(a, t0 + tid, ptype, kCls, pst, lastB);
-            if (ptype != T_RAW && ptype != T_LIF0) pdeg = (int32_t)(a.row_ptr[t0 + tid + 1] - a.row_ptr[t0 + tid]);
+        if (full && kw == 0) {
+            if (fed) ring_slice_in(ring, gring, D, tn, rprev, nprev, RW);
+            else if (integ)                             // (nothing ever arrives: all zero)
+                for (int32_t k = tid; k < RW * D * tn; k += bd) ring[k] = 0u;
+        }
+        if (own && kw == 0) {
+            // the class cache's classes are read by every thread below
+            if (kCls) __syncthreads();
+            if (tid < tn) load_neuron(t0 + tid, own_st, kPl ? lastB : nullptr);
         }
         __syncthreads();
 
@@ -1206,20 +1311,8 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             const int32_t j = j0 + tid;
             const bool active = j < tn;
             const int32_t i = t0 + j;
-            const int type = active ? (pre ? ptype : (int)a.type[i]) : T_RAW;
-            NState st;
-            int32_t outdeg = 0;
-            if (pre) {
-                st = pst;
-                outdeg = pdeg;
-            } else if (active) {
-                neuron_load(a, i, type, kCls, st, lastB);
-                if (type != T_RAW && type != T_LIF0) outdeg = (int32_t)(a.row_ptr[i + 1] - a.row_ptr[i]);
-            }
-            const bool integ = integrates(type);
-            // wave-uniform fast path: every active lane an LIFB neuron of a cached class
-            int32_t csl = -1;
-            if (kCls && active && integ) csl = (st.cls == ccls[0]) ? 0 : ((st.cls == ccls[1]) ? 1 : -1);
+            TNeu st = own_st;
+            if (!own && active) load_neuron(i, st, kPl ? lastB : nullptr);
             // spikes of step w: one wave ballot; the wave's leader reserves their places in
             // the LDS list (one LDS atomic per wave and step)
             auto append = [&](bool fired, int32_t w, int32_t s) {
@@ -1272,122 +1365,134 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 if (fired) {
                     const uint32_t r = lb + rank_below(m);
                     if (r < cap) lsp[r] = (uint32_t)i | ((uint32_t)w << 26);
-                    se_local += (unsigned long long)outdeg;
+                    se_local += (unsigned long long)st.deg;
                 }
             };
-            if (tile_lean) {
-                // every neuron an LIFB neuron of a cached class (tile_lean): the steps
-                // (mgcore.cu:164-196) as selects, the next step's ring word loaded ahead,
-                // spikes kept as a bit per step; the consumed rows are cleared and the
-                // spikes appended after the steps
-                const float* cc = &ccache[csl < 0 ? 0 : csl][0][0];
-                int32_t slot = slot0;
-                uint32_t x = active ? ring[slot * tn + j] : 0u;
-                uint64_t fmask = 0ull;
-                for (int32_t w = 0; w < nsteps; ++w) {
-                    const uint32_t ke = x & 0xFFFFu, ki = x >> 16;
-                    float be = cc[min(ke, (uint32_t)kClassCache - 1u)];
-                    float bi = cc[kClassCache + min(ki, (uint32_t)kClassCache - 1u)];
-                    if (ke >= (uint32_t)kClassCache) be = a.seq[st.off_e + ke];
-                    if (ki >= (uint32_t)kClassCache) bi = a.seq[st.off_i + ki];
+            // The window's steps, spikes kept as a bit per step.  The ring words of four
+            // steps (and their class sums) are read together, so that a step waits for its
+            // own arithmetic only (ten steps of a 250-neuron tile 3.5 -> 2.4 us).
+            uint64_t fmask = 0ull;
+            int32_t slot = slot0;
+            const int32_t jr = active ? j : 0;             // lanes past the tile read neuron 0's words
+            auto steps = [&](auto type, auto batch, int32_t w0, const float* k) {
+                constexpr int T = decltype(type)::value, NB = decltype(batch)::value;
+                uint32_t x[NB], y[NB];
+#pragma unroll
+                for (int u = 0; u < NB; ++u) {
+                    const int32_t at = slot * tn + jr;
+                    x[u] = ring[at];
+                    y[u] = (!kCls && RW == 2) ? ring[D * tn + at] : 0u;
+                    if (PW && active) {                     // clearInput (the slice stays in LDS)
+                        ring[at] = 0u;
+                        if (!kCls && RW == 2) ring[D * tn + at] = 0u;
+                    }
                     slot = (slot + 1 == D) ? 0 : slot + 1;
-                    x = (active && w + 1 < nsteps) ? ring[slot * tn + j] : 0u;
-                    const bool ref = st.refr > 0;
-                    const bool fire = active && !ref && st.V >= st.c4;
-                    const float vn = st.V + fmaf(-0.005f, st.V, be + bi);
-                    st.V = fire ? st.c3 : (ref ? st.V : vn);
-                    st.refr = fire ? st.refr_steps : (ref ? st.refr - 1 : st.refr);
-                    fmask |= (uint64_t)fire << w;
                 }
-                if (fmask) {
-                    st.cnt += __popcll(fmask);
-                    st.last = (int32_t)(s0 + 63 - __clzll((long long)fmask));
-                }
-                for (uint64_t fm = fmask; __any(fm != 0ull);) {   // one step's spikes per lane and pass
-                    const bool f = fm != 0ull;
-                    const int32_t w = f ? __ffsll((unsigned long long)fm) - 1 : 0;
-                    fm &= fm - 1ull;
-                    append(f, w, (int32_t)(s0 + w));
-                }
-            } else {
-                const bool lean = kCls && __all(!active || (type == T_LIFB && csl >= 0));
-                int32_t slot = slot0;
-                for (int32_t w = 0; w < nsteps; ++w) {
-                    const int32_t s = (int32_t)(s0 + w);
-                    bool fired = false;
+                float be[NB], bi[NB];
+                if (kCls) {
                     // class sums of a cached class: one LDS read per side (the table for
                     // counts past the cache)
-                    auto cached_input = [&](uint32_t x, float& be, float& bi) {
-                        const uint32_t ke = x & 0xFFFFu, ki = x >> 16;
-                        const float* cc = &ccache[csl][0][0];
-                        be = cc[min(ke, (uint32_t)kClassCache - 1u)];
-                        bi = cc[kClassCache + min(ki, (uint32_t)kClassCache - 1u)];
-                        if (ke >= (uint32_t)kClassCache) be = a.seq[st.off_e + ke];
-                        if (ki >= (uint32_t)kClassCache) bi = a.seq[st.off_i + ki];
-                    };
-                    if (lean) {
-                        if (active) {
-                            uint32_t* r = &ring[slot * tn + j];
-                            const uint32_t x = *r;
-                            *r = 0u;                                          // clearInput
-                            float be, bi;
-                            cached_input(x, be, bi);
-                            fired = integrate_lifb(st, s, be + bi);
+                    const float* cc = &ccache[st.csl < 0 ? 0 : st.csl][0][0];
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) {
+                        const uint32_t ke = x[u] & 0xFFFFu, ki = x[u] >> 16;
+                        be[u] = cc[min(ke, (uint32_t)kClassCache - 1u)];
+                        bi[u] = cc[kClassCache + min(ki, (uint32_t)kClassCache - 1u)];
+                    }
+                    uint32_t big = st.csl < 0 ? 1u : 0u;
+#pragma unroll
+                    for (int u = 0; u < NB; ++u)
+                        big |= ((x[u] & 0xFFFFu) >= (uint32_t)kClassCache || (x[u] >> 16) >= (uint32_t)kClassCache);
+                    if (big) {
+                        const uint32_t cl = a.tbl[t0 + jr];
+                        const float* se = a.seq + a.tbl_off[2 * cl];
+                        const float* si = a.seq + a.tbl_off[2 * cl + 1];
+#pragma unroll
+                        for (int u = 0; u < NB; ++u) {
+                            be[u] = se[x[u] & 0xFFFFu];
+                            bi[u] = si[x[u] >> 16];
                         }
-                    } else if (type == T_POISSON) {
-                        fired = poisson_step(st, s, w);
-                    } else if (integ) {
-                        float be, bi;
-                        uint32_t* r = &ring[slot * tn + j];
-                        if (kCls) {
-                            const uint32_t x = *r;
-                            *r = 0u;                                          // clearInput
-                            if (csl >= 0) cached_input(x, be, bi);
-                            else class_input(x, a.seq, st, be, bi);
-                        } else {
-                            uint32_t* ri = r + (size_t)D * tn;
-                            const int32_t qe = (int32_t)*r, qi = RW == 2 ? (int32_t)*ri : 0;
-                            *r = 0u;
-                            if (RW == 2) *ri = 0u;
-                            fixed_input(type, qe, qi, fsc.y, be, bi);
-                        }
-                        fired = integrate_step(type, st, s, be, bi);
                     }
-                    if (PW && active && !integ) {
-                        // the slice stays in LDS across windows: the consumed row of a neuron
-                        // that does not read its input is cleared here (a per-window launch
-                        // reloads consumed rows as zeros)
-                        ring[slot * tn + j] = 0u;
-                        if (!kCls && RW == 2) ring[((size_t)D + slot) * tn + j] = 0u;
-                    }
-                    if (kPl && fired) {
-                        // the history moves down one entry (the oldest drops out), in LDS and HBM
-                        int4* hq = reinterpret_cast<int4*>(hL + (size_t)j * kStdpHist);
-                        const int4 q0 = hq[0], q1 = hq[1], q2 = hq[2], q3 = hq[3];
-                        const int4 n0 = make_int4(s, q0.x, q0.y, q0.z), n1 = make_int4(q0.w, q1.x, q1.y, q1.z);
-                        const int4 n2 = make_int4(q1.w, q2.x, q2.y, q2.z), n3 = make_int4(q2.w, q3.x, q3.y, q3.z);
-                        hq[0] = n0; hq[1] = n1; hq[2] = n2; hq[3] = n3;
-                        int4* hg = reinterpret_cast<int4*>(a.hist + (size_t)i * kStdpHist);
-                        hg[0] = n0; hg[1] = n1; hg[2] = n2; hg[3] = n3;
-                    }
-                    append(fired, w, s);
-                    slot = (slot + 1 == D) ? 0 : slot + 1;
+                    if (T == T_LIFB)
+#pragma unroll
+                        for (int u = 0; u < NB; ++u) be[u] = be[u] + bi[u];
+                } else {
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) fixed_input(T, (int32_t)x[u], (int32_t)y[u], fsc.y, be[u], bi[u]);
                 }
+                fmask |= (uint64_t)tneu_steps<T, NB>(st, be, bi, k) << w0;
+            };
+            auto window = [&](auto type) {
+                float k[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                if (decltype(type)::value == T_LIF) {
+                    const CSet& C = a.csets[a.cset[t0 + jr]];
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) k[c] = C.c[12 + c];
+                }
+                int32_t w = 0;
+                for (; w + 4 <= nsteps; w += 4) steps(type, Int<4>{}, w, k);
+                if (w + 2 <= nsteps) {
+                    steps(type, Int<2>{}, w, k);
+                    w += 2;
+                }
+                if (w < nsteps) steps(type, Int<1>{}, w, k);
+            };
+            if (ttype == T_LIFB) {
+                window(Int<T_LIFB>{});
+            } else if (ttype == T_LIFE) {
+                window(Int<T_LIFE>{});
+            } else if (ttype == T_LIF) {
+                window(Int<T_LIF>{});
+            } else {
+                if (ttype == T_POISSON && active) {
+                    NState ps;
+                    const uint32_t sidx = a.stream ? a.stream[i] : 0u;
+                    ps.rate = a.rate[i];
+                    const uint64_t seed = a.stream_seed[sidx];
+                    ps.key0 = (uint32_t)seed;
+                    ps.key1 = (uint32_t)(seed >> 32);
+                    ps.lid = (uint32_t)(i - a.stream_base[sidx]);
+                    for (int32_t w = 0; w < nsteps; ++w)
+                        fmask |= (uint64_t)poisson_step(ps, (int32_t)(s0 + w), w) << w;
+                }
+                if (PW && fed && active)
+                    // the slice stays in LDS across windows: the consumed rows of a neuron
+                    // that does not read its input are cleared here (a per-window launch
+                    // reloads consumed rows as zeros)
+                    for (int32_t w = 0; w < min(nsteps, D); ++w) {
+                        ring[slot * tn + j] = 0u;
+                        if (!kCls && RW == 2) ring[(D + slot) * tn + j] = 0u;
+                        slot = (slot + 1 == D) ? 0 : slot + 1;
+                    }
             }
-            if (active) neuron_store(a, i, type, st, lastC);
+            if (!active) fmask = 0ull;
+            if (fmask) {
+                st.dcnt += __popcll(fmask);
+                st.last = (int32_t)(s0 + 63 - __clzll((long long)fmask));
+            }
+            for (uint64_t fm = fmask; __any(fm != 0ull);) {   // one step's spikes per lane and pass
+                const bool f = fm != 0ull;
+                const int32_t w = f ? __ffsll((unsigned long long)fm) - 1 : 0;
+                fm &= fm - 1ull;
+                if (kPl && f) {
+                    // the history moves down one entry (the oldest drops out), in LDS and HBM
+                    int4* hq = reinterpret_cast<int4*>(hL + (size_t)j * kStdpHist);
+                    const int4 q0 = hq[0], q1 = hq[1], q2 = hq[2], q3 = hq[3];
+                    const int4 n0 = make_int4((int32_t)(s0 + w), q0.x, q0.y, q0.z);
+                    const int4 n1 = make_int4(q0.w, q1.x, q1.y, q1.z);
+                    const int4 n2 = make_int4(q1.w, q2.x, q2.y, q2.z), n3 = make_int4(q2.w, q3.x, q3.y, q3.z);
+                    hq[0] = n0; hq[1] = n1; hq[2] = n2; hq[3] = n3;
+                    int4* hg = reinterpret_cast<int4*>(a.hist + (size_t)i * kStdpHist);
+                    hg[0] = n0; hg[1] = n1; hg[2] = n2; hg[3] = n3;
+                }
+                append(f, w, (int32_t)(s0 + w));
+            }
+            if (kPl && active) lastC[i] = st.last;
+            if (own) own_st = st;
+            else if (active) store_neuron(i, st);
         }
         if (se_local) atomicAdd(&se_blk, se_local);
         __syncthreads();
-        if (PW && tile_lean && kw + 1 < nw) {
-            // the lean steps leave the rows they consumed for here, after every wave's
-            // last read; the slice stays in LDS for the next window
-            const int32_t nr = min(nsteps, D);
-            int32_t sl = slot0;
-            for (int32_t r = 0; r < nr; ++r) {
-                for (int32_t jj = tid; jj < tn; jj += bd) ring[sl * tn + jj] = 0u;
-                sl = (sl + 1 == D) ? 0 : sl + 1;
-            }
-        }
         const uint32_t nl = min(lsp_n, (uint32_t)kTiledBatch);
         if (tid == 0) {
             if (rgp) {
@@ -1410,7 +1515,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         // 4. LDS -> ring slice, except the slots this window consumed (cleared above,
         // or never read for neurons that do not integrate); meanwhile the list's
         // offset comes back from the atomic above
-        if (!PW || kw + 1 == nw) ring_slice_out(ring, gring, D, tn, slot0, nsteps, RW);
+        if (fed && (!PW || kw + 1 == nw)) ring_slice_out(ring, gring, D, tn, slot0, nsteps, RW);
         __syncthreads();
         for (uint32_t k = (uint32_t)tid; k < ((rgp && !a.rec) ? 0u : nl); k += (uint32_t)bd) {
             const uint32_t ent = lsp[k];
@@ -1435,6 +1540,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 return;
         }
     }   // windows
+    if (own && tid0 < tn) store_neuron(t0 + tid0, own_st);
 }
 
 // Flush of deferred dendrite updates (fused STDP): for each neuron j the fused
@@ -1643,31 +1749,11 @@ __global__ void k_tile_ccache(const int32_t* tile_lo, const uint16_t* tbl, const
     if (side == 0 && k == 0) cls[2 * g + c] = cl;
 }
 
-// The class cache holds the classes of the tile's last and first neurons.
-__global__ void k_tile_lean(const int32_t* tile_lo, const uint8_t* type, const uint16_t* tbl, uint8_t* lean) {
-    const int32_t g = (int32_t)blockIdx.x, tid = (int32_t)threadIdx.x;
-    const int32_t t0 = tile_lo[g], t1 = tile_lo[g + 1];
-    const uint32_t cl0 = tbl[t1 - 1], cl1 = tbl[t0];
-    int ok = 1;
-    for (int32_t i = t0 + tid; i < t1; i += (int32_t)blockDim.x)
-        ok &= type[i] == T_LIFB && (tbl[i] == cl0 || tbl[i] == cl1);
-    ok = __syncthreads_and(ok);
-    if (tid == 0) lean[g] = ok ? 1 : 0;
-}
-
 hipError_t launch_tile_ccache(const int32_t* tile_lo, int32_t G, const uint16_t* tbl, const uint32_t* tbl_off,
                               const float* seq, float* cc, uint32_t* cls, hipStream_t st) {
     if (G <= 0) return hipSuccess;
     if (!tile_lo || !tbl || !tbl_off || !seq || !cc || !cls) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_tile_ccache, dim3(G), dim3(4 * kClassCache), 0, st, tile_lo, tbl, tbl_off, seq, cc, cls);
-    return hipGetLastError();
-}
-
-hipError_t launch_tile_lean(const int32_t* tile_lo, int32_t G, const uint8_t* type, const uint16_t* tbl,
-                            uint8_t* lean, hipStream_t st) {
-    if (G <= 0) return hipSuccess;
-    if (!tile_lo || !type || !tbl || !lean) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_tile_lean, dim3(G), dim3(256), 0, st, tile_lo, type, tbl, lean);
     return hipGetLastError();
 }
 
