@@ -257,8 +257,8 @@ struct TiledArgs {
     // tile's own part of the list (tile_lo * window on) and publish the count with the
     // wait's flag, instead of reserving list space with a returning global atomic
     int32_t region;
-    // persistent launches: one flag per tile (kBarStride words apart; a 64-bit word:
-    // window epoch | spike count << 32) for the wait between windows, its error word,
+    // persistent launches: one flag per tile (kBarStride words apart; two 64-bit words, for
+    // even and odd epochs: window epoch | spike count << 32) for the wait between windows, its error word,
     // and the wait's bound in wall-clock ticks
     uint32_t* bar;
     uint32_t* bar_err;

@@ -563,9 +563,12 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
 // waits for its own stores to complete (s_waitcnt vmcnt(0): the agent-scope
 // stores above are then visible at agent scope), then the workgroup publishes
 // `epoch` and `count` (the window's spikes of the tile, when its list went to
-// the tile's region) in its flag, one 64-bit word per tile kBarStride words apart
-// (a cache line each), and waits until every workgroup's flag holds at least
-// `epoch`, one flag per thread; with `cnt`, the counts of tiles [ct0, ct1) land in
+// the tile's region) in its flag, a pair of 64-bit words per tile kBarStride words apart
+// (a cache line each), even epochs in the first and odd ones in the second, and waits
+// until every workgroup's flag of this parity holds `epoch`, one flag per thread (a
+// workgroup can be one window ahead -- its tile may have little to do -- and have
+// published epoch + 1 before this one reads its flag: with one word for both, its count
+// would be the next window's; two ahead it cannot be); with `cnt`, the counts of tiles [ct0, ct1) land in
 // cnt[h] (0 for the others).  A poll is one load, back to back with the next (each a
 // round trip past the L2, the pace of the loop); the error word and the clock, a round
 // trip of their own, are read every 16th poll only.  The wait is bounded: past `limit`
@@ -576,7 +579,7 @@ __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g,
                                           uint32_t* cnt, uint32_t ct0, uint32_t ct1, uint32_t* err, uint64_t limit) {
     __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0)
     __syncthreads();
-    uint64_t* flag = reinterpret_cast<uint64_t*>(bar);
+    uint64_t* flag = reinterpret_cast<uint64_t*>(bar) + (epoch & 1u);
     constexpr size_t kStride64 = kBarStride / 2;
     if (threadIdx.x == 0) st_agent64(&flag[(size_t)g * kStride64], ((uint64_t)count << 32) | epoch);
     int bad = 0;

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from mgbrain_amd import native as N
+from mgbrain_amd import workloads as W
 from oracle import pyoracle as po
 from tests import harness as H
 from tests import netmodels as M
@@ -42,3 +43,25 @@ def test_steps_of_a_window(kind, wf, window, tile, block, persist):
                      gpu_kw=dict(weight_format=wf, window=window, tile_size=tile, prop_block=block, propagation=2,
                                  persistent=persist))
     assert n > 100
+
+
+def test_regions_with_tiles_a_window_ahead():
+    """List regions where some tiles have next to nothing to do (three Poisson neurons)
+    beside tiles of many synapses: the light tiles publish the next window's count while
+    others still wait for this one's."""
+    _say("case: 3-neuron Poisson tiles beside LIFB tiles, 30000 steps, list regions")
+    pops = [dict(num=3, type=N.POISSON, rate=0.3), dict(num=900, type=N.POISSON, rate=0.05),
+            dict(num=6000, type=N.LIFB)]
+    projs = [dict(src=s, tar=2, kind=N.CONN_FIXED_INDEGREE, k=k, w=w, dmin=1e-3, dmax=2e-3, index=i, seed=9)
+             for i, (s, k, w) in enumerate(((0, 3, 1e-5), (1, 300, 1e-5), (2, 400, -1e-5)))]
+    out = []
+    for mode in (N.PERSIST_REGIONS, N.PERSIST_OFF):
+        g = N.Simulator.generated(pops, projs, W.lifb_consts(), seed=9, propagation=2, tile_size=60, prop_block=512,
+                                  persistent=mode)
+        assert g.info()["persistent"] == (2 if mode == N.PERSIST_REGIONS else 0)
+        g.run(30000)
+        out.append((g.fire_counts(), g.state(N.F_V).view(np.uint32), g.info()["spikes"]))
+        g.close()
+    (ca, va, na), (cb, vb, nb) = out
+    assert na == nb and na > 100000
+    assert np.array_equal(ca, cb) and np.array_equal(va, vb)
