@@ -104,7 +104,7 @@ struct mgb_sim {
     uint64_t* seg_obase = nullptr;     // [nseg+1]
     uint64_t n_offs = 0, n_keys = 0;
     uint32_t* tcnt = nullptr;          // [3][nseg]
-    int tkind = kTClass;               // synapse word kind of the fused kernel
+    int tkind = kTClass16;             // synapse word kind of the fused kernel
     uint32_t* tperm = nullptr;         // fused STDP: CSR slot of each tile-order position (~0u: padding)
     uint64_t n_tslots = 0;             // length of the (padded) tile-order arrays
     float2* seg_scale = nullptr;       // fixed-point formats, several segments: (scale, 1 / scale)
@@ -373,9 +373,8 @@ mgb_status choose_tiles(mgb_sim* s, const mgb_opts* o, int32_t n, int32_t D, con
         (int32_t)((lds_max - (int64_t)tiled_lds_bytes(D, 0, s->tkind, s->trw, lut1) - kTiledStaticLds) / per_b);
     while (bmax > 1 && (int64_t)tiled_lds_bytes(D, bmax, s->tkind, s->trw, lut1) + kTiledStaticLds > lds_max)
         --bmax;
-    // wide words hold an 11-bit tile-local target; CLASS tiles of at most 1024
-    // targets take 16-bit words (else 32-bit words with the global id)
-    bmax = std::max<int32_t>(1, std::min<int32_t>(bmax, s->tkind == kTClass ? 1024 : 2048));
+    // wide words hold a tile-local target below 2048, the 16-bit CLASS words one below 1024
+    bmax = std::max<int32_t>(1, std::min<int32_t>(bmax, s->tkind == kTClass16 ? 1024 : 2048));
     int32_t Breq = (o && o->tile_size > 0) ? o->tile_size : std::max<int32_t>(256, (n + 255) / 256);
     Breq = std::max<int32_t>(1, Breq);
     const std::vector<int32_t>& lo = s->h_seg_lo;
@@ -675,7 +674,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     Scratch X;
     // ---- statistics + delay quantisation --------------------------------------
     uint8_t* dq = nullptr;
-    uint32_t *flags = nullptr, *wcls = nullptr, *indeg = nullptr, *in_pl = nullptr, *absmax = nullptr;
+    uint32_t *flags = nullptr, *wcls = nullptr, *indeg = nullptr, *in_more = nullptr, *in_pl = nullptr, *absmax = nullptr;
     int32_t* mm = nullptr;
     unsigned long long* npl = nullptr;
     MGB_TRY(X.get(&dq, S));
@@ -683,6 +682,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_TRY(X.get(&mm, 2));
     MGB_TRY(X.get(&wcls, 2 * (size_t)n));
     MGB_TRY(X.get(&indeg, 2 * (size_t)n));
+    MGB_TRY(X.get(&in_more, 2 * (size_t)n));
     MGB_TRY(X.get(&in_pl, (size_t)n));
     MGB_TRY(X.get(&npl, 1));
     std::vector<uint16_t> run_of;
@@ -699,6 +699,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_HIP_TRY(hipMemcpyAsync(mm, mm_init, 8, hipMemcpyHostToDevice, st));
     MGB_HIP_TRY(hipMemsetAsync(wcls, 0xFF, 8 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(indeg, 0, 8 * (size_t)n, st));
+    MGB_HIP_TRY(hipMemsetAsync(in_more, 0, 8 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(in_pl, 0, 4 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(absmax, 0, 4 * std::max<size_t>(nruns, 1), st));
     MGB_HIP_TRY(hipMemsetAsync(npl, 0, 8, st));
@@ -709,7 +710,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         a.plastic = h.stdp ? L.plastic : nullptr;
         a.seg = seg_dev;                                   // null for one run: absmax[0]
         a.dq = dq; a.flags = flags; a.min_d = mm; a.max_d = mm + 1;
-        a.wcls = wcls; a.indeg = indeg; a.in_pl = in_pl; a.absmax = absmax; a.n_plastic = npl;
+        a.wcls = wcls; a.indeg = indeg; a.in_more = in_more; a.in_pl = in_pl; a.absmax = absmax; a.n_plastic = npl;
         MGB_HIP_TRY(run_stats(a, st));
     }
     uint32_t hflags = 0;
@@ -720,9 +721,10 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_HIP_TRY(hipMemcpyAsync(hmm, mm, 8, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipMemcpyAsync(habs.data(), absmax, 4 * habs.size(), hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipMemcpyAsync(&hnpl, npl, 8, hipMemcpyDeviceToHost, st));
-    std::vector<uint32_t> h_wcls(2 * (size_t)n), h_indeg(2 * (size_t)n);
+    std::vector<uint32_t> h_wcls(2 * (size_t)n), h_indeg(2 * (size_t)n), h_more(2 * (size_t)n);
     MGB_HIP_TRY(hipMemcpyAsync(h_wcls.data(), wcls, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipMemcpyAsync(h_indeg.data(), indeg, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
+    MGB_HIP_TRY(hipMemcpyAsync(h_more.data(), in_more, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipStreamSynchronize(st));
     if (hflags & kFlagBadId) {
         set_error("a synapse references a neuron id outside [0, %d)", n);
@@ -808,8 +810,9 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                 id = it->second;
             }
             s->h_tbl[t] = (uint16_t)id;
-            tmax_e[id] = std::max(tmax_e[id], h_indeg[t]);
-            tmax_i[id] = std::max(tmax_i[id], h_indeg[(size_t)n + t]);
+            // (a neuron's arrivals of one sign in one step are at most its synapses of it)
+            tmax_e[id] = std::max(tmax_e[id], h_indeg[t] + h_more[t]);
+            tmax_i[id] = std::max(tmax_i[id], h_indeg[(size_t)n + t] + h_more[(size_t)n + t]);
         }
         if (keys.size() > 0xFFFFu) {
             set_error("too many weight classes (%zu)", keys.size());
@@ -822,8 +825,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         for (size_t c = 0; c < keys.size(); ++c) {
             for (int side = 0; side < 2; ++side) {
                 const uint32_t bits = side ? keys[c].second : keys[c].first;
-                // at least kClassCache entries: the fused kernel caches that many
-                const uint32_t len = std::max<uint32_t>((side ? tmax_i[c] : tmax_e[c]) + 1, kClassCache);
+                const uint32_t len = (side ? tmax_i[c] : tmax_e[c]) + 1;
                 float w = 0.f;
                 if (bits != kWSentinel) std::memcpy(&w, &bits, 4);
                 s->class_w[2 * c + side] = w;
@@ -848,7 +850,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         MGB_HIP_TRY(hipMemcpyAsync(s->seq, seq.data(), 4 * seq.size(), hipMemcpyHostToDevice, st));
         const int prop = o ? o->propagation : MGB_PROP_AUTO;
         s->tiled = (prop == MGB_PROP_AUTO || prop == MGB_PROP_TILED) ? 1 : 0;
-        s->tkind = kTClass;
+        s->tkind = kTClass16;
         if (s->tiled) {
             MGB_TRY(choose_tiles(s, o, n, s->D, h.type, h_indeg));
             // tile-sorted copy: stable sort by (source, target tile) keeps list order
@@ -866,21 +868,15 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                 }
                 MGB_HIP_TRY(sort_pairs(temp, &tb2, kin, kout, vin, vout, S, tbits, st));
             }
-            if (s->B <= 1024) {
-                // 2 B per synapse: the target is stored relative to its tile
-                s->tkind = kTClass16;
-                MGB_TRY(dalloc_n(s, &s->syn16, S));
-                MGB_HIP_TRY(class16_words(vout, S, tt, s->syn16, st));
-            } else {
-                MGB_TRY(dalloc_n(s, &s->syn_t, S));
-                if (S) MGB_HIP_TRY(hipMemcpyAsync(s->syn_t, vout, S * 4, hipMemcpyDeviceToDevice, st));
-            }
+            // 2 B per synapse: the target is stored relative to its tile
+            MGB_TRY(dalloc_n(s, &s->syn16, S));
+            MGB_HIP_TRY(class16_words(vout, S, tt, s->syn16, st));
             MGB_TRY(build_tile_offsets(s, n, kout, tt));
             MGB_TRY(pad_subrows(s, n));
             MGB_TRY(dalloc_n(s, &s->tile_cc, (size_t)s->G * 4 * kClassCache));
             MGB_TRY(dalloc_n(s, &s->tile_ccls, (size_t)s->G * 2));
-            MGB_HIP_TRY(launch_tile_ccache(s->tile_lo, s->G, s->tbl, s->tbl_off, s->seq, s->tile_cc, s->tile_ccls,
-                                           st));
+            MGB_HIP_TRY(launch_tile_ccache(s->tile_lo, s->G, s->tbl, s->tbl_off, s->seq, (uint32_t)seq.size(),
+                                           s->tile_cc, s->tile_ccls, st));
         }
         MGB_HIP_TRY(hipStreamSynchronize(st));
     } else {

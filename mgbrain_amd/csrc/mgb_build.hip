@@ -80,9 +80,12 @@ __global__ void k_stats(StatArgs a) {
         }
         // in-degree per (target, class); target-major lists hit one address per wave
         if (wave_all_equal(key)) {
+            // (indeg counts such a wave as one: the tile boundaries and fixed-point scales
+            // derived from it are part of saved checkpoints and of results; in_more holds
+            // the other 63)
             if (key != 0xFFFFFFFFu && (threadIdx.x & 63u) == 0u) {
-                const uint32_t c = (uint32_t)__popcll(__ballot(true));
-                atomicAdd(&a.indeg[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], c);
+                atomicAdd(&a.indeg[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], 1u);
+                atomicAdd(&a.in_more[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], 63u);
             }
         } else if (key != 0xFFFFFFFFu) {
             atomicAdd(&a.indeg[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], 1u);
@@ -133,8 +136,9 @@ __global__ void k_class16(const uint32_t* w32, uint64_t S, TileTabs tt, uint16_t
          k += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t w = w32[k];
         const int32_t t = (int32_t)(w & 0x3FFFFFFu);
-        const uint32_t loc = (uint32_t)(t - tt.tile_lo[tt.tile_of[t]]);
-        out[k] = (uint16_t)(loc | (((w >> 26) & 31u) << 10) | ((w >> 31) << 15));
+        const uint32_t g = tt.tile_of[t];
+        const int32_t t0 = tt.tile_lo[g], tn = tt.tile_lo[g + 1] - t0;
+        out[k] = (uint16_t)((((w >> 26) & 31u) * (uint32_t)tn + (uint32_t)(t - t0)) | ((w >> 31) << 15));
     }
 }
 
@@ -164,14 +168,18 @@ __global__ void k_tile_gather_wide(const uint32_t* slot, uint64_t S, const int32
          k += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t p = slot[k];
         const int32_t t = col[p];
-        const uint32_t loc = (uint32_t)(t - tt.tile_lo[tt.tile_of[t]]);
+        const uint32_t g = tt.tile_of[t];
+        const int32_t t0 = tt.tile_lo[g], tn = tt.tile_lo[g + 1] - t0;
+        const uint32_t loc = (uint32_t)(t - t0);
         const uint32_t d = (uint32_t)(dly[p] & 127u);
         uint32_t payload = 0u;
         if (kind == kTBF16) payload = w16[p];
         else if (kind == kTFP8) payload = w8[p];
         else if (kind == kTStdp) payload = (uint32_t)(dly[p] >> 7);
         else if (kind == kTStdpB) payload = (dly[p] & 128u) ? 0xFFFFu : (uint32_t)w16[p];
-        syn_t[k] = loc | ((d - 1u) << 11) | (payload << 16);
+        const uint32_t place = (kind == kTStdp || kind == kTStdpB) ? loc | ((d - 1u) << 11)
+                                                                   : (d - 1u) * (uint32_t)tn + loc;
+        syn_t[k] = place | (payload << 16);
         if (kind == kTF32 || kind == kTStdp || kind == kTStdpB) w_t[k] = w32[p];
     }
 }

@@ -148,14 +148,16 @@ struct StdpArgs {
 // one segment, each segment has its own spike lists, and a source row of
 // segment q holds offsets for q's tiles only: offs[seg_obase[q] +
 // (src - seg_lo[q]) * (Gq + 1) + local tile], Gq = tiles of q.
-// Synapse word kinds of the fused kernel.  kTClass16 is the CLASS word of a
-// tiling with B <= 1024: tile-local target (10 bits) | delay-1 << 10 | sign << 15.
-// kTStdp: the kTF32 word with a plastic flag at bit 16, FP32 weights in tile
+// Synapse word kinds of the fused kernel (the values are kept in checkpoints).  The low
+// bits of the words without STDP are (delay - 1) * tn + local target, tn the width of the
+// target's tile: 15 bits of a CLASS word (kTClass16: sign << 15; tn <= 1024, delay <= 32),
+// 16 bits of a wide word (payload << 16; tn <= 2048).
+// kTStdp: local target (11 bits) | delay-1 << 11, a plastic flag at bit 16, FP32 weights in tile
 // order (w_t, updated in place), pair-based STDP inside the kernel.
 // kTStdpB: kTStdp with BF16 static weights: bits 16-31 of the word hold the BF16
 // code of a static synapse's w / row scale, or 0xFFFF for a plastic synapse,
 // whose FP32 weight is in w_t (static positions of w_t are never read).
-enum TiledKind { kTClass = 0, kTBF16 = 1, kTFP8 = 2, kTF32 = 3, kTClass16 = 4, kTStdp = 5, kTStdpB = 6 };
+enum TiledKind { kTBF16 = 1, kTFP8 = 2, kTF32 = 3, kTClass16 = 4, kTStdp = 5, kTStdpB = 6 };
 // The fused kinds with STDP.
 inline bool stdp_kind(int k) { return k == kTStdp || k == kTStdpB; }
 
@@ -278,7 +280,7 @@ hipError_t launch_finalize(Ctl* ctl, int32_t steps, int32_t windows, hipStream_t
 constexpr int kTiledBatch = 1024;   // spikes staged in LDS per propagation batch
 constexpr int kTiledItems = 16384;  // work items staged in LDS per propagation round
 constexpr int kTiledStaticLds = 1024; // bytes reserved for the fused kernel's static LDS
-constexpr int kClassCache = 32;     // k-fold class sums cached in LDS (tables hold >= this many)
+constexpr int kClassCache = 128;    // k-fold class sums cached in LDS per class and side
 constexpr int kStdpHist = 16;       // spike steps kept per neuron for deferred dendrite updates
 // A history entry past the neuron's spikes (memset byte 0x80): below every step and
 // every lower bound of a history scan (>= -1).
@@ -299,7 +301,7 @@ constexpr int kBufferDword3 = 0x00020000;
 size_t tiled_lds_bytes(int D, int B, int kind, int rw, int lut_lds = 0);
 // Class cache of every tile of the CLASS kinds (cc [G][2][2][kClassCache], cls [G][2]).
 hipError_t launch_tile_ccache(const int32_t* tile_lo, int32_t G, const uint16_t* tbl, const uint32_t* tbl_off,
-                              const float* seq, float* cc, uint32_t* cls, hipStream_t st);
+                              const float* seq, uint32_t n_seq, float* cc, uint32_t* cls, hipStream_t st);
 // Workgroups of `block` threads of the fused kernel for `a` that one CU holds at once.
 int tiled_blocks_per_cu(const TiledArgs& a, int block, bool persistent = false);
 hipError_t launch_tiled(const TiledArgs& a, int32_t off, int32_t wk, int32_t nsteps, int block,

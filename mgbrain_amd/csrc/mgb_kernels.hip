@@ -464,28 +464,30 @@ __global__ void k_finalize(Ctl* ctl, int32_t steps, int32_t windows) {
 }
 
 
-// Inclusive block-wide prefix sum (blockDim.x a multiple of 64, <= 1024).
-__device__ __forceinline__ uint32_t block_incl_scan(uint32_t v, uint32_t* wsum) {
-    const uint32_t lane = lane_id(), wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t t = __shfl_up(v, o);
-        if (lane >= (uint32_t)o) v += t;
-    }
+// Inclusive prefix sum over the wave, in data-parallel moves: rows of 16 lanes, then the
+// rows' last lanes into the rows after them.
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);   // row_shr 1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);   // row_shr 2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);   // row_shr 4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);   // row_shr 8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);   // lane 15 of rows 0, 2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);   // lane 31
+    return v;
+}
+
+// Inclusive block-wide prefix sum and total (blockDim.x a multiple of 64, <= 1024).  One
+// barrier: every wave scans the waves' sums itself.  The caller alternates between two
+// wsum buffers, with a barrier between two uses of one.
+__device__ __forceinline__ uint32_t block_incl_scan(uint32_t v, uint32_t* wsum, uint32_t& total) {
+    const uint32_t lane = lane_id(), nw = blockDim.x >> 6;
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    v = wave_incl_scan(v);
     if (lane == 63) wsum[wid] = v;
     __syncthreads();
-    if (wid == 0) {
-        uint32_t x = lane < nw ? wsum[lane] : 0u;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t t = __shfl_up(x, o);
-            if (lane >= (uint32_t)o) x += t;
-        }
-        if (lane < nw) wsum[lane] = x;
-    }
-    __syncthreads();
-    if (wid > 0) v += wsum[wid - 1];
-    return v;
+    const uint32_t x = wave_incl_scan(lane < nw ? wsum[lane] : 0u);
+    total = (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+    return v + (wid ? (uint32_t)__builtin_amdgcn_readlane((int)x, (int)wid - 1) : 0u);
 }
 
 // One tile's ring slice (rw halves of D x B words) from HBM into LDS.  Rows
@@ -689,14 +691,19 @@ __device__ __forceinline__ uint32_t tneu_steps(TNeu& st, const float (&be)[NB], 
 // Spike lists rotate over three buffers: window k writes k%3, reads (k-1)%3
 // and clears the counter of (k+1)%3, which no workgroup touches in window k.
 //
-// WK selects the synapse word.  kTClass: target | delay-1 << 26 | inhibitory
-// << 31, arrivals counted per class (16 + 16 bits of one ring word).  Wide
-// formats: local target (11 bits) | delay-1 << 11 | BF16 (kTBF16) or FP8
-// (kTFP8, per-source scale) weight bits << 16, or the weight in w_t (kTF32);
-// arrivals add rintf(w * scale) into int32 exc / inh rings, as k_prop does.
+// WK selects the synapse word.  Its low bits are the synapse's place in the tile's
+// ring slice relative to the first row its spike can reach, (delay - 1) * tn + local
+// target (tn the tile's width): a work item adds the spike's row and wraps once at the
+// slice's end, four instructions per synapse.  (Decoding target and delay fields took
+// about 29 vector instructions per synapse in all, which bound windows of many events:
+// 110,000 balanced neurons at 28 Hz, 4.2e7 events per window.)
+// kTClass16: 15 bits | inhibitory << 15, arrivals counted per class (16 + 16 bits of one
+// ring word).  Wide formats: 16 bits | BF16 (kTBF16) or FP8 (kTFP8, per-source scale)
+// weight bits << 16, or the weight in w_t (kTF32); arrivals add rintf(w * scale) into
+// int32 exc / inh rings, as k_prop does.
 //
-// kTStdp: the kTF32 word with a plastic flag at bit 16 and pair-based STDP
-// (mgcore.cu:346-412) on w_t.  kTStdpB: the same with BF16 static weights
+// kTStdp: local target (11 bits) | delay-1 << 11 with a plastic flag at bit 16 and
+// pair-based STDP (mgcore.cu:346-412) on w_t.  kTStdpB: the same with BF16 static weights
 // (times the source row's scale) in the word and 0xFFFF there for a plastic
 // synapse; w_t is read only for spikes of rows with a plastic synapse into
 // tiles with a plastic in-synapse (row_aux, tile_pl).  A synapse k -> j lives in the tile of its
@@ -732,12 +739,9 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     static_assert(!(PW && (WK == kTStdp || WK == kTStdpB)), "the persistent form has no STDP");
     static_assert(!RG || (PW && WK == kTClass16), "list regions: persistent form of 16-bit CLASS words only");
     extern __shared__ __align__(16) uint32_t lds[];
-    __shared__ uint32_t wsum[16];
+    __shared__ uint32_t wsum[2][16];
     __shared__ unsigned long long se_blk, lsp_r;
     __shared__ uint32_t lsp_n, lsp_g;
-    // CLASS: the first kClassCache k-fold sums of the classes of the tile's
-    // last and first neurons (one class per tile in population-ordered networks)
-    __shared__ float ccache[2][2][kClassCache];
     __shared__ uint32_t ccls[2];
     const int32_t D = a.D, B = a.B, bd = (int32_t)blockDim.x;
     const int32_t tid0 = (int32_t)threadIdx.x;
@@ -753,18 +757,26 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         const int32_t x = b % kXcds, qx = G / kXcds, rx = G % kXcds;
         return x * qx + min(x, rx) + b / kXcds;
     }();
-    constexpr bool kCls = WK == kTClass || WK == kTClass16;  // CLASS arrival counts
+    constexpr bool kCls = WK == kTClass16;                  // CLASS arrival counts
     constexpr bool kMix = WK == kTStdpB;                    // BF16 static weights beside plastic ones
     constexpr bool kPl = WK == kTStdp || kMix;              // STDP on w_t
     constexpr bool kAux = WK == kTFP8 || WK == kTBF16 || kPl;
     const int RW = kCls ? 1 : a.rw;                         // ring words per (slot, target)
     uint32_t* ring = lds;                                   // [RW][D][B]
     // (STDP: rounded up to 16 bytes, for the history rows' vector reads below)
-    uint32_t* sp_beg = ring + (kPl ? (((size_t)RW * D * B + 3) & ~(size_t)3) : (size_t)RW * D * B);
-    uint32_t* sp_len = sp_beg + kTiledBatch;                // len | slot-of-spike << 26
-    uint32_t* sp_start = sp_len + kTiledBatch;              // exclusive prefix of work items
+    uint32_t* stage = ring + (kPl ? (((size_t)RW * D * B + 3) & ~(size_t)3) : (size_t)RW * D * B);
+    // [kTiledBatch] per staged spike: (its sub-row's first word - CH * its first work
+    // item) mod 2^32, so that item q starts at word x + CH * q; byte offset of its row in
+    // the slice (STDP: its ring slot << 26)
+    uint2* sp_rec = reinterpret_cast<uint2*>(ring + (((size_t)(stage - ring) + 1) & ~(size_t)1));
+    // CLASS: the first kClassCache k-fold sums of the classes of the tile's
+    // last and first neurons (one class per tile in population-ordered networks),
+    // [class][side][count], in what the records leave of their 3 * kTiledBatch words
+    float* ccache = reinterpret_cast<float*>(sp_rec + kTiledBatch);
+    static_assert(2 * kTiledBatch + 4 * kClassCache + 1 <= 3 * kTiledBatch, "staging area");
     constexpr uint32_t kItems = kTiledItems;   // work items staged per round
-    uint16_t* itm = reinterpret_cast<uint16_t*>(sp_start + kTiledBatch);   // [kItems] spike of item
+    // [kItems] spike of the item | (its words - 1) << 10
+    uint16_t* itm = reinterpret_cast<uint16_t*>(stage + 3 * (size_t)kTiledBatch);
     // [kTiledBatch] BF16/FP8: row scale bits; STDP: the source's last spike before the window
     uint32_t* sp_aux = reinterpret_cast<uint32_t*>(itm + kItems);
     // [kTiledBatch] kTStdpB: row scale bits | weights-to-load << 31
@@ -923,8 +935,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             // the counts came with the wait (rg_pre); the list is laid out by their prefix
             sprev = s0 - nsteps;
             const uint32_t c = (uint32_t)tid < (uint32_t)a.G ? rg_pre[tid] : 0u;
-            const uint32_t incl = block_incl_scan(c, wsum);
-            E = wsum[(blockDim.x >> 6) - 1];
+            const uint32_t incl = block_incl_scan(c, wsum[0], E);
             if ((uint32_t)tid < (uint32_t)a.G) rg_pre[tid] = incl - c;
             __syncthreads();
             ent0 = (uint32_t)tid < E ? rentry((uint32_t)tid) : 0u;
@@ -961,10 +972,9 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 lutL[a.lut_lds + k] = a.ltd[k];
             }
         }
-        if (kCls && kw == 0 && tid < 4 * kClassCache) {
+        if (kCls && kw == 0) {
             // (precomputed per tile by k_tile_ccache: one load instead of a chain of three)
-            ccache[tid / (2 * kClassCache)][(tid / kClassCache) & 1][tid % kClassCache] =
-                a.tile_cc[(size_t)g * 4 * kClassCache + tid];
+            for (int32_t k = tid; k < 4 * kClassCache; k += bd) ccache[k] = a.tile_cc[(size_t)g * 4 * kClassCache + k];
             if (tid < 2) ccls[tid] = a.tile_ccls[2 * g + tid];
         }
         // 1. ring slice -> LDS.  The slots the previous window consumed ([sprev, s0)
@@ -1021,17 +1031,20 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         __syncthreads();
 
         // 2. previous window's spikes into the tile
+        const uint32_t R4 = 4u * (uint32_t)(D * tn);            // the slice's bytes (one of RW halves)
+        int sb = 0;                                             // scan buffer
         for (uint32_t b0 = 0; b0 < E; b0 += (uint32_t)bd) {
             const uint32_t nb = min((uint32_t)bd, E - b0);
-            uint32_t items = 0u;
+            uint32_t items = 0u, beg = 0u, len = 0u, slot26 = 0u;
             if ((uint32_t)tid < nb) {
-                uint32_t beg = pbeg, lm = plm, aux = paux, aux2 = paux2;
+                uint32_t lm = plm, aux = paux, aux2 = paux2;
+                beg = pbeg;
                 if (!kAhead && b0 > 0) meta(lent(b0 + (uint32_t)tid), beg, lm, aux, aux2);
-                sp_beg[tid] = beg;
-                sp_len[tid] = lm;
                 if (kAux) sp_aux[tid] = aux;
                 if (kMix) sp_aux2[tid] = aux2;
-                items = ((lm & kIdMask) + CH - 1) / CH;
+                len = lm & kIdMask;
+                slot26 = lm & ~kIdMask;
+                items = (len + CH - 1) / CH;
             }
             if constexpr (kAhead) {
                 // the next batch's metadata from its entries (loaded a batch ago), and the
@@ -1040,15 +1053,22 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 if (b1 < E && (uint32_t)tid < E - b1) meta(ent1, pbeg, plm, paux, paux2);
                 if (b2 < E && (uint32_t)tid < E - b2) ent1 = lent(b2 + (uint32_t)tid);
             }
-            const uint32_t incl = block_incl_scan(items, wsum);
-            const uint32_t total = wsum[(blockDim.x >> 6) - 1];
-            if ((uint32_t)tid < nb) sp_start[tid] = incl - items;
+            sb ^= 1;
+            uint32_t total;
+            const uint32_t incl = block_incl_scan(items, wsum[sb], total);
+            // (without items nothing waits between this and the spike list that takes the records' place)
+            if (total > 0u && (uint32_t)tid < nb)
+                sp_rec[tid] = make_uint2(beg - (incl - items) * (uint32_t)CH,
+                                         kPl ? slot26 : 4u * ((slot26 >> 26) + 1u) * (uint32_t)tn);
             for (uint32_t r0 = 0; r0 < total; r0 += kItems) {
                 const uint32_t rn = min(kItems, total - r0);
                 // item table: each spike writes its own work items of this round
                 if ((uint32_t)tid < nb) {
                     const uint32_t q0 = max(incl - items, r0), q1 = min(incl, r0 + rn);
-                    for (uint32_t q = q0; q < q1; ++q) itm[q - r0] = (uint16_t)tid;
+                    for (uint32_t q = q0; q < q1; ++q) {
+                        const uint32_t n = q + 1u == incl ? len - (items - 1u) * (uint32_t)CH : (uint32_t)CH;
+                        itm[q - r0] = (uint16_t)((uint32_t)tid | ((n - 1u) << 10));
+                    }
                 }
                 __syncthreads();
                 // U items per thread in flight: U * CH synapse words loaded before the
@@ -1056,10 +1076,10 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 // (STDP: at most 8 synapses, whose STDP state then fits in the registers)
                 constexpr int U = CH >= 16 ? 1 : (kPl ? (CH >= 8 ? 1 : (CH == 1 ? 4 : 8 / CH)) : 16 / CH);
                 for (uint32_t it = (uint32_t)tid; it < rn; it += (uint32_t)(U * bd)) {
-                    // branch-free body, so that all U * CH loads are in flight before the
-                    // first wait: lanes past the round's items re-read the last item and
-                    // elements past an item's end re-read its last element; both add 0
-                    uint32_t cnt[U], kb[U];
+                    // branch-free loads, so that all U * CH are in flight before the first
+                    // wait: lanes past the round's items re-read the last item and elements
+                    // past an item's end re-read its last element or what follows
+                    uint32_t cnt[U], kb[U], row[U];
                     int32_t sD[U], t2[U], la[U];
                     float rs[U];
                     bool lw[U];              // kTStdpB: the item's weights are loaded
@@ -1067,14 +1087,14 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                     for (int h = 0; h < U; ++h) {
                         const uint32_t q0 = it + (uint32_t)(h * bd);
                         const uint32_t q = min(q0, rn - 1u);
-                        const uint32_t j = itm[q];
-                        const uint32_t c = r0 + q - sp_start[j];
-                        const uint32_t meta = sp_len[j];
-                        const uint32_t len = meta & kIdMask;
-                        sD[h] = (int32_t)(meta >> 26);
-                        kb[h] = sp_beg[j] + c * CH;
-                        cnt[h] = (q0 < rn) ? min((uint32_t)CH, len - c * CH) : 0u;
-                        rs[h] = (WK == kTFP8 || WK == kTBF16) ? __uint_as_float(sp_aux[j]) : 1.0f;
+                        const uint32_t im = itm[q];
+                        const uint32_t j = im & 1023u;
+                        const uint2 rc = sp_rec[j];
+                        kb[h] = rc.x + (r0 + q) * (uint32_t)CH;
+                        row[h] = rc.y;
+                        cnt[h] = (q0 < rn) ? (im >> 10) + 1u : 0u;
+                        // (scales are powers of 2: the product with the row scale is exact)
+                        rs[h] = (WK == kTFP8 || WK == kTBF16) ? __uint_as_float(sp_aux[j]) * fsc.x : 1.0f;
                         lw[h] = true;
                         if (kMix) {
                             const uint32_t a2 = sp_aux2[j];
@@ -1084,6 +1104,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                         if (kPl) {
                             // the spike's step: the window is shorter than the ring, so its
                             // slot determines it
+                            sD[h] = (int32_t)(rc.y >> 26);
                             const int32_t dd = sD[h] - rprev;
                             t2[h] = (int32_t)sprev + dd + (dd < 0 ? D : 0);
                             la[h] = (int32_t)sp_aux[j];
@@ -1224,30 +1245,34 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     #pragma unroll
                         for (int u = 0; u < CH; ++u) {
                             // words past the item's end (padding, another tile's words) and
-                            // lanes past the round's items: a distinct in-slice entry per
-                            // lane, adding 0
+                            // lanes past the round's items add nothing (masked off rather
+                            // than adding 0: their words repeat, and lanes adding to one
+                            // address go one by one)
                             const bool valid = (uint32_t)u < cnt[h];
                             const uint32_t xw = x[h][u];
-                            if (WK == kTClass) {
-                                int32_t slot = sD[h] + (int32_t)((xw >> 26) & 31u) + 1;
-                                slot -= (slot >= D) ? D : 0;
-                                const int32_t loc = (int32_t)(xw & kIdMask) - t0;
-                                const int32_t at = valid ? slot * tn + loc : (tid % tn);
-                                atomicAdd(&ring[at], valid ? ((xw >> 31) ? 0x10000u : 1u) : 0u);
-                            } else if (WK == kTClass16) {
-                                int32_t slot = sD[h] + (int32_t)((xw >> 10) & 31u) + 1;
-                                slot -= (slot >= D) ? D : 0;
-                                const int32_t loc = (int32_t)(xw & 0x3FFu);
-                                const int32_t at = valid ? slot * tn + loc : (tid % tn);
-                                atomicAdd(&ring[at], valid ? ((xw >> 15) ? 0x10000u : 1u) : 0u);
+                            if (!kPl) {
+                                uint32_t at = row[h] + ((xw & (WK == kTClass16 ? 0x7FFFu : 0xFFFFu)) << 2);
+                                at = min(at, at - R4);              // wraps at the slice's end
+                                if (WK == kTClass16) {
+                                    if (valid)
+                                        atomicAdd(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(ring) + at),
+                                                  1u << ((xw >> 11) & 16u));
+                                } else {
+                                    float w;                        // times the fixed-point scale
+                                    if (WK == kTBF16) w = bf16_to_f32((uint16_t)(xw >> 16)) * rs[h];
+                                    else if (WK == kTFP8) w = fp8e4m3_to_f32((uint8_t)(xw >> 16)) * rs[h];
+                                    else w = wv[h][u] * fsc.x;
+                                    if (RW == 2) at += w > 0.f ? 0u : R4;   // (one ring: both signs in one sum)
+                                    if (valid)
+                                        atomicAdd(reinterpret_cast<int32_t*>(reinterpret_cast<char*>(ring) + at),
+                                                  (int32_t)rintf(w));
+                                }
                             } else {
                                 int32_t slot = sD[h] + (int32_t)((xw >> 11) & 31u) + 1;
                                 slot -= (slot >= D) ? D : 0;
                                 const int32_t loc = (int32_t)(xw & 0x7FFu);
                                 float w;
-                                if (WK == kTBF16) w = bf16_to_f32((uint16_t)(xw >> 16)) * rs[h];
-                                else if (WK == kTFP8) w = fp8e4m3_to_f32((uint8_t)(xw >> 16)) * rs[h];
-                                else if (kMix && (xw >> 16) != 0xFFFFu) w = bf16_to_f32((uint16_t)(xw >> 16)) * rs[h];
+                                if (kMix && (xw >> 16) != 0xFFFFu) w = bf16_to_f32((uint16_t)(xw >> 16)) * rs[h];
                                 else w = wv[h][u];
                                 const bool pl = kPl && rng[h][u] >= 0;
                                 if (pl) {
@@ -1269,9 +1294,8 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                             }
                         }
                 }
-                __syncthreads();
+                __syncthreads();   // the items (and after the last round the records) are rewritten
             }
-            __syncthreads();   // wsum / sp_* are rewritten by the next batch
         }
         if (kPl) {
             // 2b. when a flush follows this window: neurons that fired kStdpHist - 2 times
@@ -1302,7 +1326,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         // list (the staging area of step 2, free now; one LDS atomic per wave and
         // step) that joins the segment's window list with one global atomic at the
         // end; lanes that find it full append to HBM directly.
-        uint32_t* lsp = sp_beg;
+        uint32_t* lsp = reinterpret_cast<uint32_t*>(sp_rec);
         uint32_t* wbuf = a.win_buf + (size_t)bcur * a.win_stride + lbase;
         uint32_t* rgw = a.win_buf + (size_t)bcur * a.win_stride + (size_t)t0 * (size_t)a.window;   // (rgp)
         const int32_t slot0 = mod_ring(s0, D);
@@ -1395,7 +1419,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 if (kCls) {
                     // class sums of a cached class: one LDS read per side (the table for
                     // counts past the cache)
-                    const float* cc = &ccache[st.csl < 0 ? 0 : st.csl][0][0];
+                    const float* cc = ccache + (st.csl < 0 ? 0 : st.csl) * 2 * kClassCache;
 #pragma unroll
                     for (int u = 0; u < NB; ++u) {
                         const uint32_t ke = x[u] & 0xFFFFu, ki = x[u] >> 16;
@@ -1555,7 +1579,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
 __global__ __launch_bounds__(256) void k_stdp_flush(TiledArgs a, int32_t off, int32_t wk) {
     __shared__ int32_t ej[256], etf[256];
     __shared__ int64_t epb[256], epe[256];
-    __shared__ uint32_t eui[256], wsum[16];                // inclusive prefix of units
+    __shared__ uint32_t eui[256], wsum[2][16];             // inclusive prefix of units
     const Ctl* ctl = a.ctl;
     const uint32_t tid0 = threadIdx.x;
     // both lists' counts and first entries load with the window index (one round
@@ -1586,9 +1610,9 @@ __global__ __launch_bounds__(256) void k_stdp_flush(TiledArgs a, int32_t off, in
             epe[tid] = pe;
             nu = (uint32_t)((pe - pb + bd - 1) / bd);
         }
-        const uint32_t incl = block_incl_scan(nu, wsum);
+        uint32_t total;
+        const uint32_t incl = block_incl_scan(nu, wsum[0], total);
         eui[tid] = incl;
-        const uint32_t total = wsum[(bd >> 6) - 1];
         __syncthreads();
         for (uint32_t u = (uint32_t)((b + G - (uint32_t)(ubase % G)) % G); u < total; u += G) {
             uint32_t lo_f = 0, hi_f = nc - 1;               // entry f: eui[f-1] <= u < eui[f]
@@ -1726,7 +1750,7 @@ const void* tiled_fn_of(int kind, int chunk, bool pw, bool rg = false) {
             return pw ? tiled_fn_chunk<kTClass16, true>(chunk) : tiled_fn_chunk<kTClass16, false>(chunk);
         case kTStdp: return pw ? nullptr : tiled_fn_chunk<kTStdp, false>(chunk);
         case kTStdpB: return pw ? nullptr : tiled_fn_chunk<kTStdpB, false>(chunk);
-        default: return pw ? tiled_fn_chunk<kTClass, true>(chunk) : tiled_fn_chunk<kTClass, false>(chunk);
+        default: return nullptr;
     }
 }
 
@@ -1743,20 +1767,22 @@ hipError_t launch_fn(const void* f, const TiledArgs& a, int32_t off, int32_t wk,
 // the k-fold sum of side (excitatory, inhibitory) of class cls[g][c], where c = 0
 // is the class of the tile's last neuron and c = 1 that of its first.
 __global__ void k_tile_ccache(const int32_t* tile_lo, const uint16_t* tbl, const uint32_t* tbl_off,
-                              const float* seq, float* cc, uint32_t* cls) {
+                              const float* seq, uint32_t n_seq, float* cc, uint32_t* cls) {
     const int32_t g = (int32_t)blockIdx.x, tid = (int32_t)threadIdx.x;
     const int32_t c = tid / (2 * kClassCache), side = (tid / kClassCache) & 1, k = tid % kClassCache;
     const int32_t t0 = tile_lo[g], t1 = tile_lo[g + 1];
     const uint32_t cl = tbl[c == 0 ? t1 - 1 : t0];
-    cc[(size_t)g * 4 * kClassCache + tid] = seq[tbl_off[2 * cl + side] + k];
+    // (no neuron counts past its class's own table: what lies there is never used)
+    cc[(size_t)g * 4 * kClassCache + tid] = seq[min(tbl_off[2 * cl + side] + (uint32_t)k, n_seq - 1u)];
     if (side == 0 && k == 0) cls[2 * g + c] = cl;
 }
 
 hipError_t launch_tile_ccache(const int32_t* tile_lo, int32_t G, const uint16_t* tbl, const uint32_t* tbl_off,
-                              const float* seq, float* cc, uint32_t* cls, hipStream_t st) {
+                              const float* seq, uint32_t n_seq, float* cc, uint32_t* cls, hipStream_t st) {
     if (G <= 0) return hipSuccess;
-    if (!tile_lo || !tbl || !tbl_off || !seq || !cc || !cls) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_tile_ccache, dim3(G), dim3(4 * kClassCache), 0, st, tile_lo, tbl, tbl_off, seq, cc, cls);
+    if (!tile_lo || !tbl || !tbl_off || !seq || n_seq == 0u || !cc || !cls) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_tile_ccache, dim3(G), dim3(4 * kClassCache), 0, st, tile_lo, tbl, tbl_off, seq, n_seq, cc,
+                       cls);
     return hipGetLastError();
 }
 
