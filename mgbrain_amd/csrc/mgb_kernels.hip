@@ -696,7 +696,8 @@ __device__ __forceinline__ uint32_t tneu_steps(TNeu& st, const float (&be)[NB], 
 // target (tn the tile's width): a work item adds the spike's row and wraps once at the
 // slice's end, four instructions per synapse.  (Decoding target and delay fields took
 // about 29 vector instructions per synapse in all, which bound windows of many events:
-// 110,000 balanced neurons at 28 Hz, 4.2e7 events per window.)
+// 110,000 balanced neurons at 28 Hz, 4.2e7 events per window, 55.6 -> 49.6 us at 1024
+// threads; 11,000 neurons 11.4 -> 10.3 us.)
 // kTClass16: 15 bits | inhibitory << 15, arrivals counted per class (16 + 16 bits of one
 // ring word).  Wide formats: 16 bits | BF16 (kTBF16) or FP8 (kTFP8, per-source scale)
 // weight bits << 16, or the weight in w_t (kTF32); arrivals add rintf(w * scale) into
