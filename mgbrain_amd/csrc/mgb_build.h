@@ -28,7 +28,6 @@ struct StatArgs {
     uint32_t* wcls;         // [2][n] class weight bits per target
     uint32_t* indeg;        // [2][n] in-degree per target and class, a wave of 64 synapses of one
                             // target and class counted as one (target-major lists)
-    uint32_t* in_more;      // [2][n] what indeg leaves out of the in-degree
     uint32_t* in_pl;        // [n] plastic in-degree
     uint32_t* absmax;       // max |w| (float bits)
     unsigned long long* n_plastic;

@@ -80,12 +80,11 @@ __global__ void k_stats(StatArgs a) {
         }
         // in-degree per (target, class); target-major lists hit one address per wave
         if (wave_all_equal(key)) {
-            // (indeg counts such a wave as one: the tile boundaries and fixed-point scales
-            // derived from it are part of saved checkpoints and of results; in_more holds
-            // the other 63)
+            // (counted as one: the ballot is of this one lane.  Tile boundaries, fixed-point
+            // scales and class tables rest on it, and with them checkpoints and results)
             if (key != 0xFFFFFFFFu && (threadIdx.x & 63u) == 0u) {
-                atomicAdd(&a.indeg[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], 1u);
-                atomicAdd(&a.in_more[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], 63u);
+                const uint32_t c = (uint32_t)__popcll(__ballot(true));
+                atomicAdd(&a.indeg[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], c);
             }
         } else if (key != 0xFFFFFFFFu) {
             atomicAdd(&a.indeg[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], 1u);

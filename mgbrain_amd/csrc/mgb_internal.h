@@ -280,6 +280,7 @@ hipError_t launch_finalize(Ctl* ctl, int32_t steps, int32_t windows, hipStream_t
 constexpr int kTiledBatch = 1024;   // spikes staged in LDS per propagation batch
 constexpr int kTiledItems = 16384;  // work items staged in LDS per propagation round
 constexpr int kTiledStaticLds = 1024; // bytes reserved for the fused kernel's static LDS
+constexpr uint32_t kClassTableMin = 32; // shortest k-fold class sum table
 constexpr int kClassCache = 128;    // k-fold class sums cached in LDS per class and side
 constexpr int kStdpHist = 16;       // spike steps kept per neuron for deferred dendrite updates
 // A history entry past the neuron's spikes (memset byte 0x80): below every step and

@@ -1773,7 +1773,7 @@ __global__ void k_tile_ccache(const int32_t* tile_lo, const uint16_t* tbl, const
     const int32_t c = tid / (2 * kClassCache), side = (tid / kClassCache) & 1, k = tid % kClassCache;
     const int32_t t0 = tile_lo[g], t1 = tile_lo[g + 1];
     const uint32_t cl = tbl[c == 0 ? t1 - 1 : t0];
-    // (no neuron counts past its class's own table: what lies there is never used)
+    // (past a class's own table: what follows it, as the reads of larger counts)
     cc[(size_t)g * 4 * kClassCache + tid] = seq[min(tbl_off[2 * cl + side] + (uint32_t)k, n_seq - 1u)];
     if (side == 0 && k == 0) cls[2 * g + c] = cl;
 }

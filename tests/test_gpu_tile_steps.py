@@ -65,19 +65,3 @@ def test_regions_with_tiles_a_window_ahead():
     (ca, va, na), (cb, vb, nb) = out
     assert na == nb and na > 100000
     assert np.array_equal(ca, cb) and np.array_equal(va, vb)
-
-
-@pytest.mark.parametrize("k,persist", [(640, N.PERSIST_AUTO), (640, N.PERSIST_OFF), (64, N.PERSIST_AUTO),
-                                       (129, N.PERSIST_REGIONS)])
-def test_many_arrivals_in_one_step_of_a_target_major_list(k, persist):
-    """Half of a neuron's k inputs arrive in every step: the class sums of hundreds of
-    arrivals, for synapses listed target by target (fixed in-degree)."""
-    _say(f"case: fixed in-degree {k} from a pool firing every other step, persistent={persist}")
-    w, lo, hi = float(np.float32(3.2e-4 / k)), float(np.float32(1e-3)), float(np.float32(2e-3))
-    net = M.Net([(2000, M.POISSON, 1), (300, M.LIFB, 0)],
-                [dict(src=0, tar=1, wmin=w, wmax=w, dmin=lo, dmax=hi, kind=M.FIXK, k=k)], M.config2().lifconst)
-    net.rates = [0.5, 0.0]
-    syn = H.host_synapses(net, seed=3)
-    n = _compare_run(net, syn, 600, seed=3, generated=True, gpu_kw=dict(weight_format=1, propagation=2,
-                                                                       persistent=persist))
-    assert n > 600 * 900
