@@ -578,7 +578,8 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
 // once another workgroup has reported a timeout, it sets *err and returns false,
 // so every workgroup leaves the kernel (the host turns *err into an error).
 __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g, uint32_t epoch, uint32_t count,
-                                          uint32_t* cnt, uint32_t ct0, uint32_t ct1, uint32_t* err, uint64_t limit) {
+                                          uint32_t* cnt, uint32_t ct0, uint32_t ct1, uint32_t* err, uint64_t limit,
+                                          uint32_t* lds_bad) {
     __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0)
     __syncthreads();
     uint64_t* flag = reinterpret_cast<uint64_t*>(bar) + (epoch & 1u);
@@ -603,11 +604,22 @@ __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g,
         }
         if (cnt) cnt[h] = (h >= ct0 && h < ct1) ? (uint32_t)(v >> 32) : 0u;
     }
-    return __syncthreads_or(bad) == 0;
+    if (bad) *lds_bad = 1u;
+    __syncthreads();
+    return *lds_bad == 0u;
 }
 
 template <int N>
 using Int = std::integral_constant<int, N>;
+
+// Words a workgroup of the fused kernel shares.
+struct TileShared {
+    uint32_t wsum[2][16];            // block_incl_scan
+    unsigned long long se, rec_at;   // the window's synaptic events; its spikes' place in the record
+    uint32_t n, list_at;             // its spikes; their place in the segment's list
+    uint32_t ccls[2];                // CLASS: the cached classes
+    uint32_t bad, pad;               // a wait timed out
+};
 
 // Registers of one neuron of a tile across the windows of a launch: the state, the
 // constants of its type's update that every step needs, and what its spikes add up to.
@@ -739,11 +751,9 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                                                 int32_t nwin) {
     static_assert(!(PW && (WK == kTStdp || WK == kTStdpB)), "the persistent form has no STDP");
     static_assert(!RG || (PW && WK == kTClass16), "list regions: persistent form of 16-bit CLASS words only");
+    // All of the LDS is the launch's (no static LDS), the ring slice first: at address 0, so
+    // that a synapse's byte offset in the slice is its LDS address (propagation below).
     extern __shared__ __align__(16) uint32_t lds[];
-    __shared__ uint32_t wsum[2][16];
-    __shared__ unsigned long long se_blk, lsp_r;
-    __shared__ uint32_t lsp_n, lsp_g;
-    __shared__ uint32_t ccls[2];
     const int32_t D = a.D, B = a.B, bd = (int32_t)blockDim.x;
     const int32_t tid0 = (int32_t)threadIdx.x;
     // the workgroup's tile.  Workgroups go round-robin to the kXcds XCDs
@@ -774,7 +784,9 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     // last and first neurons (one class per tile in population-ordered networks),
     // [class][side][count], in what the records leave of their 3 * kTiledBatch words
     float* ccache = reinterpret_cast<float*>(sp_rec + kTiledBatch);
-    static_assert(2 * kTiledBatch + 4 * kClassCache + 1 <= 3 * kTiledBatch, "staging area");
+    TileShared* sh = reinterpret_cast<TileShared*>(ccache + 4 * kClassCache);
+    static_assert(sizeof(TileShared) % 8 == 0 &&
+                  2 * kTiledBatch + 4 * kClassCache + sizeof(TileShared) / 4 + 1 <= 3 * kTiledBatch, "staging area");
     constexpr uint32_t kItems = kTiledItems;   // work items staged per round
     // [kItems] spike of the item | (its words - 1) << 10
     uint16_t* itm = reinterpret_cast<uint16_t*>(stage + 3 * (size_t)kTiledBatch);
@@ -859,8 +871,8 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     own_st.c4 = __int_as_float(0x7F800000);               // lanes without a neuron never fire
     own_st.csl = 0;
     auto load_neuron = [&](int32_t i, TNeu& st, const int32_t* last) {
-        if (ttype == T_LIFB) tneu_load<T_LIFB>(a, i, kCls, ccls, st, last);
-        else if (integ) tneu_load<T_LIF>(a, i, kCls, ccls, st, last);
+        if (ttype == T_LIFB) tneu_load<T_LIFB>(a, i, kCls, sh->ccls, st, last);
+        else if (integ) tneu_load<T_LIF>(a, i, kCls, sh->ccls, st, last);
         else {
             st.deg = (int32_t)(a.row_ptr[i + 1] - a.row_ptr[i]);
             if (last) st.last = last[i];
@@ -936,7 +948,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             // the counts came with the wait (rg_pre); the list is laid out by their prefix
             sprev = s0 - nsteps;
             const uint32_t c = (uint32_t)tid < (uint32_t)a.G ? rg_pre[tid] : 0u;
-            const uint32_t incl = block_incl_scan(c, wsum[0], E);
+            const uint32_t incl = block_incl_scan(c, sh->wsum[0], E);
             if ((uint32_t)tid < (uint32_t)a.G) rg_pre[tid] = incl - c;
             __syncthreads();
             ent0 = (uint32_t)tid < E ? rentry((uint32_t)tid) : 0u;
@@ -955,8 +967,9 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         if (kPl && full && g == 0 && tid == 0) a.fcnt[(kwin + 1) & 1] = 0u;
         if (full && g == 0 && tid == 0) ctl->tbase[bcur] = s0;
         if (tid == 0) {
-            se_blk = 0ull;
-            lsp_n = 0u;
+            sh->se = 0ull;
+            sh->n = 0u;
+            if (kw == 0) sh->bad = 0u;
         }
         const int32_t* lastA = kPl ? a.last3 + (size_t)bprev * a.last_stride : nullptr;   // window k-1 start
         const int32_t* lastB = kPl ? a.last3 + (size_t)bcur * a.last_stride : a.last;     // window k-1 end
@@ -976,7 +989,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         if (kCls && kw == 0) {
             // (precomputed per tile by k_tile_ccache: one load instead of a chain of three)
             for (int32_t k = tid; k < 4 * kClassCache; k += bd) ccache[k] = a.tile_cc[(size_t)g * 4 * kClassCache + k];
-            if (tid < 2) ccls[tid] = a.tile_ccls[2 * g + tid];
+            if (tid < 2) sh->ccls[tid] = a.tile_ccls[2 * g + tid];
         }
         // 1. ring slice -> LDS.  The slots the previous window consumed ([sprev, s0)
         // mod D) were cleared by it and not stored back (step 4): they are zero here.
@@ -1056,7 +1069,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             }
             sb ^= 1;
             uint32_t total;
-            const uint32_t incl = block_incl_scan(items, wsum[sb], total);
+            const uint32_t incl = block_incl_scan(items, sh->wsum[sb], total);
             // (without items nothing waits between this and the spike list that takes the records' place)
             if (total > 0u && (uint32_t)tid < nb)
                 sp_rec[tid] = make_uint2(beg - (incl - items) * (uint32_t)CH,
@@ -1120,29 +1133,22 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                             // multiples of kSubAlign words; the words past the sub-row's end
                             // are padding, the next sub-row or the slack after the last one)
                             const uint16_t* p16 = a.syn16 + kb[h];
+                            // (x[h][u]: the 32 bits that hold word u, low half for even u)
                             if constexpr (CH == 2) {
-                                const uint32_t v = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p16));
-                                x[h][0] = v & 0xFFFFu;
-                                x[h][1] = v >> 16;
+                                x[h][0] = x[h][1] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p16));
                             } else if constexpr (CH == 4) {
                                 const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p16));
-                                x[h][0] = v.x & 0xFFFFu;
-                                x[h][1] = v.x >> 16;
-                                x[h][2] = v.y & 0xFFFFu;
-                                x[h][3] = v.y >> 16;
+                                x[h][0] = x[h][1] = v.x;
+                                x[h][2] = x[h][3] = v.y;
                             } else {
     #pragma unroll
                                 for (int v8 = 0; v8 < CH / 8; ++v8) {
                                     const u32x4 v =
                                         __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p16) + v8);
-                                    x[h][8 * v8 + 0] = v.x & 0xFFFFu;
-                                    x[h][8 * v8 + 1] = v.x >> 16;
-                                    x[h][8 * v8 + 2] = v.y & 0xFFFFu;
-                                    x[h][8 * v8 + 3] = v.y >> 16;
-                                    x[h][8 * v8 + 4] = v.z & 0xFFFFu;
-                                    x[h][8 * v8 + 5] = v.z >> 16;
-                                    x[h][8 * v8 + 6] = v.w & 0xFFFFu;
-                                    x[h][8 * v8 + 7] = v.w >> 16;
+                                    x[h][8 * v8 + 0] = x[h][8 * v8 + 1] = v.x;
+                                    x[h][8 * v8 + 2] = x[h][8 * v8 + 3] = v.y;
+                                    x[h][8 * v8 + 4] = x[h][8 * v8 + 5] = v.z;
+                                    x[h][8 * v8 + 6] = x[h][8 * v8 + 7] = v.w;
                                 }
                             }
                             continue;
@@ -1252,21 +1258,32 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                             const bool valid = (uint32_t)u < cnt[h];
                             const uint32_t xw = x[h][u];
                             if (!kPl) {
-                                uint32_t at = row[h] + ((xw & (WK == kTClass16 ? 0x7FFFu : 0xFFFFu)) << 2);
+                                // (the builtins and empty asm statements keep the shortest forms:
+                                // one field extract, one shift-and-add, and a masked block of one
+                                // instruction, which takes no branch)
+                                uint32_t e = WK == kTClass16 ? __builtin_amdgcn_ubfe(xw, 16u * (u & 1), 15u) : xw & 0xFFFFu;
+                                asm("" : "+v"(e));
+                                uint32_t at = row[h] + (e << 2);
                                 at = min(at, at - R4);              // wraps at the slice's end
+                                auto* word = reinterpret_cast<__attribute__((address_space(3))) uint32_t*>(at);
                                 if (WK == kTClass16) {
-                                    if (valid)
-                                        atomicAdd(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(ring) + at),
-                                                  1u << ((xw >> 11) & 16u));
+                                    uint32_t sg = (u & 1) ? xw >> 31 : __builtin_amdgcn_ubfe(xw, 15u, 1u);
+                                    asm("" : "+v"(sg));
+                                    uint32_t one = __umul24(sg, 0xFFFFu) + 1u;      // 1 or 0x10000
+                                    asm("" : "+v"(one));
+                                    if (valid) __hip_atomic_fetch_add(word, one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                                 } else {
                                     float w;                        // times the fixed-point scale
                                     if (WK == kTBF16) w = bf16_to_f32((uint16_t)(xw >> 16)) * rs[h];
                                     else if (WK == kTFP8) w = fp8e4m3_to_f32((uint8_t)(xw >> 16)) * rs[h];
                                     else w = wv[h][u] * fsc.x;
-                                    if (RW == 2) at += w > 0.f ? 0u : R4;   // (one ring: both signs in one sum)
+                                    // (one ring: both signs in one sum)
+                                    if (RW == 2) word += w > 0.f ? 0u : R4 / 4u;
+                                    int32_t v = (int32_t)rintf(w);
+                                    asm("" : "+v"(v));
                                     if (valid)
-                                        atomicAdd(reinterpret_cast<int32_t*>(reinterpret_cast<char*>(ring) + at),
-                                                  (int32_t)rintf(w));
+                                        __hip_atomic_fetch_add(word, (uint32_t)v, __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_WORKGROUP);
                                 }
                             } else {
                                 int32_t slot = sD[h] + (int32_t)((xw >> 11) & 31u) + 1;
@@ -1349,7 +1366,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 const uint32_t leader = (uint32_t)__ffsll((unsigned long long)m) - 1u;
                 const uint32_t pc = (uint32_t)__popcll(m);
                 uint32_t lb = 0u;
-                if (lane_id() == leader) lb = atomicAdd(&lsp_n, pc);
+                if (lane_id() == leader) lb = atomicAdd(&sh->n, pc);
                 lb = __shfl(lb, (int)leader);
                 const uint32_t cap = (uint32_t)kTiledBatch;
                 const uint32_t over0 = max(lb, cap);                 // first index past the LDS list
@@ -1519,24 +1536,24 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             if (own) own_st = st;
             else if (active) store_neuron(i, st);
         }
-        if (se_local) atomicAdd(&se_blk, se_local);
+        if (se_local) atomicAdd(&sh->se, se_local);
         __syncthreads();
-        const uint32_t nl = min(lsp_n, (uint32_t)kTiledBatch);
+        const uint32_t nl = min(sh->n, (uint32_t)kTiledBatch);
         if (tid == 0) {
             if (rgp) {
                 // region window: no list space to reserve; the counters wait for the
                 // launch's last window (records still take their places now)
-                se_acc += se_blk;
-                if (!a.rec) spk_acc += lsp_n;
-                else if (nl) lsp_r = atomicAdd((unsigned long long*)&ctl->rec_cnt, (unsigned long long)nl);
+                se_acc += sh->se;
+                if (!a.rec) spk_acc += sh->n;
+                else if (nl) sh->rec_at = atomicAdd((unsigned long long*)&ctl->rec_cnt, (unsigned long long)nl);
             } else {
-                if (se_blk + se_acc) atomicAdd((unsigned long long*)&ctl->se, se_blk + se_acc);
+                if (sh->se + se_acc) atomicAdd((unsigned long long*)&ctl->se, sh->se + se_acc);
                 if (spk_acc) atomicAdd((unsigned long long*)&ctl->rec_cnt, spk_acc);
                 se_acc = 0ull;
                 spk_acc = 0ull;
                 if (nl) {
-                    lsp_g = atomicAdd(&tcnt[bcur * nseg], nl);
-                    lsp_r = atomicAdd((unsigned long long*)&ctl->rec_cnt, (unsigned long long)nl);
+                    sh->list_at = atomicAdd(&tcnt[bcur * nseg], nl);
+                    sh->rec_at = atomicAdd((unsigned long long*)&ctl->rec_cnt, (unsigned long long)nl);
                 }
             }
         }
@@ -1550,12 +1567,12 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             if (rgp) {
                 // (the entry is in the region already)
             } else if (PW) {
-                st_agent(&wbuf[lsp_g + k], ent);
+                st_agent(&wbuf[sh->list_at + k], ent);
             } else {
-                wbuf[lsp_g + k] = ent;
+                wbuf[sh->list_at + k] = ent;
             }
             if (a.rec) {
-                const uint64_t at = lsp_r + k;
+                const uint64_t at = sh->rec_at + k;
                 if (at < a.rec_cap)
                     a.rec[at] = ((uint64_t)(uint32_t)(s0 + (int64_t)(ent >> 26)) << 32) | (ent & kIdMask);
                 else ctl->rec_overflow = 1;
@@ -1563,8 +1580,8 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         }
         if constexpr (PW) {
             if (kw + 1 < nw &&
-                !grid_wait(a.bar, (uint32_t)a.G, (uint32_t)g, (uint32_t)(kwin + 1), rgp ? lsp_n : 0u,
-                           rgn_on ? rg_pre : nullptr, gt0, gt1, a.bar_err, a.spin_limit))
+                !grid_wait(a.bar, (uint32_t)a.G, (uint32_t)g, (uint32_t)(kwin + 1), rgp ? sh->n : 0u,
+                           rgn_on ? rg_pre : nullptr, gt0, gt1, a.bar_err, a.spin_limit, &sh->bad))
                 return;
         }
     }   // windows
