@@ -133,9 +133,15 @@ struct mgb_sim {
     uint32_t* bar_err = nullptr;       // set by a wait that timed out
     uint64_t spin_limit = 0;           // wall-clock ticks
     bool failed = false;               // a persistent launch timed out: results void
-    uint32_t* h_err = nullptr;         // pinned host copy of *bar_err, written at the end of each run
-    uint32_t* h_err_dev = nullptr;     // its address on the device (the run's last kernel writes it)
-    bool err_pending = false;          // h_err is due with the stream's completion
+    HostMirror* mir = nullptr;         // pinned host copy of *ctl and *bar_err, written at the end of each run
+    HostMirror* mir_dev = nullptr;     // its address on the device (the run's last kernel writes it)
+    bool err_pending = false;          // mir->err is due with the stream's completion
+    // read-back of large arrays: two pinned buffers (kStageBytes each) and the device
+    // workspace that sorts spike records, kept from the first such call on
+    uint8_t* stage[2] = {nullptr, nullptr};
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};
+    uint8_t* rd_ws = nullptr;
+    size_t rd_ws_bytes = 0;
     int xcd_map = -1;                  // fused launches: XCD-contiguous tile order (-1: not computed yet)
     int region = 0;                    // persistent launches: per-tile list regions (TiledArgs::region)
     uint64_t tile_hash = 0;            // FNV-1a of the tile boundaries (the ring slices' layout)
@@ -240,7 +246,11 @@ void free_all(mgb_sim* s) {
     if (s->ev0) (void)hipEventDestroy(s->ev0);
     if (s->ev1) (void)hipEventDestroy(s->ev1);
     if (s->stream) (void)hipStreamDestroy(s->stream);
-    if (s->h_err) (void)hipHostFree(s->h_err);
+    for (int k = 0; k < 2; ++k) {
+        if (s->stage_ev[k]) (void)hipEventDestroy(s->stage_ev[k]);
+        if (s->stage[k]) (void)hipHostFree(s->stage[k]);
+    }
+    if (s->mir) (void)hipHostFree(s->mir);
 }
 
 // Per-neuron host inputs common to both construction paths.
@@ -1053,6 +1063,9 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
     std::memcpy(s->sc, h.stdpconst, sizeof(s->sc));
     const size_t np = (size_t)s->npad;
     MGB_TRY(dalloc_n(s, &s->ctl, 1));
+    MGB_HIP_TRY(hipHostMalloc((void**)&s->mir, sizeof(HostMirror), hipHostMallocMapped));
+    std::memset(s->mir, 0, sizeof(HostMirror));
+    MGB_HIP_TRY(hipHostGetDevicePointer((void**)&s->mir_dev, s->mir, 0));
     MGB_TRY(dalloc_n(s, &s->type, np));
     MGB_TRY(dalloc_n(s, &s->cset, np));
     MGB_TRY(dalloc_n(s, &s->stream_idx, np));
@@ -1175,9 +1188,6 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
             khz = 100000;
         const uint64_t us = (o && o->spin_limit_us > 0) ? (uint64_t)o->spin_limit_us : 2000000ull;
         s->spin_limit = us * (uint64_t)khz / 1000ull;
-        MGB_HIP_TRY(hipHostMalloc((void**)&s->h_err, 4, hipHostMallocMapped));
-        *s->h_err = 0u;
-        MGB_HIP_TRY(hipHostGetDevicePointer((void**)&s->h_err_dev, s->h_err, 0));
     }
     if (s->tiled) update_persist(s);
     MGB_HIP_TRY(hipStreamSynchronize(st));
@@ -1387,8 +1397,8 @@ mgb_status issue_windows(mgb_sim* s, int32_t nsteps, bool finalize, bool capturi
             ++wk;
         }
         if (finalize) {
-            MGB_HIP_TRY(launch_finalize_tiled(s->ctl, nsteps, wk, s->persist ? s->bar_err : nullptr,
-                                              s->persist ? s->h_err_dev : nullptr, s->stream));
+            MGB_HIP_TRY(launch_finalize_tiled(s->ctl, nsteps, wk, s->persist ? s->bar_err : nullptr, s->mir_dev,
+                                              s->stream));
             s->launches += 1;
         }
         return MGB_OK;
@@ -1416,7 +1426,7 @@ mgb_status issue_windows(mgb_sim* s, int32_t nsteps, bool finalize, bool capturi
         ++wk;
     }
     if (finalize) {
-        MGB_HIP_TRY(launch_finalize(s->ctl, nsteps, wk, s->stream));
+        MGB_HIP_TRY(launch_finalize(s->ctl, nsteps, wk, s->mir_dev, s->stream));
         s->launches += 1;
     }
     return MGB_OK;
@@ -1872,7 +1882,7 @@ mgb_status mgb_run(mgb_sim* s, int32_t nsteps) {
     if (nsteps - done > 0) MGB_TRY(issue_windows(s, nsteps - done, true));
     // the waits' error word comes back with the run (the finalize kernel writes it to
     // pinned host memory; mgb_sync reads it)
-    if (s->persist && s->h_err) s->err_pending = true;
+    if (s->persist) s->err_pending = true;
     MGB_HIP_TRY(hipEventRecord(s->ev1, s->stream));
     s->timed = true;
     return MGB_OK;
@@ -1886,7 +1896,7 @@ mgb_status mgb_sync(mgb_sim* s) {
     MGB_HIP_TRY(hipSetDevice(s->device));
     MGB_HIP_TRY(hipStreamSynchronize(s->stream));
     if (s->err_pending) {
-        s->failed = s->failed || *s->h_err != 0u;
+        s->failed = s->failed || s->mir->err != 0u;
         s->err_pending = false;
     }
     if (s->failed) {
@@ -1928,8 +1938,7 @@ mgb_status mgb_get_info(mgb_sim* s, mgb_info* out) {
         return MGB_ERR_INVALID;
     }
     MGB_TRY(mgb_sync(s));
-    Ctl c;
-    MGB_HIP_TRY(hipMemcpy(&c, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+    const Ctl c = s->mir->ctl;
     std::memset(out, 0, sizeof(*out));
     out->n_neurons = s->n;
     out->ring_len = s->D;
@@ -1977,22 +1986,103 @@ mgb_status mgb_get_info(mgb_sim* s, mgb_info* out) {
     return MGB_OK;
 }
 
+namespace {
+
+// Device memory to pageable host memory.  Large copies go through two pinned buffers of
+// the simulator, the host copying one out while the other fills.
+constexpr size_t kStageBytes = size_t(4) << 20;
+
+mgb_status copy_out(mgb_sim* s, void* dst, const void* src, size_t bytes) {
+    if (bytes < 2 * kStageBytes) {
+        if (bytes) MGB_HIP_TRY(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+        return MGB_OK;
+    }
+    for (int k = 0; k < 2; ++k) {
+        if (!s->stage[k]) MGB_HIP_TRY(hipHostMalloc((void**)&s->stage[k], kStageBytes, hipHostMallocDefault));
+        if (!s->stage_ev[k]) MGB_HIP_TRY(hipEventCreateWithFlags(&s->stage_ev[k], hipEventDisableTiming));
+    }
+    const uint8_t* from = static_cast<const uint8_t*>(src);
+    uint8_t* to = static_cast<uint8_t*>(dst);
+    const size_t n = (bytes + kStageBytes - 1) / kStageBytes;
+    for (size_t k = 0; k <= n; ++k) {
+        if (k < n) {
+            const size_t len = std::min(kStageBytes, bytes - k * kStageBytes);
+            MGB_HIP_TRY(hipMemcpyAsync(s->stage[k & 1], from + k * kStageBytes, len, hipMemcpyDeviceToHost, s->stream));
+            MGB_HIP_TRY(hipEventRecord(s->stage_ev[k & 1], s->stream));
+        }
+        if (k > 0) {
+            const size_t j = k - 1;
+            MGB_HIP_TRY(hipEventSynchronize(s->stage_ev[j & 1]));
+            std::memcpy(to + j * kStageBytes, s->stage[j & 1], std::min(kStageBytes, bytes - j * kStageBytes));
+        }
+    }
+    return MGB_OK;
+}
+
+// Spike records from this many on are sorted on the device.
+constexpr uint64_t kDeviceSortMin = 2048;
+
+// The first w of the `have` records in order of (step, id): radix-sorted on the device by
+// the id's bits, then the step's (the record itself stays as it is), and split into the
+// caller's two arrays.  *done stays false where the workspace cannot be allocated.
+mgb_status read_records_sorted(mgb_sim* s, uint64_t have, uint64_t w, int32_t* steps, int32_t* ids, bool* done) {
+    const Ctl& c = s->mir->ctl;
+    const int ibits = bits_for((uint64_t)s->n);
+    const int sbits = c.base_step > 0x7FFFFFFFll ? 32 : bits_for((uint64_t)c.base_step);
+    size_t t1 = 0, t2 = 0;
+    MGB_HIP_TRY(sort_keys64(nullptr, &t1, nullptr, nullptr, have, 0, ibits, s->stream));
+    MGB_HIP_TRY(sort_keys64(nullptr, &t2, nullptr, nullptr, have, 32, 32 + sbits, s->stream));
+    const size_t keys = (8 * (size_t)have + 255) & ~(size_t)255, temp = std::max(t1, t2);
+    const size_t need = 2 * keys + temp;
+    if (need > s->rd_ws_bytes) {
+        if (s->rd_ws) {
+            dfree(s, s->rd_ws);
+            s->bytes -= (int64_t)s->rd_ws_bytes;
+            s->rd_ws = nullptr;
+            s->rd_ws_bytes = 0;
+        }
+        const size_t room = need + need / 4;
+        if (dalloc_n(s, &s->rd_ws, room) != MGB_OK) {
+            (void)hipGetLastError();
+            return MGB_OK;
+        }
+        s->rd_ws_bytes = room;
+    }
+    uint64_t* a = reinterpret_cast<uint64_t*>(s->rd_ws);
+    uint64_t* b = reinterpret_cast<uint64_t*>(s->rd_ws + keys);
+    void* tmp = s->rd_ws + 2 * keys;
+    MGB_HIP_TRY(sort_keys64(tmp, &t1, s->rec, a, have, 0, ibits, s->stream));
+    MGB_HIP_TRY(sort_keys64(tmp, &t2, a, b, have, 32, 32 + sbits, s->stream));
+    int32_t* col = reinterpret_cast<int32_t*>(a);              // both columns in the first buffer
+    MGB_HIP_TRY(split_records(b, w, col, col + w, s->stream));
+    MGB_HIP_TRY(hipStreamSynchronize(s->stream));
+    MGB_TRY(copy_out(s, steps, col, 4 * w));
+    MGB_TRY(copy_out(s, ids, col + w, 4 * w));
+    *done = true;
+    return MGB_OK;
+}
+
+}  // namespace
+
 mgb_status mgb_read_spikes(mgb_sim* s, int64_t cap, int32_t* steps, int32_t* ids, int64_t* n_out) {
     if (!s || cap < 0 || (cap > 0 && (!steps || !ids)) || !n_out) {
         set_error("invalid arguments to mgb_read_spikes");
         return MGB_ERR_INVALID;
     }
     MGB_TRY(mgb_sync(s));
-    Ctl c;
-    MGB_HIP_TRY(hipMemcpy(&c, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+    const Ctl c = s->mir->ctl;
     const uint64_t have = std::min<uint64_t>(c.rec_cnt, (uint64_t)s->rec_cap);
-    std::vector<uint64_t> r(have);
-    if (have) MGB_HIP_TRY(hipMemcpy(r.data(), s->rec, 8 * have, hipMemcpyDeviceToHost));
-    std::sort(r.begin(), r.end());
     const uint64_t w = std::min<uint64_t>(have, (uint64_t)cap);
-    for (uint64_t k = 0; k < w; ++k) {
-        steps[k] = (int32_t)(r[k] >> 32);
-        ids[k] = (int32_t)(r[k] & 0xFFFFFFFFu);
+    bool sorted = false;
+    if (have >= kDeviceSortMin) MGB_TRY(read_records_sorted(s, have, w, steps, ids, &sorted));
+    if (!sorted) {
+        std::vector<uint64_t> r(have);
+        if (have) MGB_HIP_TRY(hipMemcpy(r.data(), s->rec, 8 * have, hipMemcpyDeviceToHost));
+        std::sort(r.begin(), r.end());
+        for (uint64_t k = 0; k < w; ++k) {
+            steps[k] = (int32_t)(r[k] >> 32);
+            ids[k] = (int32_t)(r[k] & 0xFFFFFFFFu);
+        }
     }
     *n_out = (int64_t)w;
     if (c.rec_cnt > (uint64_t)s->rec_cap || c.rec_overflow || w < have) {
@@ -2009,11 +2099,11 @@ mgb_status mgb_clear_spikes(mgb_sim* s) {
         return MGB_ERR_INVALID;
     }
     MGB_TRY(mgb_sync(s));
-    Ctl c;
-    MGB_HIP_TRY(hipMemcpy(&c, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+    Ctl c = s->mir->ctl;
     c.rec_cnt = 0;
     c.rec_overflow = 0;
     MGB_HIP_TRY(hipMemcpy(s->ctl, &c, sizeof(Ctl), hipMemcpyHostToDevice));
+    s->mir->ctl = c;
     return MGB_OK;
 }
 
@@ -2037,8 +2127,7 @@ mgb_status mgb_read_state(mgb_sim* s, int32_t field, void* out) {
     MGB_TRY(mgb_sync(s));
     if (field == MGB_F_LAST && s->tiled && stdp_kind(s->tkind)) {
         // the next window reads buffer base_window % 3
-        Ctl c;
-        MGB_HIP_TRY(hipMemcpy(&c, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+        const Ctl c = s->mir->ctl;
         src = s->last + (size_t)(c.base_window % 3) * (size_t)s->npad;
     }
     MGB_HIP_TRY(hipMemcpy(out, src, 4 * (size_t)s->n, hipMemcpyDeviceToHost));
@@ -2110,8 +2199,7 @@ CkptHeader ckpt_header(const mgb_sim* s, uint64_t n_rec) {
 }
 
 mgb_status ckpt_records(mgb_sim* s, uint64_t* n_rec) {
-    Ctl c;
-    MGB_HIP_TRY(hipMemcpy(&c, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+    const Ctl c = s->mir->ctl;
     *n_rec = std::min<uint64_t>(c.rec_cnt, (uint64_t)s->rec_cap);
     return MGB_OK;
 }
@@ -2190,6 +2278,7 @@ mgb_status mgb_checkpoint_load(mgb_sim* s, const void* buf, int64_t bytes) {
         if (g.bytes) MGB_HIP_TRY(hipMemcpy(g.p, in + off, g.bytes, hipMemcpyHostToDevice));
         off += g.bytes;
     }
+    MGB_HIP_TRY(hipMemcpy(&s->mir->ctl, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
     // the persistent waits' flags hold window indices of the run before (epochs)
     if (s->bar) MGB_HIP_TRY(hipMemset(s->bar, 0, 4 * (size_t)s->G * kBarStride));
     return MGB_OK;
@@ -2298,58 +2387,22 @@ mgb_status mgb_read_csr(mgb_sim* s, int64_t* row_ptr, int32_t* col, int32_t* del
         }
         return MGB_OK;
     }
-    if (col && S) MGB_HIP_TRY(hipMemcpy(col, s->col, 4 * S, hipMemcpyDeviceToHost));
+    if (col) MGB_TRY(copy_out(s, col, s->col, 4 * S));
     std::vector<uint8_t> dl;
-    if (delay || (weight && s->wide_kind != kWideF32)) {
+    if (delay) {
         dl.resize(S);
         if (S) MGB_HIP_TRY(hipMemcpy(dl.data(), s->dly, S, hipMemcpyDeviceToHost));
-    }
-    if (delay)
         for (size_t k = 0; k < S; ++k) delay[k] = (int32_t)(dl[k] & 127u);
+    }
     if (weight && S) {
         if (s->tiled && stdp_kind(s->tkind)) MGB_TRY(current_weights(s));
-        MGB_HIP_TRY(hipMemcpy(weight, s->w32, 4 * S, hipMemcpyDeviceToHost));
-        if (s->wide_kind == kWideBF16) {
-            std::vector<uint16_t> w16(S);
-            std::vector<float> rs((size_t)s->n);
-            std::vector<int64_t> rp((size_t)s->n + 1);
-            MGB_HIP_TRY(hipMemcpy(w16.data(), s->w16, 2 * S, hipMemcpyDeviceToHost));
-            MGB_HIP_TRY(hipMemcpy(rs.data(), s->row_scale, 4 * (size_t)s->n, hipMemcpyDeviceToHost));
-            MGB_HIP_TRY(hipMemcpy(rp.data(), s->row_ptr, 8 * ((size_t)s->n + 1), hipMemcpyDeviceToHost));
-            for (int32_t i = 0; i < s->n; ++i)
-                for (int64_t k = rp[i]; k < rp[i + 1]; ++k) {
-                    if (dl[k] & 128u) continue;
-                    const uint32_t b = (uint32_t)w16[k] << 16;
-                    float v;
-                    std::memcpy(&v, &b, 4);
-                    weight[k] = v * rs[i];                  // as the kernels decode it
-                }
-        } else if (s->wide_kind == kWideFP8) {
-            std::vector<uint8_t> w8(S);
-            std::vector<float> rs((size_t)s->n);
-            std::vector<int64_t> rp((size_t)s->n + 1);
-            MGB_HIP_TRY(hipMemcpy(w8.data(), s->w8, S, hipMemcpyDeviceToHost));
-            MGB_HIP_TRY(hipMemcpy(rs.data(), s->row_scale, 4 * (size_t)s->n, hipMemcpyDeviceToHost));
-            MGB_HIP_TRY(hipMemcpy(rp.data(), s->row_ptr, 8 * ((size_t)s->n + 1), hipMemcpyDeviceToHost));
-            for (int32_t i = 0; i < s->n; ++i)
-                for (int64_t k = rp[i]; k < rp[i + 1]; ++k) {
-                    if (dl[k] & 128u) continue;
-                    const uint8_t b = w8[k];
-                    const uint32_t sg = (uint32_t)(b >> 7) << 31, e = (b >> 3) & 15u, m = b & 7u;
-                    float v;
-                    if (e == 0) {
-                        v = (float)m * 0x1p-9f;
-                        uint32_t u;
-                        std::memcpy(&u, &v, 4);
-                        u |= sg;
-                        std::memcpy(&v, &u, 4);
-                    } else {
-                        const uint32_t u = sg | ((e + 120u) << 23) | (m << 20);
-                        std::memcpy(&v, &u, 4);
-                    }
-                    weight[k] = v * rs[i];
-                }
-        }
+        // BF16 / FP8: decoded on the device in place (the FP32 copy of a static synapse is
+        // read by nothing else)
+        if (s->wide_kind != kWideF32)
+            MGB_HIP_TRY(wide_weights(s->row_ptr, s->n, s->dly, s->w32, s->wide_kind == kWideBF16 ? s->w16 : nullptr,
+                                     s->wide_kind == kWideFP8 ? s->w8 : nullptr, s->row_scale, s->w32, s->stream));
+        MGB_HIP_TRY(hipStreamSynchronize(s->stream));
+        MGB_TRY(copy_out(s, weight, s->w32, 4 * S));
     }
     return MGB_OK;
 }

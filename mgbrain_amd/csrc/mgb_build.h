@@ -84,6 +84,11 @@ hipError_t make_sort_input(const int32_t* src, const int32_t* tar, const float* 
                            hipStream_t st);
 hipError_t make_tile_keys(const int32_t* src, const int32_t* tar, const float* w, const uint8_t* dq,
                           const TileTabs& tt, uint32_t* keys, uint32_t* vals, uint64_t S, hipStream_t st);
+// Stable radix sort of 64-bit keys by their bits [bit0, bit1) (temp as sort_pairs).
+hipError_t sort_keys64(void* temp, size_t* temp_bytes, const uint64_t* kin, uint64_t* kout, uint64_t n, int bit0,
+                       int bit1, hipStream_t st);
+// Spike records (step << 32 | id) into their two columns.
+hipError_t split_records(const uint64_t* r, uint64_t n, int32_t* steps, int32_t* ids, hipStream_t st);
 hipError_t class16_words(const uint32_t* w32, uint64_t S, const TileTabs& tt, uint16_t* out, hipStream_t st);
 hipError_t make_tile_keys_csr(const uint32_t* src, const int32_t* col, const TileTabs& tt, uint32_t* keys,
                               uint32_t* vals, uint64_t S, hipStream_t st);

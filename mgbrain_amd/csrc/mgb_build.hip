@@ -130,6 +130,15 @@ __global__ void k_tile_keys(const int32_t* src, const int32_t* tar, const float*
 
 // 16-bit CLASS words (tiles of at most 1024 targets): tile-local target |
 // delay-1 << 10 | inhibitory << 15, from the 32-bit words in tile order.
+__global__ void k_split_records(const uint64_t* r, uint64_t n, int32_t* steps, int32_t* ids) {
+    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
+         k += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t x = r[k];
+        steps[k] = (int32_t)(x >> 32);
+        ids[k] = (int32_t)(uint32_t)x;
+    }
+}
+
 __global__ void k_class16(const uint32_t* w32, uint64_t S, TileTabs tt, uint16_t* out) {
     for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < S;
          k += (uint64_t)gridDim.x * blockDim.x) {
@@ -687,6 +696,20 @@ hipError_t sort_pairs(void* temp, size_t* temp_bytes, const uint32_t* kin, uint3
                                              (unsigned)bits, st);
     if (!temp) *temp_bytes = sz;
     return e;
+}
+
+hipError_t sort_keys64(void* temp, size_t* temp_bytes, const uint64_t* kin, uint64_t* kout, uint64_t n, int bit0,
+                       int bit1, hipStream_t st) {
+    size_t sz = temp ? *temp_bytes : 0;
+    hipError_t e = rocprim::radix_sort_keys(temp, sz, kin, kout, (size_t)n, (unsigned)bit0, (unsigned)bit1, st);
+    if (!temp) *temp_bytes = sz;
+    return e;
+}
+
+hipError_t split_records(const uint64_t* r, uint64_t n, int32_t* steps, int32_t* ids, hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_split_records, dim3(blocks_for(n, 256)), dim3(256), 0, st, r, n, steps, ids);
+    return hipGetLastError();
 }
 
 hipError_t row_bounds(const uint32_t* sorted_keys, uint64_t S, int32_t n, int64_t* out,

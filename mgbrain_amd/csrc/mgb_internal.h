@@ -55,6 +55,13 @@ struct Ctl {
 };
 
 
+// Pinned host memory that a run's last kernel fills: the persistent waits' error word and
+// a copy of the control block, so that reading counters after a run is no copy of its own.
+struct HostMirror {
+    Ctl ctl;
+    uint32_t err, pad;
+};
+
 // Constant set: LIFECONSTS[30] (mgcore.cu:32-63) + refractory steps in c[30].
 struct CSet {
     float c[32];
@@ -276,7 +283,8 @@ hipError_t launch_neurons(int mode, const NeuArgs& a, int32_t off, int32_t wk, i
 hipError_t launch_prop(int mode, int wide_kind, const PropArgs& a, int32_t off, int32_t wk,
                        int grid, int block, hipStream_t st);
 hipError_t launch_stdp(const StdpArgs& a, int32_t off, int32_t wk, int grid, hipStream_t st);
-hipError_t launch_finalize(Ctl* ctl, int32_t steps, int32_t windows, hipStream_t st);
+// (m: the host mirror's address on the device)
+hipError_t launch_finalize(Ctl* ctl, int32_t steps, int32_t windows, HostMirror* m, hipStream_t st);
 constexpr int kTiledBatch = 1024;   // spikes staged in LDS per propagation batch
 constexpr int kTiledItems = 16384;  // work items staged in LDS per propagation round
 constexpr int kTiledStaticLds = 1024; // bytes reserved for the fused kernel's static LDS
@@ -318,8 +326,8 @@ hipError_t set_tiled_pw_lds_limit(const TiledArgs& a);
 // window index goes back (a restored checkpoint).
 hipError_t launch_tiled_persistent(const TiledArgs& a, int32_t off, int32_t wk, int32_t nsteps, int32_t nwin,
                                    int block, hipStream_t st);
-// err, h_err: the persistent waits' error word and its pinned host copy (or null)
-hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, uint32_t* h_err,
+// err: the persistent waits' error word (or null)
+hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, HostMirror* m,
                                  hipStream_t st);
 hipError_t set_tiled_lds_limit(int kind, size_t bytes);
 // kTStdp: brings the plastic in-synapses of the neurons the fused kernel listed

@@ -496,14 +496,28 @@ __global__ void k_stdp(StdpArgs a, int32_t off, int32_t wk) {
     }
 }
 
-__global__ void k_finalize(Ctl* ctl, int32_t steps, int32_t windows) {
-    const int par = (int)((ctl->base_window + windows - 1) & 1);
-    if (windows > 0) {
-        ctl->rec_cnt += ctl->win_cnt[par];
-        ctl->win_cnt[par] = 0u;
+// The control block into the host mirror (one wave, after thread 0's changes to it).
+__device__ __forceinline__ void mirror_ctl(const Ctl* ctl, HostMirror* m) {
+    __threadfence_block();
+    __syncthreads();
+    static_assert(sizeof(Ctl) % 4 == 0 && sizeof(Ctl) / 4 <= 64, "one word per lane");
+    if (threadIdx.x < sizeof(Ctl) / 4)
+        __hip_atomic_store(reinterpret_cast<uint32_t*>(&m->ctl) + threadIdx.x,
+                           reinterpret_cast<const volatile uint32_t*>(ctl)[threadIdx.x], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void k_finalize(Ctl* ctl, int32_t steps, int32_t windows, HostMirror* m) {
+    if (threadIdx.x == 0) {
+        const int par = (int)((ctl->base_window + windows - 1) & 1);
+        if (windows > 0) {
+            ctl->rec_cnt += ctl->win_cnt[par];
+            ctl->win_cnt[par] = 0u;
+        }
+        ctl->base_step += steps;
+        ctl->base_window += windows;
     }
-    ctl->base_step += steps;
-    ctl->base_window += windows;
+    mirror_ctl(ctl, m);
 }
 
 
@@ -1707,12 +1721,15 @@ __global__ __launch_bounds__(256) void k_stdp_flush(TiledArgs a, int32_t off, in
     }
 }
 
-// End of a run: the step and window counters move on, and the persistent waits'
-// error word goes to the host (pinned memory the host reads after the run).
-__global__ void k_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, uint32_t* h_err) {
-    ctl->base_step += steps;
-    ctl->base_window += windows;
-    if (err && h_err) __hip_atomic_store(h_err, *err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+// End of a run: the step and window counters move on, and the control block and the
+// persistent waits' error word go to the host (pinned memory the host reads after the run).
+__global__ void k_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, HostMirror* m) {
+    if (threadIdx.x == 0) {
+        ctl->base_step += steps;
+        ctl->base_window += windows;
+        if (err) __hip_atomic_store(&m->err, *err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    mirror_ctl(ctl, m);
 }
 
 }  // namespace
@@ -1751,8 +1768,8 @@ hipError_t launch_stdp(const StdpArgs& a, int32_t off, int32_t wk, int grid, hip
     return hipGetLastError();
 }
 
-hipError_t launch_finalize(Ctl* ctl, int32_t steps, int32_t windows, hipStream_t st) {
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1), 0, st, ctl, steps, windows);
+hipError_t launch_finalize(Ctl* ctl, int32_t steps, int32_t windows, HostMirror* m, hipStream_t st) {
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, st, ctl, steps, windows, m);
     return hipGetLastError();
 }
 
@@ -1895,9 +1912,9 @@ hipError_t launch_stdp_flush(const TiledArgs& a, int32_t off, int32_t wk, hipStr
     return hipGetLastError();
 }
 
-hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, uint32_t* h_err,
+hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, HostMirror* m,
                                  hipStream_t st) {
-    hipLaunchKernelGGL(k_finalize_tiled, dim3(1), dim3(1), 0, st, ctl, steps, windows, err, h_err);
+    hipLaunchKernelGGL(k_finalize_tiled, dim3(1), dim3(64), 0, st, ctl, steps, windows, err, m);
     return hipGetLastError();
 }
 
