@@ -66,7 +66,7 @@ typedef struct mgb_opts {
     int32_t propagation;       /* MGB_PROP_* */
     int32_t tile_size;         /* TILED: mean target neurons per workgroup (tiles are balanced by
                                   in-degree and never mix neuron types); 0 = default */
-    int32_t chunk;             /* TILED: synapses per propagation work item (1, 2, 4, 8, 16; 0 = 8) */
+    int32_t chunk;             /* TILED: synapses per propagation work item (1, 2, 4, 8, 16; 0 = tuned default) */
     int32_t persistent;        /* TILED without STDP: MGB_PERSIST_* */
     int32_t spin_limit_us;     /* persistent launches: bound on a workgroup's wait between two
                                   windows before the run fails with MGB_ERR_HIP; 0 = 2 s */

@@ -91,6 +91,7 @@ struct mgb_sim {
     // fused tiled path
     int tiled = 0;
     int32_t B = 0, G = 0, chunk = 8, tblock = 512;
+    bool tblock_auto = false;          // the caller gave no workgroup size
     int32_t trw = 1;                   // fused path: ring words per (slot, target)
     int32_t nseg = 1;
     std::vector<int32_t> h_seg_lo;     // [nseg+1] segment boundaries (independent networks)
@@ -457,8 +458,18 @@ mgb_status choose_tiles(mgb_sim* s, const mgb_opts* o, int32_t n, int32_t D, con
     std::vector<uint32_t> tof((size_t)n);
     for (size_t g = 0; g + 1 < tlo.size(); ++g)
         for (int32_t t = tlo[g]; t < tlo[g + 1]; ++t) tof[t] = (uint32_t)g;
-    s->chunk = (o && (o->chunk == 1 || o->chunk == 2 || o->chunk == 4 || o->chunk == 16)) ? o->chunk : 8;
-    s->tblock = (o && o->prop_block >= 64 && o->prop_block <= 1024) ? (o->prop_block / 64) * 64 : 512;
+    // Launch shape where the caller gives none.  A work item is one 16-byte load: 8 words of
+    // 16 bits or 4 of 32 (BF16 batch of six networks 18.9 us a window with 8, 16.5 with 4;
+    // STDP on 4e7 synapses 35.7, 33.2; conductance nets within 2 %).  The workgroup has a
+    // thread for each neuron of the widest tile, whose state then stays in registers, and
+    // at least 512 (narrower tiles lose with more: 80,000 conductance neurons, tiles of 313,
+    // 8.8 us at 512 and 9.15 at 1024; tiles of 732: 10.4 at 512, 9.8 at 768; of 1024:
+    // 61.4 at 512, 53.4 at 1024).  STDP spends its windows in the synapses: always 1024.
+    s->chunk = (o && (o->chunk == 1 || o->chunk == 2 || o->chunk == 4 || o->chunk == 8 || o->chunk == 16))
+                   ? o->chunk : (s->tkind == kTClass16 ? 8 : 4);
+    s->tblock_auto = !(o && o->prop_block >= 64 && o->prop_block <= 1024);
+    s->tblock = !s->tblock_auto ? (o->prop_block / 64) * 64
+                                : (stdp_kind(s->tkind) || B > 768 ? 1024 : (B > 512 ? 768 : 512));
     std::vector<uint32_t> kbase(nseg + 1, 0);
     std::vector<uint64_t> obase(nseg + 1, 0);
     uint64_t kb = 0, ob = 0;
@@ -1189,7 +1200,20 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
         const uint64_t us = (o && o->spin_limit_us > 0) ? (uint64_t)o->spin_limit_us : 2000000ull;
         s->spin_limit = us * (uint64_t)khz / 1000ull;
     }
-    if (s->tiled) update_persist(s);
+    if (s->tiled) {
+        update_persist(s);
+        if (s->tblock_auto && s->tblock > 512 && !s->persist && !stdp_kind(s->tkind) &&
+            s->persist_req != MGB_PERSIST_OFF) {
+            // (two workgroups of 512 may fit on a CU where one of more does)
+            const int32_t wide = s->tblock;
+            s->tblock = 512;
+            update_persist(s);
+            if (!s->persist) {
+                s->tblock = wide;
+                update_persist(s);
+            }
+        }
+    }
     MGB_HIP_TRY(hipStreamSynchronize(st));
     return MGB_OK;
 }
