@@ -84,7 +84,7 @@ struct mgb_sim {
     float* tbl_w = nullptr;
     float *ltp = nullptr, *ltd = nullptr;
     int32_t lut_n = 1;
-    int32_t lut_lds = 0;               // fused STDP: table entries the fused kernel keeps in LDS
+    int32_t lut_lds = 0;               // fused STDP: table entries the widest tile keeps in LDS
     uint32_t* win_buf = nullptr;
     uint32_t win_stride = 0;
     uint64_t* rec = nullptr;
@@ -1328,7 +1328,8 @@ TiledArgs tiled_args(const mgb_sim* s) {
         a.hist = s->hist; a.tf = s->tf; a.cntf = s->cntf;
         a.flist = s->flist; a.fcnt = s->fcnt; a.flist_cap = (uint32_t)s->npad;
         a.din_ptr = s->in_ptr; a.din_pos = s->in_pos; a.din_src = s->in_src;
-        a.ltp = s->ltp; a.ltd = s->ltd; a.lut_n = s->lut_n; a.lut_lds = s->lut_lds;
+        a.ltp = s->ltp; a.ltd = s->ltd; a.lut_n = s->lut_n;
+        a.lds_words = (int32_t)(tiled_lds_bytes(s->D, s->B, s->tkind, s->trw, s->lut_lds) / 4);
         a.w_max = s->sc[4]; a.w_min = s->sc[5];
     }
     a.bar = s->bar; a.bar_err = s->bar_err; a.spin_limit = s->spin_limit;

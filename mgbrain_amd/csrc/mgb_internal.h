@@ -244,7 +244,7 @@ struct TiledArgs {
     const float* ltp;           // ltp[k] = A_LTP * expf(-k / TAU_LTP)
     const float* ltd;           // ltd[k] = A_LTD * expf(-k / TAU_LTD); ltd == ltp + lut_n
     int32_t lut_n;
-    int32_t lut_lds;            // leading entries of each table copied to LDS (>= 1)
+    int32_t lds_words;          // the launch's dynamic LDS, in words
     float w_max, w_min;
     // Fused STDP read-back: the launch applies the pending window's updates to w_t
     // (a copy) and lists every neuron with deferred dendrite updates for the
@@ -290,6 +290,10 @@ constexpr int kTiledItems = 16384;  // work items staged in LDS per propagation 
 constexpr int kTiledStaticLds = 1024; // bytes reserved for the fused kernel's static LDS
 constexpr uint32_t kClassTableMin = 32; // shortest k-fold class sum table
 constexpr int kClassCache = 128;    // k-fold class sums cached in LDS per class and side
+// Most leading entries of an STDP table copied to LDS in every window (4e7 synapses at
+// 26 Hz: 33.2 us with 1024, 33.4 with 2048, 33.6 with 4096, 34.0 with 8192; slower networks
+// have longer intervals)
+constexpr int kLutLdsMax = 2048;
 constexpr int kStdpHist = 16;       // spike steps kept per neuron for deferred dendrite updates
 // A history entry past the neuron's spikes (memset byte 0x80): below every step and
 // every lower bound of a history scan (>= -1).

@@ -796,7 +796,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     // All of the LDS is the launch's (no static LDS), the ring slice first: at address 0, so
     // that a synapse's byte offset in the slice is its LDS address (propagation below).
     extern __shared__ __align__(16) uint32_t lds[];
-    const int32_t D = a.D, B = a.B, bd = (int32_t)blockDim.x;
+    const int32_t D = a.D, bd = (int32_t)blockDim.x;
     const int32_t tid0 = (int32_t)threadIdx.x;
     // the workgroup's tile.  Workgroups go round-robin to the kXcds XCDs
     // (blockIdx.x % kXcds), each with its own L2; neighbouring tiles share the
@@ -814,10 +814,16 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     constexpr bool kMix = WK == kTStdpB;                    // BF16 static weights beside plastic ones
     constexpr bool kPl = WK == kTStdp || kMix;              // STDP on w_t
     constexpr bool kAux = WK == kTFP8 || WK == kTBF16 || kPl;
+    const int32_t t0 = a.tile_lo[g];
+    const int32_t tn = a.tile_lo[g + 1] - t0;
     const int RW = kCls ? 1 : a.rw;                         // ring words per (slot, target)
-    uint32_t* ring = lds;                                   // [RW][D][B]
+    // (laid out by the tile's own width; the launch brings the widest tile's LDS, and what a
+    // narrower one leaves holds more of the STDP tables: with the widest tile's layout, 8
+    // entries beside Poisson tiles of 702, most updates read theirs from HBM, 4e7 synapses
+    // 36.6 us a window, now 33.4)
+    uint32_t* ring = lds;                                   // [RW][D][tn]
     // (STDP: rounded up to 16 bytes, for the history rows' vector reads below)
-    uint32_t* stage = ring + (kPl ? (((size_t)RW * D * B + 3) & ~(size_t)3) : (size_t)RW * D * B);
+    uint32_t* stage = ring + (kPl ? (((size_t)RW * D * tn + 3) & ~(size_t)3) : (size_t)RW * D * tn);
     // [kTiledBatch] per staged spike: (its sub-row's first word - CH * its first work
     // item) mod 2^32, so that item q starts at word x + CH * q; byte offset of its row in
     // the slice (STDP: its ring slot << 26)
@@ -836,33 +842,37 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     uint32_t* sp_aux = reinterpret_cast<uint32_t*>(itm + kItems);
     // [kTiledBatch] kTStdpB: row scale bits | weights-to-load << 31
     uint32_t* sp_aux2 = sp_aux + kTiledBatch;
-    // STDP, per tile neuron: spike history [B][kStdpHist] (newest first, kHistNone past
+    // STDP, per tile neuron: spike history [tn][kStdpHist] (newest first, kHistNone past
     // the neuron's spikes; 64-byte rows), fire count, tf
     int32_t* hL = reinterpret_cast<int32_t*>(sp_aux + (kMix ? 2 : 1) * kTiledBatch);
-    int32_t* cL = hL + (size_t)B * kStdpHist;
-    int32_t* tfL = cL + B;
+    int32_t* cL = hL + (size_t)tn * kStdpHist;
+    int32_t* tfL = cL + tn;
     // the first lut_lds entries of the LTP and LTD tables
-    float* lutL = reinterpret_cast<float*>(tfL + B);
-    // STDP weight change for dt = t_pre - t_post (stdp_dw) from the LDS copy where it holds |dt|
-    // (lut_lds >= 1; entry 0 of both tables is 0, so dt = 0 gives 0), else from HBM.  The HBM
-    // read is a buffer load over both tables (ltd follows ltp), so that the compiler keeps an
-    // LDS load and a buffer load instead of one flat load through a selected pointer
+    float* lutL = reinterpret_cast<float*>(tfL + tn);
+    const int32_t lut_lds =
+        kPl ? min(min(a.lut_n, kLutLdsMax), (int32_t)((lds + a.lds_words - reinterpret_cast<uint32_t*>(lutL)) / 2)) : 0;
+    // STDP weight change of a pair k steps apart (stdp_dw) from the LDS copy where it holds
+    // k (lut_lds >= 1; entry 0 of both tables is 0, so k = 0 gives 0), else from HBM: ltp for
+    // a post spike k >= 0 steps after the pre spike, ltd for k >= 0 steps before it.  (Each
+    // use knows which: choosing by the sign of dt took a third of a deferred update's
+    // instructions.)  The HBM read is a buffer load over both tables (ltd follows ltp), so
+    // that the compiler keeps an LDS load and a buffer load instead of one flat load through
+    // a selected pointer
     const __amdgpu_buffer_rsrc_t lut_rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(kPl ? a.ltp : nullptr), (short)0, kPl ? 8 * a.lut_n : 0, kBufferDword3);
-    auto dw = [&](int32_t dt) -> float {
-        const int32_t k = dt < 0 ? -dt : dt;
-        float v = lutL[(dt < 0 ? 0 : a.lut_lds) + min(k, a.lut_lds - 1)];
-        if (k >= a.lut_lds)
+    auto lut = [&](uint32_t k, int32_t lds0, int32_t hbm0) -> float {
+        float v = lutL[lds0 + (int32_t)min(k, (uint32_t)lut_lds - 1u)];
+        if (k >= (uint32_t)lut_lds)
             v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                lut_rs, 4 * ((dt < 0 ? 0 : a.lut_n) + min(k, a.lut_n - 1)), 0, 0));
+                lut_rs, 4 * (hbm0 + (int32_t)min(k, (uint32_t)a.lut_n - 1u)), 0, 0));
         return v;
     };
+    auto ltp = [&](int32_t k) { return lut((uint32_t)k, 0, 0); };
+    auto ltd = [&](int32_t k) { return lut((uint32_t)k, lut_lds, a.lut_n); };
     const bool full = !kPl || a.apply_only == 0;
     Ctl* ctl = a.ctl;
     // fixed-point (scale, 1 / scale) of the tile's segment (scale_e == scale_i)
     const float2 fsc = a.seg_scale ? a.seg_scale[a.tile_seg[g]] : make_float2(a.scale_e, a.inv_e);
-    const int32_t t0 = a.tile_lo[g];
-    const int32_t tn = a.tile_lo[g + 1] - t0;
     // kTStdpB: a tile without plastic in-synapses never loads w_t
     const uint32_t plmask = (kMix && a.tile_pl[g]) ? 0xFFFFFFFFu : 0x7FFFFFFFu;
     // the tile's segment (one segment: all of it known without loads)
@@ -1021,11 +1031,15 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 cL[j] = a.cnt[t0 + j];
                 tfL[j] = a.tf[t0 + j];
             }
-            const int32_t* hg = a.hist + (size_t)t0 * kStdpHist;
-            for (int32_t k = tid; k < tn * kStdpHist; k += bd) hL[k] = hg[k];
-            for (int32_t k = tid; k < a.lut_lds; k += bd) {
-                lutL[k] = a.ltp[k];
-                lutL[a.lut_lds + k] = a.ltd[k];
+            const int4* hg = reinterpret_cast<const int4*>(a.hist + (size_t)t0 * kStdpHist);
+            for (int32_t k = tid; k < tn * (kStdpHist / 4); k += bd) reinterpret_cast<int4*>(hL)[k] = hg[k];
+            for (int32_t k = tid; k < lut_lds; k += 2 * bd) {
+                const int32_t k1 = min(k + bd, lut_lds - 1);
+                const float p0 = a.ltp[k], d0 = a.ltd[k], p1 = a.ltp[k1], d1 = a.ltd[k1];
+                lutL[k] = p0;
+                lutL[lut_lds + k] = d0;
+                lutL[k1] = p1;
+                lutL[lut_lds + k1] = d1;
             }
         }
         if (kCls && kw == 0) {
@@ -1287,7 +1301,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                         for (int h = 0; h < U; ++h)
     #pragma unroll
                             for (int u = 0; u < CH; ++u)
-                                ax[h][u] = rng[h][u] >= 0 ? dw(adt[h][u]) : 0.0f;
+                                ax[h][u] = rng[h][u] >= 0 ? ltd(adt[h][u]) : 0.0f;
                     }
     #pragma unroll
                     for (int h = 0; h < U; ++h)
@@ -1341,14 +1355,15 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                                     const int32_t mlo = rng[h][u] & 0xFF, mhi = rng[h][u] >> 8;
                                     for (int32_t m = mhi; m >= mlo; --m) {
                                         const int32_t e = hj[m];
-                                        w = clipw(w + dw(la[h] - e), a.w_max, a.w_min);
+                                        w = clipw(w + ltp(e - la[h]), a.w_max, a.w_min);   // e >= la
                                     }
                                 }
                                 const bool exc = w > 0.f;
                                 const int32_t v = (int32_t)rintf(w * fsc.x);
                                 // (one ring: both signs into one fixed-point sum)
-                                const int32_t at = valid ? ((exc || RW == 1 ? 0 : D) + slot) * tn + loc : (tid % tn);
-                                if (full) atomicAdd(reinterpret_cast<int32_t*>(ring) + at, valid ? v : 0);
+                                if (full && valid)
+                                    atomicAdd(reinterpret_cast<int32_t*>(ring) + ((exc || RW == 1 ? 0 : D) + slot) * tn + loc,
+                                              v);
                                 if (pl && valid)                           // axon update of t2
                                     a.w_t[kb[h] + (uint32_t)u] = clipw(w + ax[h][u], a.w_max, a.w_min);
                             }
@@ -1849,9 +1864,14 @@ hipError_t launch_tile_ccache(const int32_t* tile_lo, int32_t G, const uint16_t*
     return hipGetLastError();
 }
 
+// Dynamic LDS of a launch of one window (STDP: with the room for its tables).
+static size_t window_lds_bytes(const TiledArgs& a) {
+    return stdp_kind(a.kind) ? 4 * (size_t)a.lds_words : tiled_lds_bytes(a.D, a.B, a.kind, a.rw);
+}
+
 hipError_t launch_tiled(const TiledArgs& a, int32_t off, int32_t wk, int32_t nsteps, int block,
                         hipStream_t st) {
-    const size_t lds = tiled_lds_bytes(a.D, a.B, a.kind, a.rw, stdp_kind(a.kind) ? a.lut_lds : 0);
+    const size_t lds = window_lds_bytes(a);
     return launch_fn(tiled_fn_of(a.kind, a.chunk, false), a, off, wk, nsteps, 1, block, lds, st);
 }
 
@@ -1878,7 +1898,7 @@ hipError_t launch_tiled_persistent(const TiledArgs& a, int32_t off, int32_t wk, 
 
 int tiled_blocks_per_cu(const TiledArgs& a, int block, bool persistent) {
     const size_t lds = persistent ? tiled_pw_lds_bytes(a)
-                                  : tiled_lds_bytes(a.D, a.B, a.kind, a.rw, stdp_kind(a.kind) ? a.lut_lds : 0);
+                                  : window_lds_bytes(a);
     const void* f = tiled_fn_of(a.kind, a.chunk, persistent, persistent && a.region != 0);
     if (!f) return 0;
     int nb = 0;
