@@ -824,22 +824,31 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     uint32_t* ring = lds;                                   // [RW][D][tn]
     // (STDP: rounded up to 16 bytes, for the history rows' vector reads below)
     uint32_t* stage = ring + (kPl ? (((size_t)RW * D * tn + 3) & ~(size_t)3) : (size_t)RW * D * tn);
-    // [kTiledBatch] per staged spike: (its sub-row's first word - CH * its first work
+    // A batch of propagation stages kES spikes per thread.  With two, windows of more than
+    // one batch wait at half as many barriers and first loads (110,000 balanced neurons 48.9
+    // -> 46.8 us a window, twelve networks 26.5 -> 25.4; not for the wide words, whose items
+    // of 4 words then fill the table: sixteen networks in BF16 76.3 -> 77.8).  The staging
+    // area (3 * kTiledBatch words, kTiledItems half-words) then holds fewer items a round.
+    constexpr uint32_t kES = kCls ? 2u : 1u, kRec = kES * (uint32_t)kTiledBatch;
+    constexpr uint32_t kItems = kCls ? 12288u : (uint32_t)kTiledItems;
+    // [kRec] per staged spike: (its sub-row's first word - CH * its first work
     // item) mod 2^32, so that item q starts at word x + CH * q; byte offset of its row in
     // the slice (STDP: its ring slot << 26)
     uint2* sp_rec = reinterpret_cast<uint2*>(ring + (((size_t)(stage - ring) + 1) & ~(size_t)1));
     // CLASS: the first kClassCache k-fold sums of the classes of the tile's
     // last and first neurons (one class per tile in population-ordered networks),
-    // [class][side][count], in what the records leave of their 3 * kTiledBatch words
-    float* ccache = reinterpret_cast<float*>(sp_rec + kTiledBatch);
-    TileShared* sh = reinterpret_cast<TileShared*>(ccache + 4 * kClassCache);
-    static_assert(sizeof(TileShared) % 8 == 0 &&
-                  2 * kTiledBatch + 4 * kClassCache + sizeof(TileShared) / 4 + 1 <= 3 * kTiledBatch, "staging area");
-    constexpr uint32_t kItems = kTiledItems;   // work items staged per round
-    // [kItems] spike of the item | (its words - 1) << 10
-    uint16_t* itm = reinterpret_cast<uint16_t*>(stage + 3 * (size_t)kTiledBatch);
+    // [class][side][count]
+    float* ccache = reinterpret_cast<float*>(sp_rec + kRec);
+    TileShared* sh = reinterpret_cast<TileShared*>(ccache + (kCls ? 4 * kClassCache : 0));
+    static_assert(sizeof(TileShared) % 8 == 0, "alignment of what follows");
+    // [kItems] record of the item's spike | (its words - 1) << 11
+    uint16_t* itm = kCls ? reinterpret_cast<uint16_t*>(sh + 1) : reinterpret_cast<uint16_t*>(stage + 3 * kTiledBatch);
+    static_assert(kCls ? 8 + kRec * 8 + 16 * kClassCache + sizeof(TileShared) + 2 * kItems <=
+                             3 * kTiledBatch * 4 + 2 * kTiledItems
+                       : 8 + kRec * 8 + sizeof(TileShared) <= 3 * kTiledBatch * 4,
+                  "staging area");
     // [kTiledBatch] BF16/FP8: row scale bits; STDP: the source's last spike before the window
-    uint32_t* sp_aux = reinterpret_cast<uint32_t*>(itm + kItems);
+    uint32_t* sp_aux = stage + 3 * kTiledBatch + kTiledItems / 2;
     // [kTiledBatch] kTStdpB: row scale bits | weights-to-load << 31
     uint32_t* sp_aux2 = sp_aux + kTiledBatch;
     // STDP, per tile neuron: spike history [tn][kStdpHist] (newest first, kHistNone past
@@ -893,7 +902,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     // tiles' spike counts, then their exclusive prefix, and the tiles' list offsets
     // (tile h's part of a list starts at tile_lo[h] * window), [G] words each of LDS
     // after the staging area (the launch brings them)
-    uint32_t* rg_pre = reinterpret_cast<uint32_t*>(itm + kItems) + (kAux ? kTiledBatch : 0);
+    uint32_t* rg_pre = stage + 3 * kTiledBatch + kTiledItems / 2 + (kAux ? kTiledBatch : 0);
     uint32_t* rg_off = rg_pre + (PW ? a.G : 0);
     // (a variant of the persistent form of the 16-bit CLASS words only: in the other
     // kinds' persistent forms the code alone, never run, cost their windows 5 %)
@@ -1080,14 +1089,25 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         // index clamped into the segment's part of the list, which holds nq * window
         // entries), and their metadata loads before the ring copy, so that these
         // latencies overlap; entries past the count are never used
-        uint32_t pbeg = 0u, plm = 0u, paux = 0u, paux2 = 0u;
-        if ((uint32_t)tid < min((uint32_t)bd, E)) meta(ent0, pbeg, plm, paux, paux2);
+        uint32_t pbeg[kES] = {}, plm[kES] = {}, paux[kES] = {}, paux2[kES] = {};
+        if ((uint32_t)tid < min((uint32_t)bd, E)) meta(ent0, pbeg[0], plm[0], paux[0], paux2[0]);
         // windows of more than one batch (not with STDP, whose registers are spent): the
         // entries of batch b + 2 load during batch b and their metadata during batch b + 1,
         // so neither latency is waited for between batches (ent1: the next batch's entries)
         constexpr bool kAhead = !kPl;
-        uint32_t ent1 = 0u;
-        if (kAhead && E > (uint32_t)bd && (uint32_t)tid < E - (uint32_t)bd) ent1 = lent((uint32_t)bd + (uint32_t)tid);
+        const uint32_t batch = kES * (uint32_t)bd;
+        uint32_t ent1[kES] = {};
+        if constexpr (kAhead) {
+            // (thread t has entries t and bd + t of a batch)
+            if (E > (uint32_t)bd) {
+                uint32_t e1 = 0u;
+                if (kES == 2 && (uint32_t)(bd + tid) < E) e1 = lent((uint32_t)(bd + tid));
+#pragma unroll
+                for (uint32_t k = 0; k < kES; ++k)
+                    if (batch + k * (uint32_t)bd + (uint32_t)tid < E) ent1[k] = lent(batch + k * (uint32_t)bd + (uint32_t)tid);
+                if (kES == 2 && (uint32_t)(bd + tid) < E) meta(e1, pbeg[kES - 1], plm[kES - 1], paux[kES - 1], paux2[kES - 1]);
+            }
+        }
         if (full && kw == 0) {
             if (fed) ring_slice_in(ring, gring, D, tn, rprev, nprev, RW);
             else if (integ)                             // (nothing ever arrives: all zero)
@@ -1103,48 +1123,64 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         // 2. previous window's spikes into the tile
         const uint32_t R4 = 4u * (uint32_t)(D * tn);            // the slice's bytes (one of RW halves)
         int sb = 0;                                             // scan buffer
-        for (uint32_t b0 = 0; b0 < E; b0 += (uint32_t)bd) {
-            const uint32_t nb = min((uint32_t)bd, E - b0);
-            uint32_t items = 0u, beg = 0u, len = 0u, slot26 = 0u;
-            if ((uint32_t)tid < nb) {
-                uint32_t lm = plm, aux = paux, aux2 = paux2;
-                beg = pbeg;
-                if (!kAhead && b0 > 0) meta(lent(b0 + (uint32_t)tid), beg, lm, aux, aux2);
-                if (kAux) sp_aux[tid] = aux;
-                if (kMix) sp_aux2[tid] = aux2;
-                len = lm & kIdMask;
-                slot26 = lm & ~kIdMask;
-                items = (len + CH - 1) / CH;
+        for (uint32_t b0 = 0; b0 < E; b0 += batch) {
+            uint32_t items[kES], beg[kES], len[kES], slot26[kES], sum = 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < kES; ++k) {
+                const uint32_t j = k * (uint32_t)bd + (uint32_t)tid;
+                items[k] = beg[k] = len[k] = slot26[k] = 0u;
+                if (b0 + j < E) {
+                    if (!kAhead && b0 > 0) meta(lent(b0 + j), pbeg[k], plm[k], paux[k], paux2[k]);
+                    beg[k] = pbeg[k];
+                    if (kAux) sp_aux[j] = paux[k];
+                    if (kMix) sp_aux2[j] = paux2[k];
+                    len[k] = plm[k] & kIdMask;
+                    slot26[k] = plm[k] & ~kIdMask;
+                    items[k] = (len[k] + CH - 1) / CH;
+                }
+                sum += items[k];
             }
             if constexpr (kAhead) {
                 // the next batch's metadata from its entries (loaded a batch ago), and the
                 // entries of the batch after it
-                const uint32_t b1 = b0 + (uint32_t)bd, b2 = b1 + (uint32_t)bd;
-                if (b1 < E && (uint32_t)tid < E - b1) meta(ent1, pbeg, plm, paux, paux2);
-                if (b2 < E && (uint32_t)tid < E - b2) ent1 = lent(b2 + (uint32_t)tid);
+#pragma unroll
+                for (uint32_t k = 0; k < kES; ++k) {
+                    const uint32_t j1 = b0 + batch + k * (uint32_t)bd + (uint32_t)tid;
+                    if (j1 < E) meta(ent1[k], pbeg[k], plm[k], paux[k], paux2[k]);
+                    if (j1 + batch < E) ent1[k] = lent(j1 + batch);
+                }
             }
             sb ^= 1;
             uint32_t total;
-            const uint32_t incl = block_incl_scan(items, sh->wsum[sb], total);
+            uint32_t first[kES];                               // first item of each spike
+            first[0] = block_incl_scan(sum, sh->wsum[sb], total) - sum;
+            if (kES == 2) first[kES - 1] = first[0] + items[0];
             // (without items nothing waits between this and the spike list that takes the records' place)
-            if (total > 0u && (uint32_t)tid < nb)
-                sp_rec[tid] = make_uint2(beg - (incl - items) * (uint32_t)CH,
-                                         kPl ? slot26 : 4u * ((slot26 >> 26) + 1u) * (uint32_t)tn);
+            if (total > 0u)
+#pragma unroll
+                for (uint32_t k = 0; k < kES; ++k)
+                    sp_rec[k * (uint32_t)bd + (uint32_t)tid] =
+                        make_uint2(beg[k] - first[k] * (uint32_t)CH,
+                                   kPl ? slot26[k] : 4u * ((slot26[k] >> 26) + 1u) * (uint32_t)tn);
             for (uint32_t r0 = 0; r0 < total; r0 += kItems) {
                 const uint32_t rn = min(kItems, total - r0);
                 // item table: each spike writes its own work items of this round
-                if ((uint32_t)tid < nb) {
-                    const uint32_t q0 = max(incl - items, r0), q1 = min(incl, r0 + rn);
+#pragma unroll
+                for (uint32_t k = 0; k < kES; ++k) {
+                    const uint32_t end = first[k] + items[k];
+                    const uint32_t q0 = max(first[k], r0), q1 = min(end, r0 + rn);
                     for (uint32_t q = q0; q < q1; ++q) {
-                        const uint32_t n = q + 1u == incl ? len - (items - 1u) * (uint32_t)CH : (uint32_t)CH;
-                        itm[q - r0] = (uint16_t)((uint32_t)tid | ((n - 1u) << 10));
+                        const uint32_t n = q + 1u == end ? len[k] - (items[k] - 1u) * (uint32_t)CH : (uint32_t)CH;
+                        itm[q - r0] = (uint16_t)((k * (uint32_t)bd + (uint32_t)tid) | ((n - 1u) << 11));
                     }
                 }
                 __syncthreads();
                 // U items per thread in flight: U * CH synapse words loaded before the
                 // first LDS atomic
-                // (STDP: at most 8 synapses, whose STDP state then fits in the registers)
-                constexpr int U = CH >= 16 ? 1 : (kPl ? (CH >= 8 ? 1 : (CH == 1 ? 4 : 8 / CH)) : 16 / CH);
+                // (STDP: at most 8 synapses, whose STDP state then fits in the registers; FP32
+                // words: 8 and their weights, 11,000 neurons at one step a window 6.92 us with
+                // 16, 6.69 with 8)
+                constexpr int U = CH >= 16 ? 1 : (kPl || WK == kTF32 ? (CH >= 8 ? 1 : (CH == 1 ? 4 : 8 / CH)) : 16 / CH);
                 for (uint32_t it = (uint32_t)tid; it < rn; it += (uint32_t)(U * bd)) {
                     // branch-free loads, so that all U * CH are in flight before the first
                     // wait: lanes past the round's items re-read the last item and elements
@@ -1158,11 +1194,11 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                         const uint32_t q0 = it + (uint32_t)(h * bd);
                         const uint32_t q = min(q0, rn - 1u);
                         const uint32_t im = itm[q];
-                        const uint32_t j = im & 1023u;
+                        const uint32_t j = im & 2047u;
                         const uint2 rc = sp_rec[j];
                         kb[h] = rc.x + (r0 + q) * (uint32_t)CH;
                         row[h] = rc.y;
-                        cnt[h] = (q0 < rn) ? (im >> 10) + 1u : 0u;
+                        cnt[h] = (q0 < rn) ? (im >> 11) + 1u : 0u;
                         // (scales are powers of 2: the product with the row scale is exact)
                         rs[h] = (WK == kTFP8 || WK == kTBF16) ? __uint_as_float(sp_aux[j]) * fsc.x : 1.0f;
                         lw[h] = true;
