@@ -612,11 +612,13 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
 // `epoch` and `count` (the window's spikes of the tile, when its list went to
 // the tile's region) in its flag, a pair of 64-bit words per tile kBarStride words apart
 // (a cache line each), even epochs in the first and odd ones in the second, and waits
-// until every workgroup's flag of this parity holds `epoch`, one flag per thread (a
-// workgroup can be one window ahead -- its tile may have little to do -- and have
-// published epoch + 1 before this one reads its flag: with one word for both, its count
-// would be the next window's; two ahead it cannot be); with `cnt`, the counts of tiles [ct0, ct1) land in
-// cnt[h] (0 for the others).  A poll is one load, back to back with the next (each a
+// until the flag of this parity of every workgroup of its segment (tiles [ct0, ct1))
+// holds `epoch`, one flag per thread.  Workgroups of other segments share no list with it
+// and may be any number of windows ahead or behind.  One of its own segment can be one
+// window ahead -- its tile may have little to do -- and have published epoch + 1 before
+// this one reads its flag (two ahead it cannot be): with one word for both parities, its
+// count would be the next window's.  With `cnt`, the segment's counts land in cnt[h] (0 for
+// other tiles).  A poll is one load, back to back with the next (each a
 // round trip past the L2, the pace of the loop); the error word and the clock, a round
 // trip of their own, are read every 16th poll only.  The wait is bounded: past `limit`
 // clock ticks (counted from the first look at the clock), or
@@ -631,7 +633,10 @@ __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g,
     constexpr size_t kStride64 = kBarStride / 2;
     if (threadIdx.x == 0) st_agent64(&flag[(size_t)g * kStride64], ((uint64_t)count << 32) | epoch);
     int bad = 0;
-    for (uint32_t h = threadIdx.x; h < G && !bad; h += blockDim.x) {
+    if (cnt)
+        for (uint32_t h = threadIdx.x; h < G; h += blockDim.x)
+            if (h < ct0 || h >= ct1) cnt[h] = 0u;
+    for (uint32_t h = ct0 + threadIdx.x; h < ct1 && !bad; h += blockDim.x) {
         uint64_t v = ld_agent64(&flag[(size_t)h * kStride64]);
         uint64_t c0 = 0;
         for (uint32_t polls = 0; (int32_t)((uint32_t)v - epoch) < 0; ++polls) {
@@ -647,7 +652,7 @@ __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g,
             }
             v = ld_agent64(&flag[(size_t)h * kStride64]);
         }
-        if (cnt) cnt[h] = (h >= ct0 && h < ct1) ? (uint32_t)(v >> 32) : 0u;
+        if (cnt) cnt[h] = (uint32_t)(v >> 32);
     }
     if (bad) *lds_bad = 1u;
     __syncthreads();
