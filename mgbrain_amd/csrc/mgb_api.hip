@@ -96,6 +96,7 @@ struct mgb_sim {
     int32_t nseg = 1;
     std::vector<int32_t> h_seg_lo;     // [nseg+1] segment boundaries (independent networks)
     std::vector<int32_t> h_seg_tile0;  // [nseg+1] first tile of each segment
+    std::vector<int32_t> h_tile_lo;    // [G+1]
     std::vector<uint64_t> h_seg_obase; // [nseg+1] first offset entry of each segment
     int32_t* tile_lo = nullptr;        // [G+1]
     uint32_t* tile_of = nullptr;       // [n] tile of each neuron
@@ -144,7 +145,9 @@ struct mgb_sim {
     uint8_t* rd_ws = nullptr;
     size_t rd_ws_bytes = 0;
     int xcd_map = -1;                  // fused launches: XCD-contiguous tile order (-1: not computed yet)
-    int region = 0;                    // persistent launches: per-tile list regions (TiledArgs::region)
+    double poisson_window = 0.0;       // most spikes expected of a tile's Poisson neurons in a window
+    int flag_cap = 0;                  // (TiledArgs::flag_cap)
+    int region = 0;                    // persistent launches: spikes with the flags (TiledArgs::region)
     uint64_t tile_hash = 0;            // FNV-1a of the tile boundaries (the ring slices' layout)
     // host mirrors for read-back
     std::vector<float> class_w;        // [n_tbl][2]
@@ -488,6 +491,7 @@ mgb_status choose_tiles(mgb_sim* s, const mgb_opts* o, int32_t n, int32_t D, con
     kbase[nseg] = (uint32_t)kb;
     obase[nseg] = ob;
     s->h_seg_tile0 = tile0;
+    s->h_tile_lo = tlo;
     s->h_seg_obase = obase;
     s->G = (int32_t)tseg.size();
     s->nseg = nseg;
@@ -1189,7 +1193,13 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
     s->prop_block = (o && o->prop_block >= 64 && o->prop_block <= 1024) ? (o->prop_block / 64) * 64 : 256;
     s->prop_grid = (o && o->prop_grid > 0) ? o->prop_grid : 0;
     if (s->tiled && !stdp_kind(s->tkind)) {
-        // persistent launches: wait flags (reset before each launch) and the wait's bound
+        for (size_t t = 0; t + 1 < s->h_tile_lo.size(); ++t) {
+            double e = 0.0;
+            for (int32_t i = s->h_tile_lo[t]; i < s->h_tile_lo[t + 1]; ++i)
+                if (h.type[i] == MGB_POISSON) e += (double)h.rate[i] * s->window;
+            s->poisson_window = std::max(s->poisson_window, e);
+        }
+        // persistent launches: wait flags (zeroed here and by a restored checkpoint) and the wait's bound
         MGB_TRY(dalloc_n(s, &s->bar, (size_t)s->G * kBarStride));
         MGB_TRY(dalloc_n(s, &s->bar_err, 1));
         MGB_HIP_TRY(hipMemsetAsync(s->bar, 0, 4 * (size_t)s->G * kBarStride, st));
@@ -1280,18 +1290,30 @@ void update_persist(mgb_sim* s) {
     TiledArgs a = tiled_args(s);
     s->xcd_map = a.xcd_map;
     if (stdp_kind(s->tkind) || s->persist_req == MGB_PERSIST_OFF || !s->bar) return;
-    // per-tile list regions (the kernel's variant with them) when asked for, or by
-    // default in networks large enough for windows of many spikes (in small ones the
-    // variant without them was the faster), when one
-    // thread per tile can scan their counts and the counts fit in LDS beside the tile's
-    // data with every workgroup still resident
+    // Spikes that pass with the wait's flags (grid_exchange) wherever a tile's mostly fit
+    // there: without Poisson tiles whose rates alone say that they do not (80,000
+    // conductance neurons 8.71 -> 8.40 us a window, 20,000 in BF16 8.16 -> 7.50, 5,000 7.3 -> 6.8;
+    // with busy Poisson tiles, 5,000 and 11,000 neurons 8.0 -> 8.7 and 9.0 -> 9.9, by lists).  16-bit
+    // CLASS words also when asked for, and in networks of windows of many spikes, where
+    // regions beat lists by themselves.  One thread per tile scans the regions' counts, and the
+    // LDS holds them beside the tile's data with every workgroup still resident
     const bool want = s->persist_req == MGB_PERSIST_REGIONS ||
                       (s->persist_req == MGB_PERSIST_AUTO && s->n >= kRegionMinNeurons);
-    if (want && s->tkind == kTClass16 && s->G <= kRegionMaxG && s->G <= s->tblock) {
-        a.region = 1;
-        if (set_tiled_pw_lds_limit(a) == hipSuccess && resident(s, a, true)) {
+    a.flag_cap = (int32_t)std::min<int64_t>(kInl, 2 * tiled_batch(s->tkind, s->tblock) / s->G);
+    const bool fits = 2 * s->G <= tiled_free_words(s->tkind);
+    const bool asked = want && s->tkind == kTClass16;
+    // (by itself only without LDS or registers beyond the list form's: several simulators'
+    // launches share the CUs, and a launch that is partly resident waits for the others)
+    const int lists_per_cu = tiled_blocks_per_cu(a, s->tblock, true);
+    if ((asked || (s->persist_req != MGB_PERSIST_LISTS && fits && a.flag_cap >= kInlMin &&
+                   s->poisson_window <= 0.5 * a.flag_cap)) &&
+        s->G <= kRegionMaxG && s->G <= s->tblock) {
+        a.region = fits ? 1 : 2;
+        if (set_tiled_pw_lds_limit(a) == hipSuccess && resident(s, a, true) &&
+            (asked || tiled_blocks_per_cu(a, s->tblock, true) >= lists_per_cu)) {
             s->region = a.region;
-            s->persist = 2;
+            s->flag_cap = a.flag_cap;
+            s->persist = asked ? 2 : 1;
             return;
         }
         (void)hipGetLastError();
@@ -1334,6 +1356,7 @@ TiledArgs tiled_args(const mgb_sim* s) {
     }
     a.bar = s->bar; a.bar_err = s->bar_err; a.spin_limit = s->spin_limit;
     a.region = s->region;
+    a.flag_cap = s->flag_cap;
     a.xcd_map = s->xcd_map >= 0 ? s->xcd_map : (resident(s, a, false) ? 1 : 0);
     return a;
 }

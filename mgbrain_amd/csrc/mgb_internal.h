@@ -146,7 +146,7 @@ struct StdpArgs {
 };
 
 // Fused tiled window kernel: workgroup g owns targets [tile_lo[g], tile_lo[g+1])
-// (at most B) and keeps their ring slice ring_t[g][D][B] in LDS while it (1)
+// (tn of them, at most B) and keeps their ring slice ring_t[g][D][tn] in LDS while it (1)
 // adds the previous window's spikes arriving in the tile (tile-sorted CSR copy
 // syn_t, per-row tile offsets) and (2) advances the tile's neurons.
 //
@@ -260,14 +260,16 @@ struct TiledArgs {
     // 1: workgroup b runs tile (b % kXcds) * (G / kXcds) + ... (a contiguous run of
     // tiles per XCD), set when every workgroup of the launch is resident at once
     int32_t xcd_map;
-    // persistent launches of 16-bit CLASS words with G <= kRegionMaxG and G <= the block
-    // size (and the counts fitting in LDS), launched as the kernel's list-region variant:
-    // windows followed by another window of the same launch write their spikes into the
-    // tile's own part of the list (tile_lo * window on) and publish the count with the
-    // wait's flag, instead of reserving list space with a returning global atomic
+    // persistent launches with G <= kRegionMaxG and G <= the block size, launched as the
+    // kernel's variant whose windows followed by another of the same launch pass their
+    // spikes with the wait's flags (grid_exchange), those past flag_cap of a tile in the
+    // tile's own part of the list (tile_lo * window on).  1: two words per tile fit in the
+    // staging area (tiled_free_words), 2: they have LDS of their own
     int32_t region;
-    // persistent launches: one flag per tile (kBarStride words apart; two 64-bit words, for
-    // even and odd epochs: window epoch | spike count << 32) for the wait between windows, its error word,
+    int32_t flag_cap;           // (region) spikes of a tile that pass with its flag: at most kInl, and
+                                // for all tiles at most two batches
+    // persistent launches: one flag per tile (kBarStride words apart, half a line for
+    // even and half for odd epochs) for the wait between windows, its error word,
     // and the wait's bound in wall-clock ticks
     uint32_t* bar;
     uint32_t* bar_err;
@@ -287,7 +289,9 @@ hipError_t launch_stdp(const StdpArgs& a, int32_t off, int32_t wk, int grid, hip
 hipError_t launch_finalize(Ctl* ctl, int32_t steps, int32_t windows, HostMirror* m, hipStream_t st);
 constexpr int kTiledBatch = 1024;   // spikes staged in LDS per propagation batch
 constexpr int kTiledItems = 16384;  // work items staged in LDS per propagation round
-constexpr int kTiledStaticLds = 1024; // bytes reserved for the fused kernel's static LDS
+// Bytes of a workgroup's LDS left out when the widest tile is chosen (the kernel has no
+// static LDS; tile boundaries belong to a checkpoint's layout, so the bound stays)
+constexpr int kTiledStaticLds = 1024;
 constexpr uint32_t kClassTableMin = 32; // shortest k-fold class sum table
 constexpr int kClassCache = 128;    // k-fold class sums cached in LDS per class and side
 // Most leading entries of an STDP table copied to LDS in every window (4e7 synapses at
@@ -304,8 +308,10 @@ constexpr int32_t kHistNone = (int32_t)0x80808080;
 constexpr int kSubAlign = 8;
 constexpr int kXcds = 8;            // MI355X: accelerator complex dies, one L2 each
 constexpr int kBarStride = 32;      // words between the flags of a persistent launch's grid wait
+constexpr int kInl = 14;            // persistent launches: most spikes of a tile that pass with its flag
+constexpr int kInlMin = 6;          // fewer are not worth it: 80,000 neurons have 2.5 a tile and window
 constexpr int kRegionMaxG = 512;    // persistent launches: most tiles whose lists go to per-tile regions
-constexpr int kRegionMinNeurons = 32768; // MGB_PERSIST_AUTO: list regions from this many neurons on
+constexpr int kRegionMinNeurons = 32768; // MGB_PERSIST_AUTO, 16-bit CLASS words: regions from this many neurons on, however busy
 // Word 3 of a raw buffer resource on gfx9 (CDNA): data format 32, no swizzle; loads past
 // the resource's byte count return 0.
 constexpr int kBufferDword3 = 0x00020000;
@@ -319,6 +325,9 @@ hipError_t launch_tile_ccache(const int32_t* tile_lo, int32_t G, const uint16_t*
 int tiled_blocks_per_cu(const TiledArgs& a, int block, bool persistent = false);
 hipError_t launch_tiled(const TiledArgs& a, int32_t off, int32_t wk, int32_t nsteps, int block,
                         hipStream_t st);
+// Spikes of a propagation batch of the kinds without STDP.
+inline int64_t tiled_batch(int kind, int block) { return (kind == kTClass16 ? 2 : 1) * (int64_t)block; }
+int32_t tiled_free_words(int kind);
 // Dynamic LDS of the persistent form for `a` (with a.region, the list regions' counts),
 // and the persistent function's limit raised to it.
 size_t tiled_pw_lds_bytes(const TiledArgs& a);

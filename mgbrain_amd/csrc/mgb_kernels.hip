@@ -5,8 +5,8 @@
 // updates of a window depend only on spikes of earlier windows:
 //   k_neurons   advances every neuron through the w steps with its state in
 //               registers (one HBM read/write of the state per window), reads
-//               and clears one ring row per step, and appends spikes to the
-//               window's list with one wave-ballot + one atomic per wave-step;
+//               the window's ring rows together and clears them, and appends a
+//               wave's spikes of the window to the list with one atomic;
 //   k_prop      walks the CSR rows of the window's spikes and adds each
 //               synapse into the ring row of its arrival step with an integer
 //               atomic (order-independent, so results are bit-reproducible);
@@ -606,36 +606,30 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Grid-wide wait between two windows of a persistent launch.  Each thread first
+// Grid-wide wait between two windows of a persistent launch (list form).  Each thread first
 // waits for its own stores to complete (s_waitcnt vmcnt(0): the agent-scope
 // stores above are then visible at agent scope), then the workgroup publishes
-// `epoch` and `count` (the window's spikes of the tile, when its list went to
-// the tile's region) in its flag, a pair of 64-bit words per tile kBarStride words apart
-// (a cache line each), even epochs in the first and odd ones in the second, and waits
-// until the flag of this parity of every workgroup of its segment (tiles [ct0, ct1))
-// holds `epoch`, one flag per thread.  Workgroups of other segments share no list with it
-// and may be any number of windows ahead or behind.  One of its own segment can be one
-// window ahead -- its tile may have little to do -- and have published epoch + 1 before
-// this one reads its flag (two ahead it cannot be): with one word for both parities, its
-// count would be the next window's.  With `cnt`, the segment's counts land in cnt[h] (0 for
-// other tiles).  A poll is one load, back to back with the next (each a
-// round trip past the L2, the pace of the loop); the error word and the clock, a round
+// `epoch` in its flag, words kBarStride apart per tile (a cache line each), even epochs in
+// one and odd ones in another, and waits until the flag of this parity of every
+// workgroup of its segment (tiles [ct0, ct1)) holds `epoch`, one flag per thread.
+// Workgroups of other segments share no list with it and may be any number of windows
+// ahead or behind.  One of its own segment can be one window ahead -- its tile may have
+// little to do -- and have published epoch + 1 before this one reads its flag (two ahead
+// it cannot be): with one word for both parities, what else the flag holds
+// (grid_exchange) would be the next window's.  A poll is one load, back to back with the
+// next (each a round trip past the L2, the pace of the loop); the error word and the clock, a round
 // trip of their own, are read every 16th poll only.  The wait is bounded: past `limit`
 // clock ticks (counted from the first look at the clock), or
 // once another workgroup has reported a timeout, it sets *err and returns false,
 // so every workgroup leaves the kernel (the host turns *err into an error).
-__device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g, uint32_t epoch, uint32_t count,
-                                          uint32_t* cnt, uint32_t ct0, uint32_t ct1, uint32_t* err, uint64_t limit,
-                                          uint32_t* lds_bad) {
+__device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t g, uint32_t epoch, uint32_t ct0, uint32_t ct1,
+                                          uint32_t* err, uint64_t limit, uint32_t* lds_bad) {
     __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0)
     __syncthreads();
-    uint64_t* flag = reinterpret_cast<uint64_t*>(bar) + (epoch & 1u);
+    uint64_t* flag = reinterpret_cast<uint64_t*>(bar) + 8u * (epoch & 1u);
     constexpr size_t kStride64 = kBarStride / 2;
-    if (threadIdx.x == 0) st_agent64(&flag[(size_t)g * kStride64], ((uint64_t)count << 32) | epoch);
+    if (threadIdx.x == 0) st_agent64(&flag[(size_t)g * kStride64], epoch);
     int bad = 0;
-    if (cnt)
-        for (uint32_t h = threadIdx.x; h < G; h += blockDim.x)
-            if (h < ct0 || h >= ct1) cnt[h] = 0u;
     for (uint32_t h = ct0 + threadIdx.x; h < ct1 && !bad; h += blockDim.x) {
         uint64_t v = ld_agent64(&flag[(size_t)h * kStride64]);
         uint64_t c0 = 0;
@@ -652,7 +646,6 @@ __device__ __forceinline__ bool grid_wait(uint32_t* bar, uint32_t G, uint32_t g,
             }
             v = ld_agent64(&flag[(size_t)h * kStride64]);
         }
-        if (cnt) cnt[h] = (uint32_t)(v >> 32);
     }
     if (bad) *lds_bad = 1u;
     __syncthreads();
@@ -666,7 +659,112 @@ struct TileShared {
     uint32_t n, list_at;             // its spikes; their place in the segment's list
     uint32_t ccls[2];                // CLASS: the cached classes
     uint32_t bad, pad;               // a wait timed out
+    uint32_t n_in, n_far;            // grid_exchange: spikes that came with the flags; 1: others did not
 };
+
+// grid_wait of the windows that pass their spikes with the flags.  A tile's flag is then 8
+// 64-bit words per parity (one store of one wave, 64 bytes), the low half of each the
+// epoch: the first word's high half is the window's spike count, the other seven hold
+// two spikes each, 16 bits: tile-local neuron | step << 11 (tiles of at most 2048,
+// windows of at most 32 steps).  Every word carries the epoch, so a reader needs no
+// order between them, and a tile's first `cap` (kInl at most) spikes pass with the wait itself: through
+// lists they took a returning atomic for list space, a wait for the entries' stores and
+// the loads of the list's count and entries, each a round trip past the L2 (80,000
+// conductance neurons, 256 tiles: 8.71 -> 8.40 us a window; 20,000 in BF16, 79 tiles: 8.16
+// -> 7.50; 2,000, 10 tiles: 7.1 -> 6.7).  Spikes past those are in the tile's region,
+// complete before the flag; they take back what the others gain (update_persist, mgb_api.hip).
+// Not kept: three spikes to a word and up to 64 words (92 instructions more between the
+// poll and propagation: 9.2 us for the 80,000), one spike to a word used where it is read
+// (no compaction, but more, emptier batches: 12.0).
+// A thread reads up to 4 words at once, the 8 words of a tile being read in one wave.  On
+// return inl[0, sh->n_in) holds the entries (neuron id | step << 26) of tiles
+// [ct0, ct1) in any order, sh->n_far is 1 if any are left in regions, far[h] each tile's number of those.
+// The caller has published, and cleared n_in and n_far before.  Bounds and errors as
+// grid_wait.
+__device__ __forceinline__ bool grid_exchange(const uint32_t* bar, uint32_t epoch, uint32_t cap, uint32_t ct0, uint32_t ct1,
+                                              const uint32_t* lo, uint32_t* far, uint32_t* inl, uint32_t* err,
+                                              uint64_t limit, TileShared* sh) {
+    const uint64_t* flag = reinterpret_cast<const uint64_t*>(bar) + 8u * (epoch & 1u);
+    const uint32_t nwords = 8u * (ct1 - ct0), bd = blockDim.x, tid = threadIdx.x;
+    const uint32_t wd = tid & 7u;                      // (bd is a multiple of 64)
+    bool bad = false;
+    for (uint32_t i0 = 0; i0 < nwords && !bad; i0 += 4u * bd) {
+        uint64_t v[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t i = i0 + k * bd + tid;
+            v[k] = (uint64_t)epoch;                    // (no word: count 0)
+            if (i < nwords) v[k] = ld_agent64(&flag[(size_t)(ct0 + (i >> 3)) * (kBarStride / 2) + wd]);
+        }
+        uint64_t c0 = 0;
+        for (uint32_t polls = 0;; ++polls) {
+            bool pend = false;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) pend |= (int32_t)((uint32_t)v[k] - epoch) < 0;
+            if (!__any(pend)) break;
+            if ((polls & 15u) == 15u) {
+                const uint64_t c = (uint64_t)wall_clock64();
+                if (polls == 15u) c0 = c;
+                const bool late = c - c0 > limit;
+                if (late) st_agent(err, 1u);
+                if (__any(late || ld_agent(err) != 0u)) {
+                    bad = true;
+                    break;
+                }
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                const uint32_t i = i0 + k * bd + tid;
+                if ((int32_t)((uint32_t)v[k] - epoch) < 0)
+                    v[k] = ld_agent64(&flag[(size_t)(ct0 + (i >> 3)) * (kBarStride / 2) + wd]);
+            }
+        }
+        if (bad) break;
+        bool any = false;                              // (a silent window ends here)
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t i = i0 + k * bd + tid;
+            const bool head = wd == 0u && i < nwords;
+            if (head) far[ct0 + (i >> 3)] = (uint32_t)max((int32_t)(uint32_t)(v[k] >> 32) - (int32_t)cap, 0);
+            any |= head && (v[k] >> 32) != 0ull;
+        }
+        if (!__any(any)) continue;
+        uint64_t m[4][2];
+        uint32_t total = 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            m[k][0] = m[k][1] = 0ull;
+            if (i0 + k * bd >= nwords) continue;
+            const uint32_t p = (uint32_t)(v[k] >> 32);
+            const uint32_t all = (uint32_t)__shfl((int)p, (int)(lane_id() & ~7u)), cnt = min(all, cap);
+            m[k][0] = __ballot(wd != 0u && cnt > 2u * (wd - 1u));
+            m[k][1] = __ballot(wd != 0u && cnt > 2u * (wd - 1u) + 1u);
+            total += (uint32_t)(__popcll(m[k][0]) + __popcll(m[k][1]));
+            if (all > cap) sh->n_far = 1u;
+        }
+        if (total == 0u) continue;
+        uint32_t r = 0u;
+        if (lane_id() == 0u) r = atomicAdd(&sh->n_in, total);
+        r = (uint32_t)__builtin_amdgcn_readfirstlane((int)r);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            if (m[k][0] == 0ull) continue;
+            const uint32_t h = ct0 + ((i0 + k * bd + tid) >> 3);
+            const uint32_t p = (uint32_t)(v[k] >> 32);
+            const uint64_t me = 1ull << lane_id();
+            const uint32_t at = r + rank_below(m[k][0]) + rank_below(m[k][1]);
+            if (m[k][0] & me) {
+                const uint32_t l0 = lo[h];
+                inl[at] = (l0 + (p & 0x7FFu)) | (((p >> 11) & 31u) << 26);
+                if (m[k][1] & me) inl[at + 1u] = (l0 + ((p >> 16) & 0x7FFu)) | ((p >> 27) << 26);
+            }
+            r += (uint32_t)(__popcll(m[k][0]) + __popcll(m[k][1]));
+        }
+    }
+    if (bad) sh->bad = 1u;
+    __syncthreads();
+    return sh->bad == 0u;
+}
 
 // Registers of one neuron of a tile across the windows of a launch: the state, the
 // constants of its type's update that every step needs, and what its spikes add up to.
@@ -737,15 +835,15 @@ __device__ __forceinline__ uint32_t tneu_steps(TNeu& st, const float (&be)[NB], 
     return m;
 }
 
-// One window of the fused tiled step (CLASS format).  Workgroup g (targets
-// [tile_lo[g], tile_lo[g+1]) of segment tile_seg[g]):
-//   1. loads its ring slice ring_t[g] (D x B words) into LDS;
+// One window of the fused tiled step.  Workgroup g (targets [tile_lo[g], tile_lo[g+1])
+// of segment tile_seg[g], tn of them; a tile that no synapse targets does step 3 only):
+//   1. loads its ring slice (D x tn words) into LDS;
 //   2. adds the previous window's spikes of its segment: for each spiker, the sub-row of its
 //      tile-sorted CSR row that targets this tile, split into work items of
 //      `chunk` synapses balanced over the block, one LDS atomic per synapse;
 //   3. advances the tile's neurons through this window's steps reading and
-//      clearing their LDS ring rows, appending spikes (+ record, synaptic
-//      events) with one wave ballot per step;
+//      clearing their LDS ring rows a few steps at a time, appending spikes
+//      (+ record, synaptic events) with one wave ballot per step that has any;
 //   4. writes the ring slice back.
 // Spike lists rotate over three buffers: window k writes k%3, reads (k-1)%3
 // and clears the counter of (k+1)%3, which no workgroup touches in window k.
@@ -797,7 +895,7 @@ template <int CH, int WK, bool PW, bool RG = false>
 __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_t wk, int32_t nsteps,
                                                 int32_t nwin) {
     static_assert(!(PW && (WK == kTStdp || WK == kTStdpB)), "the persistent form has no STDP");
-    static_assert(!RG || (PW && WK == kTClass16), "list regions: persistent form of 16-bit CLASS words only");
+    static_assert(!RG || PW, "exchange with the flags: persistent form only");
     // All of the LDS is the launch's (no static LDS), the ring slice first: at address 0, so
     // that a synapse's byte offset in the slice is its LDS address (propagation below).
     extern __shared__ __align__(16) uint32_t lds[];
@@ -903,18 +1001,20 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
     const int64_t sbase = ctl->base_step + off;
     const int64_t wbase = ctl->base_window + wk;
     const int32_t nw = PW ? nwin : 1;
-    // persistent launches with per-tile list regions (a.region): between windows the
-    // tiles' spike counts, then their exclusive prefix, and the tiles' list offsets
-    // (tile h's part of a list starts at tile_lo[h] * window), [G] words each of LDS
-    // after the staging area (the launch brings them)
-    uint32_t* rg_pre = stage + 3 * kTiledBatch + kTiledItems / 2 + (kAux ? kTiledBatch : 0);
-    uint32_t* rg_off = rg_pre + (PW ? a.G : 0);
-    // (a variant of the persistent form of the 16-bit CLASS words only: in the other
-    // kinds' persistent forms the code alone, never run, cost their windows 5 %)
-    constexpr bool kRg = RG;
-    const bool rgn_on = kRg && a.region != 0;
+    // spikes with the flags (RG): between windows the counts of the tiles' spikes in their
+    // regions, then their exclusive prefix, and the tiles' first neurons (tile h's part of
+    // a list starts at tile_lo[h] * window), [G] words each
+    // (in the staging area's end where it has room for them)
+    uint32_t* rg_pre = a.region == 2 ? stage + 3 * kTiledBatch + kTiledItems / 2 + (kAux ? kTiledBatch : 0)
+                                     : stage + 3 * kTiledBatch + (kCls ? kTiledItems / 2 : 0) - 2 * a.G;
+    uint32_t* rg_lo = rg_pre + a.G;
+    // the spikes that came with the flags, in the item table: all read before its first use
+    // (flag_cap * G entries are two batches at most)
+    uint32_t* inl = reinterpret_cast<uint32_t*>(itm);
+    const uint32_t fcap = (uint32_t)a.flag_cap;
+    constexpr bool rgn_on = RG;
     if (rgn_on)
-        for (int32_t h = tid0; h < a.G; h += bd) rg_off[h] = (uint32_t)a.tile_lo[h] * (uint32_t)a.window;
+        for (int32_t h = tid0; h < a.G; h += bd) rg_lo[h] = (uint32_t)a.tile_lo[h];
     // every window's list but a launch's last goes to the regions; whether the previous
     // window's did (thread-uniform)
     bool rg_prev = false;
@@ -988,10 +1088,12 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 if (rg_pre[mid] <= e) lo = mid;
                 else hi = mid - 1u;
             }
-            return ld_agent(&a.win_buf[(size_t)bprev * a.win_stride + rg_off[lo] + (e - rg_pre[lo])]);
+            return ld_agent(&a.win_buf[(size_t)bprev * a.win_stride + (size_t)rg_lo[lo] * (size_t)a.window +
+                                       (fcap + e - rg_pre[lo])]);
         };
+        uint32_t n_in = 0u;
         auto lent = [&](uint32_t e) -> uint32_t {
-            if (rgc) return rentry(e);
+            if (rgc) return e < n_in ? inl[e] : rentry(e - n_in);
             return PW ? ld_agent(&L[e]) : L[e];
         };
         int64_t sprev;
@@ -1011,13 +1113,21 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             E = 0u;
             ent0 = 0u;
         } else if (rgc) {
-            // the counts came with the wait (rg_pre); the list is laid out by their prefix
+            // the spikes came with the wait; those past a tile's kInl follow in the regions,
+            // by the prefix of their counts
             sprev = s0 - nsteps;
-            const uint32_t c = (uint32_t)tid < (uint32_t)a.G ? rg_pre[tid] : 0u;
-            const uint32_t incl = block_incl_scan(c, sh->wsum[0], E);
-            if ((uint32_t)tid < (uint32_t)a.G) rg_pre[tid] = incl - c;
-            __syncthreads();
-            ent0 = (uint32_t)tid < E ? rentry((uint32_t)tid) : 0u;
+            n_in = sh->n_in;
+            E = n_in;
+            if (sh->n_far) {
+                uint32_t nf;
+                const uint32_t h = gt0 + (uint32_t)tid;
+                const uint32_t c = h < gt1 ? rg_pre[h] : 0u;
+                const uint32_t incl = block_incl_scan(c, sh->wsum[0], nf);
+                if (h < gt1) rg_pre[h] = incl - c;
+                __syncthreads();
+                E += nf;
+            }
+            ent0 = (uint32_t)tid < E ? lent((uint32_t)tid) : 0u;
         } else {
             sprev = s0 - nsteps;
             E = ld_agent(&tcnt[bprev * nseg]);
@@ -1124,6 +1234,10 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             if (tid < tn) load_neuron(t0 + tid, own_st, kPl ? lastB : nullptr);
         }
         __syncthreads();
+        if (RG && tid == 0) {                                   // (read above; next counted behind the steps' barrier)
+            sh->n_in = 0u;
+            sh->n_far = 0u;
+        }
 
         // 2. previous window's spikes into the tile
         const uint32_t R4 = 4u * (uint32_t)(D * tn);            // the slice's bytes (one of RW halves)
@@ -1469,11 +1583,11 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
                 const uint32_t cap = (uint32_t)kTiledBatch;
                 const uint32_t over0 = max(lb, cap);                 // first index past the LDS list
                 if (rgp) {
-                    // the tile's region holds every entry at its place in the tile's list
-                    // (written now, complete by the wait); the LDS list keeps the first cap
-                    // for the records, and records past them take their places here
+                    // the LDS list keeps the first cap entries (published below); past them
+                    // an entry goes to its place in the tile's region, and its record
+                    // takes one here
                     const uint32_t r = lb + rank_below(m);
-                    if (fired) st_agent(&rgw[r], (uint32_t)i | ((uint32_t)w << 26));
+                    if (fired && r >= cap) st_agent(&rgw[r], (uint32_t)i | ((uint32_t)w << 26));
                     if (a.rec && lb + pc > cap) {
                         unsigned long long rb = 0ull;
                         if (lane_id() == leader)
@@ -1637,6 +1751,26 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         if (se_local) atomicAdd(&sh->se, se_local);
         __syncthreads();
         const uint32_t nl = min(sh->n, (uint32_t)kTiledBatch);
+        if (RG && rgp) {
+            // publish the window's spikes: those past fcap in the region first
+            const uint32_t nt = sh->n;
+            if (nt > fcap) {
+                for (uint32_t k = fcap + (uint32_t)tid; k < nl; k += (uint32_t)bd) st_agent(&rgw[k], lsp[k]);
+                __builtin_amdgcn_s_waitcnt(0x0F70);             // vmcnt(0)
+                __syncthreads();
+            }
+            if (tid < 8) {
+                const uint32_t k0 = 2u * (uint32_t)max(tid - 1, 0);
+                const uint32_t x0 = lsp[k0], x1 = lsp[k0 + 1u];  // (past nl: never read)
+                const uint32_t p = ((x0 & kIdMask) - (uint32_t)t0) | (x0 >> 26) << 11;
+                const uint32_t p1 = ((x1 & kIdMask) - (uint32_t)t0) | (x1 >> 26) << 11;
+                const uint32_t hi = tid == 0 ? nt : ((p & 0xFFFFu) | (p1 << 16));
+                __builtin_amdgcn_s_waitcnt(0x0F70);             // (the cleared count of list bnext)
+                const uint32_t ep = (uint32_t)(kwin + 1);
+                st_agent64(reinterpret_cast<uint64_t*>(a.bar) + (size_t)g * (kBarStride / 2) + 8u * (ep & 1u) + tid,
+                           ((uint64_t)hi << 32) | ep);
+            }
+        }
         if (tid == 0) {
             if (rgp) {
                 // region window: no list space to reserve; the counters wait for the
@@ -1659,7 +1793,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         // or never read for neurons that do not integrate); meanwhile the list's
         // offset comes back from the atomic above
         if (fed && (!PW || kw + 1 == nw)) ring_slice_out(ring, gring, D, tn, slot0, nsteps, RW);
-        __syncthreads();
+        if (!rgp || a.rec) __syncthreads();
         for (uint32_t k = (uint32_t)tid; k < ((rgp && !a.rec) ? 0u : nl); k += (uint32_t)bd) {
             const uint32_t ent = lsp[k];
             if (rgp) {
@@ -1677,10 +1811,12 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             }
         }
         if constexpr (PW) {
-            if (kw + 1 < nw &&
-                !grid_wait(a.bar, (uint32_t)a.G, (uint32_t)g, (uint32_t)(kwin + 1), rgp ? sh->n : 0u,
-                           rgn_on ? rg_pre : nullptr, gt0, gt1, a.bar_err, a.spin_limit, &sh->bad))
-                return;
+            if (kw + 1 < nw) {
+                const uint32_t ep = (uint32_t)(kwin + 1);
+                const bool ok = RG ? grid_exchange(a.bar, ep, fcap, gt0, gt1, rg_lo, rg_pre, inl, a.bar_err, a.spin_limit, sh)
+                                   : grid_wait(a.bar, (uint32_t)g, ep, gt0, gt1, a.bar_err, a.spin_limit, &sh->bad);
+                if (!ok) return;
+            }
         }
     }   // windows
     if (own && tid0 < tn) store_neuron(t0 + tid0, own_st);
@@ -1857,10 +1993,19 @@ const void* tiled_fn_chunk(int chunk) {
     }
 }
 
-// The fused kernel for (kind, chunk); the persistent form exists for every kind without
-// STDP, and for the 16-bit CLASS words also with per-tile list regions (rg).
+// The fused kernel for (kind, chunk); the persistent forms, with lists and with spikes
+// that pass with the flags (rg), exist for every kind without STDP.
 const void* tiled_fn_of(int kind, int chunk, bool pw, bool rg = false) {
-    if (rg) return pw && kind == kTClass16 ? tiled_fn_chunk<kTClass16, true, true>(chunk) : nullptr;
+    if (rg) {
+        if (!pw) return nullptr;
+        switch (kind) {
+            case kTBF16: return tiled_fn_chunk<kTBF16, true, true>(chunk);
+            case kTFP8: return tiled_fn_chunk<kTFP8, true, true>(chunk);
+            case kTF32: return tiled_fn_chunk<kTF32, true, true>(chunk);
+            case kTClass16: return tiled_fn_chunk<kTClass16, true, true>(chunk);
+            default: return nullptr;
+        }
+    }
     switch (kind) {
         case kTBF16: return pw ? tiled_fn_chunk<kTBF16, true>(chunk) : tiled_fn_chunk<kTBF16, false>(chunk);
         case kTFP8: return pw ? tiled_fn_chunk<kTFP8, true>(chunk) : tiled_fn_chunk<kTFP8, false>(chunk);
@@ -1916,9 +2061,16 @@ hipError_t launch_tiled(const TiledArgs& a, int32_t off, int32_t wk, int32_t nst
     return launch_fn(tiled_fn_of(a.kind, a.chunk, false), a, off, wk, nsteps, 1, block, lds, st);
 }
 
-// Dynamic LDS of the persistent form: the window's, plus the list regions' counts.
+// Dynamic LDS of the persistent form: the window's, plus (region 2) two words per tile.
 size_t tiled_pw_lds_bytes(const TiledArgs& a) {
-    return tiled_lds_bytes(a.D, a.B, a.kind, a.rw, 0) + (a.region ? 2 * sizeof(uint32_t) * (size_t)a.G : 0);
+    return tiled_lds_bytes(a.D, a.B, a.kind, a.rw, 0) + (a.region == 2 ? 2 * sizeof(uint32_t) * (size_t)a.G : 0);
+}
+
+// Words of the staging area that the fused kernel leaves free (those without STDP).
+int32_t tiled_free_words(int kind) {
+    const size_t used = kind == kTClass16 ? 8 + 2 * kTiledBatch * 8 + 16 * kClassCache + sizeof(TileShared) + 2 * 12288
+                                          : 8 + kTiledBatch * 8 + sizeof(TileShared);
+    return (int32_t)((3 * kTiledBatch * 4 + (kind == kTClass16 ? 2 * kTiledItems : 0) - used) / 4);
 }
 
 hipError_t set_tiled_pw_lds_limit(const TiledArgs& a) {
@@ -1931,7 +2083,10 @@ hipError_t set_tiled_pw_lds_limit(const TiledArgs& a) {
 hipError_t launch_tiled_persistent(const TiledArgs& a, int32_t off, int32_t wk, int32_t nsteps, int32_t nwin,
                                    int block, hipStream_t st) {
     if (stdp_kind(a.kind) || !a.bar || !a.bar_err) return hipErrorInvalidValue;
-    if (a.region && (a.G > kRegionMaxG || a.G > block)) return hipErrorInvalidValue;
+    if (a.region && (a.G > kRegionMaxG || a.G > block || a.flag_cap < 0 || a.flag_cap > kInl ||
+                     (int64_t)a.flag_cap * a.G > 2 * tiled_batch(a.kind, block) ||
+                     (a.region == 1 && 2 * a.G > tiled_free_words(a.kind))))
+        return hipErrorInvalidValue;
     const void* f = tiled_fn_of(a.kind, a.chunk, true, a.region != 0);
     if (!f) return hipErrorInvalidDeviceFunction;
     return launch_fn(f, a, off, wk, nsteps, nwin, block, tiled_pw_lds_bytes(a), st);
