@@ -1069,6 +1069,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
 }
 
 void update_persist(mgb_sim* s);
+int32_t persistent_launches(const mgb_sim* s);
 
 mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
     const int32_t n = h.n;
@@ -1213,13 +1214,16 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
     }
     if (s->tiled) {
         update_persist(s);
-        if (s->tblock_auto && s->tblock > 512 && !s->persist && !stdp_kind(s->tkind) &&
-            s->persist_req != MGB_PERSIST_OFF) {
-            // (two workgroups of 512 may fit on a CU where one of more does)
-            const int32_t wide = s->tblock;
+        if (s->tblock_auto && s->tblock > 512 && !stdp_kind(s->tkind) && s->persist_req != MGB_PERSIST_OFF) {
+            // Two workgroups of 512 may fit on a CU where one of more does: 512 where only
+            // that is persistent, or where fewer launches of the wider block fit on the
+            // device at once, up to four (as many as the hardware queues run at once).
+            // Simulators run side by side on their streams, and two launches that are each
+            // partly resident would wait for each other.
+            const int32_t wide = s->tblock, launches = persistent_launches(s);
             s->tblock = 512;
             update_persist(s);
-            if (!s->persist) {
+            if (!s->persist || std::min(persistent_launches(s), 4) <= std::min(launches, 4)) {
                 s->tblock = wide;
                 update_persist(s);
             }
@@ -1277,6 +1281,15 @@ bool resident(const mgb_sim* s, const TiledArgs& a, bool persistent) {
 }
 
 TiledArgs tiled_args(const mgb_sim* s);
+
+// Launches of the simulator's persistent form that fit on the device at once.
+int32_t persistent_launches(const mgb_sim* s) {
+    int cus = 0;
+    if (!s->persist ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess)
+        return 0;
+    return (int32_t)((int64_t)cus * tiled_blocks_per_cu(tiled_args(s), s->tblock, true) / s->G);
+}
 
 // The launch form of the current launch shape, computed once per shape: the
 // XCD-contiguous tile order when every workgroup is resident, and persistent launches

@@ -43,3 +43,25 @@ def test_spikes_with_the_flags_without_records():
     (ca, va, na, ea), (cb, vb, nb, eb) = out
     assert na == nb > 200 and ea == eb
     assert np.array_equal(ca, cb) and np.array_equal(va, vb)
+
+
+def test_default_block_keeps_two_launches_on_the_device():
+    """256 tiles of 700: two persistent launches with workgroups of 512 fit on the device at
+    once, one with wider ones.  Two simulators side by side run as one by itself."""
+    _say("case: 179,200 neurons in 256 tiles, two simulators side by side")
+    pops = [dict(num=179200, type=N.LIFB, v_min=0.0, v_max=0.019)]
+    projs = [dict(src=0, tar=0, kind=N.CONN_FIXED_INDEGREE, k=20, w=2e-4, dmin=8e-4, dmax=8e-4, index=0, seed=3)]
+
+    def sim():
+        return N.Simulator.generated(pops, projs, W.lifb_consts(0.012), seed=3, propagation=N.PROP_TILED, tile_size=700)
+
+    alone, a, b = sim(), sim(), sim()
+    i = a.info()
+    assert i["persistent"] and 129 <= i["tiles"] <= 256 and i["tile_size"] > 512 and i["block"] == 512
+    alone.run(400)
+    v = alone.state(N.F_V).view(np.uint32)
+    for _ in range(4):
+        a.run(100)
+        b.run(100)
+    assert alone.info()["spikes"] > 1000
+    assert np.array_equal(a.state(N.F_V).view(np.uint32), v) and np.array_equal(b.state(N.F_V).view(np.uint32), v)
