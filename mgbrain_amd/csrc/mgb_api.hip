@@ -106,6 +106,7 @@ struct mgb_sim {
     uint64_t* seg_obase = nullptr;     // [nseg+1]
     uint64_t n_offs = 0, n_keys = 0;
     uint32_t* tcnt = nullptr;          // [3][nseg]
+    int64_t* tbase = nullptr;          // [3][nseg] (one segment: the control block's words)
     int tkind = kTClass16;             // synapse word kind of the fused kernel
     uint32_t* tperm = nullptr;         // fused STDP: CSR slot of each tile-order position (~0u: padding)
     uint64_t n_tslots = 0;             // length of the (padded) tile-order arrays
@@ -1161,6 +1162,12 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
     if (s->tiled) {
         MGB_TRY(dalloc_n(s, &s->tcnt, 3 * (size_t)s->nseg));
         MGB_HIP_TRY(hipMemsetAsync(s->tcnt, 0, 12 * (size_t)s->nseg, st));
+        if (s->nseg == 1) {
+            s->tbase = reinterpret_cast<int64_t*>(reinterpret_cast<uint8_t*>(s->ctl) + offsetof(Ctl, tbase));
+        } else {
+            MGB_TRY(dalloc_n(s, &s->tbase, 3 * (size_t)s->nseg));
+            MGB_HIP_TRY(hipMemsetAsync(s->tbase, 0, 24 * (size_t)s->nseg, st));
+        }
     }
     // record
     s->rec_cap = o ? std::max<int64_t>(o->record_capacity, 0) : 0;
@@ -1347,6 +1354,7 @@ TiledArgs tiled_args(const mgb_sim* s) {
     a.nseg = s->nseg; a.window = s->window;
     a.tile_lo = s->tile_lo; a.tile_seg = s->tile_seg; a.seg_lo = s->seg_lo;
     a.seg_tile0 = s->seg_tile0; a.seg_obase = s->seg_obase; a.tcnt = s->tcnt;
+    a.tbase = s->tbase;
     a.type = s->type; a.cset = s->cset; a.tbl = s->tbl; a.stream = s->stream_idx;
     a.rate = s->rate; a.V = s->V; a.Ie = s->Ie; a.Ii = s->Ii;
     a.refr = s->refr; a.last = s->last; a.cnt = s->cnt;
@@ -2362,6 +2370,12 @@ mgb_status mgb_checkpoint_load(mgb_sim* s, const void* buf, int64_t bytes) {
         off += g.bytes;
     }
     MGB_HIP_TRY(hipMemcpy(&s->mir->ctl, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+    if (s->tiled && s->nseg > 1) {
+        // the lists' start steps, the same in every segment between runs
+        std::vector<int64_t> tb(3 * (size_t)s->nseg);
+        for (int b = 0; b < 3; ++b) std::fill_n(tb.begin() + (size_t)b * s->nseg, s->nseg, s->mir->ctl.tbase[b]);
+        MGB_HIP_TRY(hipMemcpy(s->tbase, tb.data(), 8 * tb.size(), hipMemcpyHostToDevice));
+    }
     // the persistent waits' flags hold window indices of the run before (epochs)
     if (s->bar) MGB_HIP_TRY(hipMemset(s->bar, 0, 4 * (size_t)s->G * kBarStride));
     return MGB_OK;

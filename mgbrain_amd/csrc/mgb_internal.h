@@ -50,8 +50,9 @@ struct Ctl {
     uint64_t rec_cnt;       // spikes recorded (may exceed capacity)
     uint64_t se;            // synaptic events
     // fused tiled path: three spike lists (write k%3, read (k-1)%3, clear (k+1)%3);
-    // their per-segment counters live in TiledArgs::tcnt
-    int64_t tbase[3];       // first step of the window that wrote each list
+    // their per-segment counters and start steps live in TiledArgs::tcnt and tbase
+    int64_t tbase[3];       // first step of the window that wrote each list (segment 0's, for
+                            // checkpoints: between runs all segments' are the same)
 };
 
 
@@ -189,6 +190,7 @@ struct TiledArgs {
     const int32_t* seg_tile0;   // [nseg+1] first tile of each segment
     const uint64_t* seg_obase;  // [nseg+1] first offset entry of each segment
     uint32_t* tcnt;             // [3][nseg] entries in each segment's spike lists
+    int64_t* tbase;             // [3][nseg] first step of the window that wrote each (mgb_lists.h)
     const uint8_t* type;
     const uint8_t* cset;
     const uint16_t* tbl;

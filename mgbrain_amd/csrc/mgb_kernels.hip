@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "mgb_internal.h"
+#include "mgb_lists.h"
 #include "mgb_rng.h"
 
 namespace mgb {
@@ -612,8 +613,8 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
 // `epoch` in its flag, words kBarStride apart per tile (a cache line each), even epochs in
 // one and odd ones in another, and waits until the flag of this parity of every
 // workgroup of its segment (tiles [ct0, ct1)) holds `epoch`, one flag per thread.
-// Workgroups of other segments share no list with it and may be any number of windows
-// ahead or behind.  One of its own segment can be one window ahead -- its tile may have
+// Workgroups of other segments share no list and no list's start step (mgb_lists.h) with it
+// and may be any number of windows ahead or behind.  One of its own segment can be one window ahead -- its tile may have
 // little to do -- and have published epoch + 1 before this one reads its flag (two ahead
 // it cannot be): with one word for both parities, what else the flag holds
 // (grid_exchange) would be the next window's.  A poll is one load, back to back with the
@@ -1100,11 +1101,10 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         uint32_t E, ent0;
         if (kw == 0) {
             const size_t ws = a.win_stride;
-            const int64_t tb0 = ctl->tbase[0], tb1 = ctl->tbase[1], tb2 = ctl->tbase[2];
+            sprev = list_start(a.tbase, q, nseg, bprev);
             const uint32_t n0 = tcnt[0], n1 = tcnt[nseg], n2 = tcnt[2 * nseg];
             const uint32_t l0 = a.win_buf[lbase + li], l1 = a.win_buf[ws + lbase + li];
             const uint32_t l2 = a.win_buf[2 * ws + lbase + li];
-            sprev = bprev == 0 ? tb0 : (bprev == 1 ? tb1 : tb2);
             E = bprev == 0 ? n0 : (bprev == 1 ? n1 : n2);
             ent0 = bprev == 0 ? l0 : (bprev == 1 ? l1 : l2);
             if (!fed) E = 0u;
@@ -1141,7 +1141,10 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             else tcnt[bnext * nseg] = 0u;
         }
         if (kPl && full && g == 0 && tid == 0) a.fcnt[(kwin + 1) & 1] = 0u;
-        if (full && g == 0 && tid == 0) ctl->tbase[bcur] = s0;
+        if (full && lt == 0 && tid == 0) {
+            set_list_start(a.tbase, q, nseg, bcur, s0);
+            if (g == 0) ctl->tbase[bcur] = s0;          // (for checkpoints)
+        }
         if (tid == 0) {
             sh->se = 0ull;
             sh->n = 0u;
