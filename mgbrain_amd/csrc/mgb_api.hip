@@ -367,14 +367,14 @@ uint64_t host_u64(const void* p) {
 
 // Tile shape of the fused path.  Tiles never straddle a segment boundary and
 // never mix neuron types (one update path per tile).  Within a segment they are
-// balanced by weight — a neuron weighs its in-degree plus half the mean
-// in-degree of the neurons that have one (its own update) — so tiles of neurons
+// balanced by weight — a neuron weighs its in-degree (StatArgs::in_bal) plus half the
+// mean in-degree of the neurons that have one (its own update) — so tiles of neurons
 // without input (Poisson) are larger and the others share the synapses evenly.
 // A segment of Nq neurons gets at most max(ceil(Nq / B), its type runs) tiles
 // (B the requested mean tile size, default max(256, n / 256)) of at most the
 // LDS limit; the smallest per-tile weight cap meeting that is found by bisection.
 mgb_status choose_tiles(mgb_sim* s, const mgb_opts* o, int32_t n, int32_t D, const std::vector<uint8_t>& type,
-                        const std::vector<uint32_t>& indeg) {
+                        const std::vector<uint32_t>& in_bal) {
     int lds_max = 65536;
     (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, s->device);
     lds_max = std::min(lds_max, 160 * 1024);
@@ -398,14 +398,14 @@ mgb_status choose_tiles(mgb_sim* s, const mgb_opts* o, int32_t n, int32_t D, con
     double sum_in = 0.0;
     int64_t cnt_in = 0;
     for (int32_t t = 0; t < n; ++t) {
-        const uint32_t d = indeg[t] + indeg[(size_t)n + t];
+        const uint32_t d = in_bal[t] + in_bal[(size_t)n + t];
         if (d) {
             sum_in += d;
             ++cnt_in;
         }
     }
     const double base = cnt_in ? 0.5 * sum_in / (double)cnt_in : 1.0;
-    for (int32_t t = 0; t < n; ++t) wt[t] = (double)(indeg[t] + indeg[(size_t)n + t]) + base;
+    for (int32_t t = 0; t < n; ++t) wt[t] = (double)(in_bal[t] + in_bal[(size_t)n + t]) + base;
     // tiles of [a, b) under weight cap T; their starts appended to `cuts`
     auto greedy = [&](int32_t a, int32_t b, double T, std::vector<int32_t>* cuts) {
         int32_t count = 0, start = a;
@@ -506,7 +506,7 @@ mgb_status choose_tiles(mgb_sim* s, const mgb_opts* o, int32_t n, int32_t D, con
     std::vector<uint8_t> tin(tseg.size(), 0);
     for (size_t g = 0; g + 1 < tlo.size(); ++g)
         for (int32_t t = tlo[g]; t < tlo[g + 1] && !tin[g]; ++t)
-            tin[g] = (indeg[t] | indeg[(size_t)n + t]) != 0u ? 1 : 0;
+            tin[g] = (in_bal[t] | in_bal[(size_t)n + t]) != 0u ? 1 : 0;
     MGB_TRY(dalloc_n(s, &s->tile_in, tin.size()));
     MGB_HIP_TRY(hipMemcpyAsync(s->tile_in, tin.data(), tin.size(), hipMemcpyHostToDevice, st));
     MGB_TRY(dalloc_n(s, &s->seg_lo, lo.size()));
@@ -700,14 +700,15 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     Scratch X;
     // ---- statistics + delay quantisation --------------------------------------
     uint8_t* dq = nullptr;
-    uint32_t *flags = nullptr, *wcls = nullptr, *indeg = nullptr, *in_pl = nullptr, *absmax = nullptr;
+    uint32_t *flags = nullptr, *wcls = nullptr, *in_bal = nullptr, *in_more = nullptr, *in_pl = nullptr, *absmax = nullptr;
     int32_t* mm = nullptr;
     unsigned long long* npl = nullptr;
     MGB_TRY(X.get(&dq, S));
     MGB_TRY(X.get(&flags, 1));
     MGB_TRY(X.get(&mm, 2));
     MGB_TRY(X.get(&wcls, 2 * (size_t)n));
-    MGB_TRY(X.get(&indeg, 2 * (size_t)n));
+    MGB_TRY(X.get(&in_bal, 2 * (size_t)n));
+    MGB_TRY(X.get(&in_more, 2 * (size_t)n));
     MGB_TRY(X.get(&in_pl, (size_t)n));
     MGB_TRY(X.get(&npl, 1));
     std::vector<uint16_t> run_of;
@@ -723,7 +724,8 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_HIP_TRY(hipMemsetAsync(flags, 0, 4, st));
     MGB_HIP_TRY(hipMemcpyAsync(mm, mm_init, 8, hipMemcpyHostToDevice, st));
     MGB_HIP_TRY(hipMemsetAsync(wcls, 0xFF, 8 * (size_t)n, st));
-    MGB_HIP_TRY(hipMemsetAsync(indeg, 0, 8 * (size_t)n, st));
+    MGB_HIP_TRY(hipMemsetAsync(in_bal, 0, 8 * (size_t)n, st));
+    MGB_HIP_TRY(hipMemsetAsync(in_more, 0, 8 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(in_pl, 0, 4 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(absmax, 0, 4 * std::max<size_t>(nruns, 1), st));
     MGB_HIP_TRY(hipMemsetAsync(npl, 0, 8, st));
@@ -734,7 +736,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         a.plastic = h.stdp ? L.plastic : nullptr;
         a.seg = seg_dev;                                   // null for one run: absmax[0]
         a.dq = dq; a.flags = flags; a.min_d = mm; a.max_d = mm + 1;
-        a.wcls = wcls; a.indeg = indeg; a.in_pl = in_pl; a.absmax = absmax; a.n_plastic = npl;
+        a.wcls = wcls; a.in_bal = in_bal; a.in_more = in_more; a.in_pl = in_pl; a.absmax = absmax; a.n_plastic = npl;
         MGB_HIP_TRY(run_stats(a, st));
     }
     uint32_t hflags = 0;
@@ -745,10 +747,12 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_HIP_TRY(hipMemcpyAsync(hmm, mm, 8, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipMemcpyAsync(habs.data(), absmax, 4 * habs.size(), hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipMemcpyAsync(&hnpl, npl, 8, hipMemcpyDeviceToHost, st));
-    std::vector<uint32_t> h_wcls(2 * (size_t)n), h_indeg(2 * (size_t)n);
+    std::vector<uint32_t> h_wcls(2 * (size_t)n), h_bal(2 * (size_t)n), h_indeg(2 * (size_t)n);
     MGB_HIP_TRY(hipMemcpyAsync(h_wcls.data(), wcls, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
-    MGB_HIP_TRY(hipMemcpyAsync(h_indeg.data(), indeg, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
+    MGB_HIP_TRY(hipMemcpyAsync(h_bal.data(), in_bal, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
+    MGB_HIP_TRY(hipMemcpyAsync(h_indeg.data(), in_more, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipStreamSynchronize(st));
+    for (size_t k = 0; k < h_indeg.size(); ++k) h_indeg[k] += h_bal[k];
     if (hflags & kFlagBadId) {
         set_error("a synapse references a neuron id outside [0, %d)", n);
         return MGB_ERR_INVALID;
@@ -769,11 +773,8 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     // spike rows of ~256 synapses per wave in the direct kernels
     s->split = (int32_t)std::max<int64_t>(1, std::min<int64_t>(32, (int64_t)(S / (uint64_t)n) / 256));
     s->n_plastic = (int64_t)hnpl;
-    uint32_t max_deg_cls = 0, max_deg_tot = 0;
-    for (int32_t t = 0; t < n; ++t) {
-        max_deg_cls = std::max({max_deg_cls, h_indeg[t], h_indeg[(size_t)n + t]});
-        max_deg_tot = std::max(max_deg_tot, h_indeg[t] + h_indeg[(size_t)n + t]);
-    }
+    uint32_t max_deg_cls = 0;
+    for (uint32_t d : h_indeg) max_deg_cls = std::max(max_deg_cls, d);
     // ---- format choice ----------------------------------------------------------
     const bool class_ok = !(hflags & kFlagMixed) && !h.stdp && max_d <= kClassMaxDelay &&
                           max_deg_cls <= 0xFFFFu;
@@ -833,8 +834,8 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                 id = it->second;
             }
             s->h_tbl[t] = (uint16_t)id;
-            tmax_e[id] = std::max(tmax_e[id], h_indeg[t]);
-            tmax_i[id] = std::max(tmax_i[id], h_indeg[(size_t)n + t]);
+            tmax_e[id] = std::max(tmax_e[id], h_bal[t]);
+            tmax_i[id] = std::max(tmax_i[id], h_bal[(size_t)n + t]);
         }
         if (keys.size() > 0xFFFFu) {
             set_error("too many weight classes (%zu)", keys.size());
@@ -881,7 +882,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         s->tiled = (prop == MGB_PROP_AUTO || prop == MGB_PROP_TILED) ? 1 : 0;
         s->tkind = kTClass16;
         if (s->tiled) {
-            MGB_TRY(choose_tiles(s, o, n, s->D, h.type, h_indeg));
+            MGB_TRY(choose_tiles(s, o, n, s->D, h.type, h_bal));
             // tile-sorted copy: stable sort by (source, target tile) keeps list order
             // inside every (source, tile) sub-row
             const TileTabs tt = tile_tabs(s, seg_dev);
@@ -916,7 +917,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         std::vector<float2> seg_sc(nseg);
         for (size_t q = 0; q < nseg; ++q) {
             uint32_t deg = 0, abits = 0;
-            for (int32_t t = slo[q]; t < slo[q + 1]; ++t) deg = std::max(deg, h_indeg[t] + h_indeg[(size_t)n + t]);
+            for (int32_t t = slo[q]; t < slo[q + 1]; ++t) deg = std::max(deg, h_bal[t] + h_bal[(size_t)n + t]);
             if (nseg == nruns) abits = habs[q];
             else for (uint32_t b : habs) abits = std::max(abits, b);      // one segment
             float wabs = 0.f;
@@ -981,7 +982,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
             for (int32_t i = 0; i < n && lifb_only; ++i)
                 lifb_only = h.type[i] != MGB_LIF && h.type[i] != MGB_LIFE;
             s->trw = lifb_only ? 1 : 2;
-            MGB_TRY(choose_tiles(s, o, n, s->D, h.type, h_indeg));
+            MGB_TRY(choose_tiles(s, o, n, s->D, h.type, h_bal));
             const TileTabs tt = tile_tabs(s, seg_dev);
             // kout holds each CSR slot's source (the keys of the sort by source)
             MGB_HIP_TRY(make_tile_keys_csr(kout, s->col, tt, kin, vin, S, st));

@@ -26,8 +26,11 @@ struct StatArgs {
     int32_t* min_d;
     int32_t* max_d;
     uint32_t* wcls;         // [2][n] class weight bits per target
-    uint32_t* indeg;        // [2][n] in-degree per target and class, a wave of 64 synapses of one
-                            // target and class counted as one (target-major lists)
+    // [2][n] in-degree per target and class, in two parts: in_bal counts a wave of 64 synapses
+    // of one target and class (target-major lists) as one, in_more has its other 63.  Tile
+    // boundaries, which saved checkpoints rest on, balance by the first part alone
+    uint32_t* in_bal;
+    uint32_t* in_more;
     uint32_t* in_pl;        // [n] plastic in-degree
     uint32_t* absmax;       // max |w| (float bits)
     unsigned long long* n_plastic;

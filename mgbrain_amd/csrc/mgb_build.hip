@@ -87,14 +87,13 @@ __global__ void k_stats(StatArgs a) {
         }
         // in-degree per (target, class); target-major lists hit one address per wave
         if (wave_all_equal(key)) {
-            // (counted as one: the ballot is of this one lane.  Tile boundaries, fixed-point
-            // scales and class tables rest on it, and with them checkpoints and results)
             if (key != 0xFFFFFFFFu && (threadIdx.x & 63u) == 0u) {
-                const uint32_t c = (uint32_t)__popcll(__ballot(true));
-                atomicAdd(&a.indeg[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], c);
+                const size_t at = (size_t)(key & 1u) * (size_t)a.n + (key >> 1);
+                atomicAdd(&a.in_bal[at], 1u);
+                atomicAdd(&a.in_more[at], 63u);
             }
         } else if (key != 0xFFFFFFFFu) {
-            atomicAdd(&a.indeg[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], 1u);
+            atomicAdd(&a.in_bal[(size_t)(key & 1u) * (size_t)a.n + (key >> 1)], 1u);
         }
     }
 #pragma unroll
