@@ -834,21 +834,31 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                 id = it->second;
             }
             s->h_tbl[t] = (uint16_t)id;
-            tmax_e[id] = std::max(tmax_e[id], h_bal[t]);
-            tmax_i[id] = std::max(tmax_i[id], h_bal[(size_t)n + t]);
+            // (a neuron's arrivals of one sign in one step are at most its synapses of it)
+            tmax_e[id] = std::max(tmax_e[id], h_indeg[t]);
+            tmax_i[id] = std::max(tmax_i[id], h_indeg[(size_t)n + t]);
         }
         if (keys.size() > 0xFFFFu) {
             set_error("too many weight classes (%zu)", keys.size());
             return MGB_ERR_UNSUPPORTED;
         }
         s->n_tbl = (int32_t)keys.size();
+        // (all tables together: at most one entry per synapse and two per class, so that their
+        // offsets fit in 32 bits)
+        uint64_t n_seq = 0;
+        for (size_t c = 0; c < keys.size(); ++c) n_seq += (uint64_t)tmax_e[c] + tmax_i[c] + 2u;
+        if (n_seq > 0xFFFFFFFFull) {
+            set_error("class sum tables of %llu entries", (unsigned long long)n_seq);
+            return MGB_ERR_UNSUPPORTED;
+        }
         std::vector<uint32_t> offs(2 * keys.size());
         std::vector<float> seq;
+        seq.reserve((size_t)n_seq);
         s->class_w.assign(2 * keys.size(), 0.f);
         for (size_t c = 0; c < keys.size(); ++c) {
             for (int side = 0; side < 2; ++side) {
                 const uint32_t bits = side ? keys[c].second : keys[c].first;
-                const uint32_t len = std::max<uint32_t>((side ? tmax_i[c] : tmax_e[c]) + 1, kClassTableMin);
+                const uint32_t len = (side ? tmax_i[c] : tmax_e[c]) + 1;
                 float w = 0.f;
                 if (bits != kWSentinel) std::memcpy(&w, &bits, 4);
                 s->class_w[2 * c + side] = w;
@@ -863,16 +873,9 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                 }
             }
         }
-        // Counts are 16 bits and a table ends at the in-degree k_stats counted, which is a
-        // 64th of the real one where a list goes target by target: a larger count reads on
-        // into the tables that follow and these zeros.  (Known: such a sum is not the k-fold
-        // one.  Results, like the tile boundaries and fixed-point scales that rest on the
-        // same count, stay as they are.)
-        constexpr size_t kSeqPad = 0x10000;
         MGB_TRY(dalloc_n(s, &s->tbl, (size_t)n));
         MGB_TRY(dalloc_n(s, &s->tbl_off, offs.size()));
-        MGB_TRY(dalloc_n(s, &s->seq, seq.size() + kSeqPad));
-        MGB_HIP_TRY(hipMemsetAsync(s->seq + seq.size(), 0, 4 * kSeqPad, st));
+        MGB_TRY(dalloc_n(s, &s->seq, seq.size()));
         MGB_TRY(dalloc_n(s, &s->tbl_w, s->class_w.size()));
         MGB_HIP_TRY(hipMemcpyAsync(s->tbl_w, s->class_w.data(), 4 * s->class_w.size(), hipMemcpyHostToDevice, st));
         MGB_HIP_TRY(hipMemcpyAsync(s->tbl, s->h_tbl.data(), 2 * (size_t)n, hipMemcpyHostToDevice, st));
@@ -905,7 +908,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
             MGB_TRY(pad_subrows(s, n));
             MGB_TRY(dalloc_n(s, &s->tile_cc, (size_t)s->G * 4 * kClassCache));
             MGB_TRY(dalloc_n(s, &s->tile_ccls, (size_t)s->G * 2));
-            MGB_HIP_TRY(launch_tile_ccache(s->tile_lo, s->G, s->tbl, s->tbl_off, s->seq, (uint32_t)(seq.size() + kSeqPad),
+            MGB_HIP_TRY(launch_tile_ccache(s->tile_lo, s->G, s->tbl, s->tbl_off, s->seq, (uint32_t)seq.size(),
                                            s->tile_cc, s->tile_ccls, st));
         }
         MGB_HIP_TRY(hipStreamSynchronize(st));

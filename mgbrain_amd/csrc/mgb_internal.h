@@ -294,7 +294,6 @@ constexpr int kTiledItems = 16384;  // work items staged in LDS per propagation 
 // Bytes of a workgroup's LDS left out when the widest tile is chosen (the kernel has no
 // static LDS; tile boundaries belong to a checkpoint's layout, so the bound stays)
 constexpr int kTiledStaticLds = 1024;
-constexpr uint32_t kClassTableMin = 32; // shortest k-fold class sum table
 constexpr int kClassCache = 128;    // k-fold class sums cached in LDS per class and side
 // Most leading entries of an STDP table copied to LDS in every window (4e7 synapses at
 // 26 Hz: 33.2 us with 1024, 33.4 with 2048, 33.6 with 4096, 34.0 with 8192; slower networks

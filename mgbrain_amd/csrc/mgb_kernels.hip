@@ -2039,7 +2039,7 @@ __global__ void k_tile_ccache(const int32_t* tile_lo, const uint16_t* tbl, const
     const int32_t c = tid / (2 * kClassCache), side = (tid / kClassCache) & 1, k = tid % kClassCache;
     const int32_t t0 = tile_lo[g], t1 = tile_lo[g + 1];
     const uint32_t cl = tbl[c == 0 ? t1 - 1 : t0];
-    // (past a class's own table: what follows it, as the reads of larger counts)
+    // (entries past a class's own table are never read: no neuron receives as many)
     cc[(size_t)g * 4 * kClassCache + tid] = seq[min(tbl_off[2 * cl + side] + (uint32_t)k, n_seq - 1u)];
     if (side == 0 && k == 0) cls[2 * g + c] = cl;
 }
