@@ -150,6 +150,7 @@ struct mgb_sim {
     int flag_cap = 0;                  // (TiledArgs::flag_cap)
     int region = 0;                    // persistent launches: spikes with the flags (TiledArgs::region)
     uint64_t tile_hash = 0;            // FNV-1a of the tile boundaries (the ring slices' layout)
+    uint64_t scale_hash = 0;           // of the fixed-point scales that fit_scales lowered (0: none)
     // host mirrors for read-back
     std::vector<float> class_w;        // [n_tbl][2]
     std::vector<uint16_t> h_tbl;       // [n]
@@ -685,6 +686,61 @@ std::vector<int32_t> stream_runs(const HostNeurons& h, std::vector<uint16_t>& ru
     return lo;
 }
 
+// Lowers the fixed-point scales of segments whose ring words could leave int32 until none
+// can: first by in-degree * max |w| alone, then, where that does not settle it, by each
+// target's own sums (RingSumArgs).  The weights' codes are those of the format (row scales
+// set).  A scale that is lowered joins the layout that a checkpoint has to match, its ring
+// words being multiples of 1 / scale.
+mgb_status fit_scales(mgb_sim* s, const HostNeurons& h, const DevList& L, const std::vector<uint32_t>& indeg,
+                      const std::vector<float>& w_seg, const uint16_t* seg, std::vector<float2>& sc) {
+    const size_t n = (size_t)h.n, nseg = sc.size();
+    const std::vector<int32_t>& lo = s->h_seg_lo;
+    constexpr double kMax = 2147483647.0;
+    bool safe = h.fp8_scale.empty();       // (a caller's FP8 scale may round far above max |w|)
+    for (size_t q = 0; q < nseg && safe; ++q) {
+        uint32_t deg = 0;
+        for (int32_t t = lo[q]; t < lo[q + 1]; ++t) deg = std::max(deg, indeg[t] + indeg[n + t]);
+        safe = (double)deg * ((double)w_seg[q] * (double)sc[q].x + 0.5) <= kMax;
+    }
+    if (safe || L.S == 0) return MGB_OK;
+    Scratch X;
+    RingSumArgs a{};
+    float* scale = nullptr;
+    MGB_TRY(X.get(&scale, nseg));
+    MGB_TRY(X.get(&a.sums, 2 * n));
+    a.S = L.S; a.n = h.n;
+    a.src = L.src; a.tar = L.tar; a.weight = L.weight;
+    a.plastic = h.stdp ? L.plastic : nullptr;
+    a.w_plastic = h.stdp ? std::max(std::fabs(h.stdpconst[4]), std::fabs(h.stdpconst[5])) : 0.f;
+    a.bits = s->wide_kind == kWideBF16 ? 16 : (s->wide_kind == kWideFP8 ? 8 : 32);
+    a.row_scale = s->row_scale;
+    a.seg = seg;
+    a.scale = scale;
+    std::vector<unsigned long long> sums(2 * n);
+    std::vector<float> now(nseg);
+    for (int pass = 0; pass < 8; ++pass) {
+        for (size_t q = 0; q < nseg; ++q) now[q] = sc[q].x;
+        MGB_HIP_TRY(hipMemcpyAsync(scale, now.data(), 4 * nseg, hipMemcpyHostToDevice, s->stream));
+        MGB_HIP_TRY(hipMemsetAsync(a.sums, 0, 16 * n, s->stream));
+        MGB_HIP_TRY(ring_sums(a, s->stream));
+        MGB_HIP_TRY(hipMemcpyAsync(sums.data(), a.sums, 16 * n, hipMemcpyDeviceToHost, s->stream));
+        MGB_HIP_TRY(hipStreamSynchronize(s->stream));
+        bool fits = true;
+        for (size_t q = 0; q < nseg; ++q) {
+            unsigned long long m = 0;
+            for (int32_t t = lo[q]; t < lo[q + 1]; ++t) m = std::max({m, sums[t], sums[n + t]});
+            if ((double)m <= kMax || sc[q].x <= 0x1p-100f) continue;
+            const int by = std::max(1, (int)std::ceil(std::log2((double)m / kMax)));
+            const int e = std::max(-100, std::ilogb(sc[q].x) - by);
+            sc[q] = make_float2(std::ldexp(1.0f, e), std::ldexp(1.0f, -e));
+            s->scale_hash = (s->scale_hash ^ (((uint64_t)q << 32) | (uint32_t)(e + 128))) * 1099511628211ull + 1ull;
+            fits = false;
+        }
+        if (fits) break;
+    }
+    return MGB_OK;
+}
+
 // Builds device CSR + tables from a device synapse list; frees nothing of `L`.
 mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int wf_req,
                          const mgb_opts* o) {
@@ -913,11 +969,14 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         }
         MGB_HIP_TRY(hipStreamSynchronize(st));
     } else {
-        // fixed-point scale per segment (a batched network gets the scale it has
-        // alone): |ring value| <= in-degree * max |w| < 2^31
+        // Fixed-point scale per segment: a power of two with in-degree * max |w| < 2^31, the
+        // in-degree by its part in_bal (for lists that are not in target order the whole of
+        // it: a batched network gets the scale it has alone).  Where that could let a
+        // target's inputs of one sign leave int32, fit_scales below lowers it
         const std::vector<int32_t>& slo = s->h_seg_lo;
         const size_t nseg = slo.size() - 1;
         std::vector<float2> seg_sc(nseg);
+        std::vector<float> w_seg(nseg);
         for (size_t q = 0; q < nseg; ++q) {
             uint32_t deg = 0, abits = 0;
             for (int32_t t = slo[q]; t < slo[q + 1]; ++t) deg = std::max(deg, h_bal[t] + h_bal[(size_t)n + t]);
@@ -927,18 +986,12 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
             std::memcpy(&wabs, &abits, 4);
             if (h.stdp) wabs = std::max({wabs, std::fabs(h.stdpconst[4]), std::fabs(h.stdpconst[5])});
             if (s->wide_kind != kWideF32) wabs *= 1.0625f;   // BF16 / FP8 rounding headroom
+            w_seg[q] = wabs;
             const double bound = (double)std::max<uint32_t>(deg, 1) * (double)wabs;
             int e = 30;
             if (bound > 0) e = (int)std::floor(std::log2(2147483520.0 / bound));
             e = std::max(-100, std::min(e, 100));
             seg_sc[q] = make_float2(std::ldexp(1.0f, e), std::ldexp(1.0f, -e));
-        }
-        s->scale_e = s->scale_i = seg_sc[0].x;
-        if (nseg > 1) {
-            MGB_TRY(dalloc_n(s, &s->seg_scale, nseg));
-            MGB_TRY(dalloc_n(s, &s->seg_of, (size_t)n));
-            MGB_HIP_TRY(hipMemcpyAsync(s->seg_scale, seg_sc.data(), sizeof(float2) * nseg, hipMemcpyHostToDevice, st));
-            MGB_HIP_TRY(hipMemcpyAsync(s->seg_of, run_of.data(), 2 * (size_t)n, hipMemcpyHostToDevice, st));
         }
         MGB_TRY(dalloc_n(s, &s->col, S));
         MGB_TRY(dalloc_n(s, &s->dly, S));
@@ -957,6 +1010,14 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                 MGB_HIP_TRY(row_scales(L.src, L.weight, S, n, s->wide_kind == kWideFP8 ? 448.f : 1.f, rmax,
                                        s->row_scale, st));
             }
+        }
+        MGB_TRY(fit_scales(s, h, L, h_indeg, w_seg, nseg > 1 ? seg_dev : nullptr, seg_sc));
+        s->scale_e = s->scale_i = seg_sc[0].x;
+        if (nseg > 1) {
+            MGB_TRY(dalloc_n(s, &s->seg_scale, nseg));
+            MGB_TRY(dalloc_n(s, &s->seg_of, (size_t)n));
+            MGB_HIP_TRY(hipMemcpyAsync(s->seg_scale, seg_sc.data(), sizeof(float2) * nseg, hipMemcpyHostToDevice, st));
+            MGB_HIP_TRY(hipMemcpyAsync(s->seg_of, run_of.data(), 2 * (size_t)n, hipMemcpyHostToDevice, st));
         }
         uint32_t* pos_of = nullptr;
         if (h.stdp) MGB_TRY(X.get(&pos_of, S));
@@ -2242,7 +2303,7 @@ struct CkptHeader {
     int32_t abi, n, npad, D, window, tiled, tkind, B, G, nseg, mode, wide_kind, stdp;
     int64_t S, n_rec;
     uint64_t payload;
-    uint64_t tiling;        // hash of the tile boundaries (the ring slices' layout)
+    uint64_t tiling;        // hash of the tile boundaries (the ring slices' layout) and lowered scales
 };
 
 struct CkptSeg {
@@ -2288,7 +2349,7 @@ CkptHeader ckpt_header(const mgb_sim* s, uint64_t n_rec) {
     h.n = s->n; h.npad = s->npad; h.D = s->D; h.window = s->window; h.tiled = s->tiled;
     h.tkind = s->tkind; h.B = s->B; h.G = s->G; h.nseg = s->nseg; h.mode = s->mode;
     h.wide_kind = s->wide_kind; h.stdp = s->stdp; h.S = s->S; h.n_rec = (int64_t)n_rec;
-    h.tiling = s->tile_hash;
+    h.tiling = s->tile_hash ^ s->scale_hash;
     for (const CkptSeg& g : ckpt_segments(s, n_rec)) h.payload += g.bytes;
     return h;
 }

@@ -65,6 +65,24 @@ struct GatherArgs {
     uint32_t* pos_of;       // [S] CSR slot of each list index (NULL if unused)
 };
 
+// The largest value a ring word can hold: per target and sign, the sum of its synapses'
+// fixed-point inputs (each arrives at most once in a step), a plastic one with the largest
+// weight it can have, of either sign.
+struct RingSumArgs {
+    uint64_t S;
+    int32_t n;
+    const int32_t* src;
+    const int32_t* tar;
+    const float* weight;
+    const uint8_t* plastic;     // NULL: none
+    float w_plastic;            // largest |w| a plastic synapse can reach
+    int bits;                   // 32, or the 16 / 8 of a BF16 / FP8 code times row_scale
+    const float* row_scale;
+    const uint16_t* seg;        // [n] segment of each target (NULL: one)
+    const float* scale;         // [segments] fixed-point scale
+    unsigned long long* sums;   // [2][n], zeroed
+};
+
 struct GenProjArgs {
     int32_t sn, tn, s0, t0, k;
     uint32_t index;         // projection index in its network (Philox counter word)
@@ -137,6 +155,7 @@ hipError_t sort_pairs(void* temp, size_t* temp_bytes, const uint32_t* kin, uint3
 hipError_t row_bounds(const uint32_t* sorted_keys, uint64_t S, int32_t n, int64_t* out,
                       hipStream_t st);
 hipError_t gather_wide(const GatherArgs& a, hipStream_t st);
+hipError_t ring_sums(const RingSumArgs& a, hipStream_t st);
 hipError_t in_fill(const uint32_t* sorted_idx, const uint32_t* pos_of, const int32_t* src,
                    uint64_t np, uint32_t* in_pos, int32_t* in_src, hipStream_t st);
 hipError_t gen_fixk(const GenProjArgs& g, hipStream_t st);

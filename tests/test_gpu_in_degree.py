@@ -77,3 +77,91 @@ def test_the_most_arrivals_of_a_class_word(prop):
         v = np.float32(v + np.float32(np.float64(acc) + np.float64(np.float32(-0.005)) * np.float64(v)))
     for o in out:
         assert np.array_equal(o.view(np.uint32), np.array([v, v]).view(np.uint32)), (o, v)
+
+
+def _driven(k, w, d=1e-3, n=300, seed=3, plastic=0, g=None):
+    """n LIFB neurons with k inputs of weight w each (fixed in-degree: listed target by
+    target) from a pool that fires in every step, and with g as many of weight g."""
+    pops = [dict(num=700, type=N.POISSON, rate=1.0), dict(num=n, type=N.LIFB, v_min=0.0, v_max=0.0)]
+    projs = [dict(src=0, tar=1, kind=N.CONN_FIXED_INDEGREE, k=k, w=x, dmin=d, dmax=d, index=j, seed=seed, plastic=plastic)
+             for j, x in enumerate((w,) if g is None else (w, g))]
+    return dict(pops=pops, projs=projs, lifconst=W.lifb_consts(), seed=seed)
+
+
+def _v_after(total, steps):
+    v = 0.0
+    for _ in range(steps):
+        v += total - 0.005 * v
+    return v
+
+
+FORMATS = [N.WF_F32, N.WF_BF16, N.WF_FP8]
+
+
+@pytest.mark.parametrize("prop", [N.PROP_TILED, N.PROP_DIRECT])
+@pytest.mark.parametrize("wf", FORMATS)
+@pytest.mark.parametrize("k", [63, 130, 1000, 6400])
+def test_all_inputs_of_a_step_fit_the_fixed_point_sum(k, wf, prop):
+    """Every input of a neuron arrives in every step.  The sum's error is at most half a
+    fixed-point unit an input; the potential rounds once a step (2^-24 relative, 4 steps)."""
+    w = float(np.float32(1e-3 / k))
+    _say(f"case: {k} inputs arriving in every step, weight_format={wf}, propagation={prop}")
+    s = N.Simulator.generated(**_driven(k, w), weight_format=wf, propagation=prop)
+    scale = s.info()["fix_scale_exc"]
+    assert k * round(w * scale) <= 2**31 - 1
+    s.run(14)                                     # arrivals in steps 10 to 13
+    want = _v_after(k * w, 4)
+    tol = 4 * (0.5 * k / scale + 4 * 2.0**-24 * want)
+    assert np.abs(s.state(N.F_V)[700:].astype(np.float64) - want).max() <= tol
+    blob = s.checkpoint()                         # the pending inputs with the scale they have
+    s.run(3)
+    t = N.Simulator.generated(**_driven(k, w), weight_format=wf, propagation=prop)
+    t.restore(blob)
+    t.run(3)
+    assert np.array_equal(s.state(N.F_V), t.state(N.F_V))
+    s.close()
+    t.close()
+
+
+@pytest.mark.parametrize("wf", FORMATS)
+def test_sums_of_a_batch_and_of_both_signs(wf):
+    """Each network of a batch has its own scale; excitatory and inhibitory inputs of a
+    neuron have sums of their own until it reads them."""
+    _say(f"case: batch of networks of 100, 3000 and 640 + 640 inputs, weight_format={wf}")
+    nets = [_driven(100, float(np.float32(1e-5))), _driven(3000, float(np.float32(4e-7)), seed=4),
+            _driven(640, float(np.float32(3e-6)), seed=5, g=float(np.float32(-1.5e-6)))]
+    want = [_v_after(x, 4) for x in (1e-3, 1.2e-3, 0.96e-3)]
+    for prop in (N.PROP_TILED, N.PROP_DIRECT):
+        s = N.Simulator.batch_generated(nets, weight_format=wf, propagation=prop)
+        s.run(14)
+        v = s.state(N.F_V).astype(np.float64)
+        for b, x in enumerate(want):
+            # (the codes of the third network's weights: 2^-9 for BF16, 2^-4 for FP8)
+            rel = {N.WF_F32: 1e-5, N.WF_BF16: 2.0**-8, N.WF_FP8: 2.0**-3}[wf] if b == 2 else 1e-5
+            assert np.abs(v[1000 * b + 700:1000 * (b + 1)] - x).max() <= 4 * rel * x, (prop, b)
+        s.close()
+
+
+@pytest.mark.parametrize("prop,wf", [(N.PROP_TILED, N.WF_F32), (N.PROP_TILED, N.WF_BF16), (N.PROP_DIRECT, N.WF_F32)])
+def test_plastic_inputs_at_their_largest(prop, wf):
+    """Plastic weights count with the largest value that plasticity can give them."""
+    w = 1e-6
+    sc = np.array(W.stdp_consts(w), dtype=np.float32)
+    s = N.Simulator.generated(**_driven(1000, w, plastic=1), weight_format=wf, propagation=prop, stdp=True, stdpconst=sc)
+    top = max(abs(float(sc[4])), abs(float(sc[5])), w)
+    assert 1000 * round(top * s.info()["fix_scale_exc"]) <= 2**31 - 1
+    s.close()
+
+
+def test_scales_that_held_stay():
+    """Where no sum can leave int32 the scale is the one of in-degree * max |w|, for lists in
+    source order (every synapse counted) as before."""
+    rng = np.random.default_rng(2)
+    n, m = 500, 40000
+    src, tar = np.sort(rng.integers(0, n, m)), rng.integers(0, n, m)
+    w = rng.choice(np.float32([1e-5, 2e-5, -3e-5]), m)
+    s = N.Simulator.from_arrays([N.LIFB] * n, [0.0] * n, W.lifb_consts(), src, tar, w, np.full(m, np.float32(1e-3)),
+                                weight_format=N.WF_F32)
+    deg = np.bincount(tar, minlength=n).max()
+    assert s.info()["fix_scale_exc"] == 2.0**np.floor(np.log2(2147483520.0 / (deg * float(np.float32(3e-5)))))
+    s.close()
