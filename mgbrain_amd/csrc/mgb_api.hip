@@ -689,10 +689,14 @@ std::vector<int32_t> stream_runs(const HostNeurons& h, std::vector<uint16_t>& ru
 // Lowers the fixed-point scales of segments whose ring words could leave int32 until none
 // can: first by in-degree * max |w| alone, then, where that does not settle it, by each
 // target's own sums (RingSumArgs).  The weights' codes are those of the format (row scales
-// set).  A scale that is lowered joins the layout that a checkpoint has to match, its ring
+// set).  Plastic networks, where every synapse would count with the largest weight it can
+// ever have, keep the scale that holds what arrives when all sources fire in one step: the
+// whole of a neuron's inputs, of any delay, would take 2 to 4 bits more (and their results
+// with them), for sums that only sources timed to cancel the delays could reach.  A scale
+// that is lowered joins the layout that a checkpoint has to match, its ring
 // words being multiples of 1 / scale.
-mgb_status fit_scales(mgb_sim* s, const HostNeurons& h, const DevList& L, const std::vector<uint32_t>& indeg,
-                      const std::vector<float>& w_seg, const uint16_t* seg, std::vector<float2>& sc) {
+mgb_status fit_scales(mgb_sim* s, const HostNeurons& h, const DevList& L, const uint8_t* dq,
+                      const std::vector<uint32_t>& indeg, const std::vector<float>& w_seg, const uint16_t* seg, std::vector<float2>& sc) {
     const size_t n = (size_t)h.n, nseg = sc.size();
     const std::vector<int32_t>& lo = s->h_seg_lo;
     constexpr double kMax = 2147483647.0;
@@ -707,28 +711,31 @@ mgb_status fit_scales(mgb_sim* s, const HostNeurons& h, const DevList& L, const 
     RingSumArgs a{};
     float* scale = nullptr;
     MGB_TRY(X.get(&scale, nseg));
-    MGB_TRY(X.get(&a.sums, 2 * n));
+    a.D = s->n_plastic > 0 && n * (size_t)s->D < (size_t(1) << 27) ? s->D : 0;
+    const size_t rows = 2 * (size_t)std::max(a.D, 1);
+    MGB_TRY(X.get(&a.sums, rows * n));
     a.S = L.S; a.n = h.n;
-    a.src = L.src; a.tar = L.tar; a.weight = L.weight;
+    a.src = L.src; a.tar = L.tar; a.weight = L.weight; a.dq = dq;
     a.plastic = h.stdp ? L.plastic : nullptr;
-    a.w_plastic = h.stdp ? std::max(std::fabs(h.stdpconst[4]), std::fabs(h.stdpconst[5])) : 0.f;
+    a.w_top = h.stdpconst[4]; a.w_low = h.stdpconst[5];
     a.bits = s->wide_kind == kWideBF16 ? 16 : (s->wide_kind == kWideFP8 ? 8 : 32);
     a.row_scale = s->row_scale;
     a.seg = seg;
     a.scale = scale;
-    std::vector<unsigned long long> sums(2 * n);
+    std::vector<unsigned long long> sums(rows * n);
     std::vector<float> now(nseg);
     for (int pass = 0; pass < 8; ++pass) {
         for (size_t q = 0; q < nseg; ++q) now[q] = sc[q].x;
         MGB_HIP_TRY(hipMemcpyAsync(scale, now.data(), 4 * nseg, hipMemcpyHostToDevice, s->stream));
-        MGB_HIP_TRY(hipMemsetAsync(a.sums, 0, 16 * n, s->stream));
+        MGB_HIP_TRY(hipMemsetAsync(a.sums, 0, 8 * rows * n, s->stream));
         MGB_HIP_TRY(ring_sums(a, s->stream));
-        MGB_HIP_TRY(hipMemcpyAsync(sums.data(), a.sums, 16 * n, hipMemcpyDeviceToHost, s->stream));
+        MGB_HIP_TRY(hipMemcpyAsync(sums.data(), a.sums, 8 * rows * n, hipMemcpyDeviceToHost, s->stream));
         MGB_HIP_TRY(hipStreamSynchronize(s->stream));
         bool fits = true;
         for (size_t q = 0; q < nseg; ++q) {
             unsigned long long m = 0;
-            for (int32_t t = lo[q]; t < lo[q + 1]; ++t) m = std::max({m, sums[t], sums[n + t]});
+            for (size_t r = 0; r < rows; ++r)
+                for (int32_t t = lo[q]; t < lo[q + 1]; ++t) m = std::max(m, sums[r * n + t]);
             if ((double)m <= kMax || sc[q].x <= 0x1p-100f) continue;
             const int by = std::max(1, (int)std::ceil(std::log2((double)m / kMax)));
             const int e = std::max(-100, std::ilogb(sc[q].x) - by);
@@ -1011,7 +1018,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
                                        s->row_scale, st));
             }
         }
-        MGB_TRY(fit_scales(s, h, L, h_indeg, w_seg, nseg > 1 ? seg_dev : nullptr, seg_sc));
+        MGB_TRY(fit_scales(s, h, L, dq, h_indeg, w_seg, nseg > 1 ? seg_dev : nullptr, seg_sc));
         s->scale_e = s->scale_i = seg_sc[0].x;
         if (nseg > 1) {
             MGB_TRY(dalloc_n(s, &s->seg_scale, nseg));

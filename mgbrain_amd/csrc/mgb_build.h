@@ -67,7 +67,8 @@ struct GatherArgs {
 
 // The largest value a ring word can hold: per target and sign, the sum of its synapses'
 // fixed-point inputs (each arrives at most once in a step), a plastic one with the largest
-// weight it can have, of either sign.
+// weight of that sign that it can have.  With D, a sum for each delay: what arrives at once
+// when every source fires in one step.
 struct RingSumArgs {
     uint64_t S;
     int32_t n;
@@ -75,12 +76,14 @@ struct RingSumArgs {
     const int32_t* tar;
     const float* weight;
     const uint8_t* plastic;     // NULL: none
-    float w_plastic;            // largest |w| a plastic synapse can reach
+    const uint8_t* dq;          // delays in steps, below D
+    int32_t D;                  // 0: all delays in one sum
+    float w_top, w_low;         // a plastic weight's bounds
     int bits;                   // 32, or the 16 / 8 of a BF16 / FP8 code times row_scale
     const float* row_scale;
     const uint16_t* seg;        // [n] segment of each target (NULL: one)
     const float* scale;         // [segments] fixed-point scale
-    unsigned long long* sums;   // [2][n], zeroed
+    unsigned long long* sums;   // [max(D, 1)][2][n], zeroed
 };
 
 struct GenProjArgs {

@@ -438,35 +438,40 @@ __global__ void k_gather_wide(GatherArgs a) {
     }
 }
 
-// (a wave of one target and sign, as in target-major lists, adds once)
+// (a wave of one target and delay, as in target-major lists, adds once)
 __global__ void k_ring_sums(RingSumArgs a) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     const uint64_t iters = (a.S + stride - 1) / stride;
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (uint64_t it = 0; it < iters; ++it, i += stride) {
-        uint32_t key = 0xFFFFFFFFu;
-        unsigned long long v = 0ull;
+        uint32_t key = 0xFFFFFFFFu, d = 0u;
+        unsigned long long v[2] = {0ull, 0ull};              // excitatory, inhibitory
         if (i < a.S) {
             const int32_t t = a.tar[i];
             float w = a.weight[i];
+            if (a.D) d = a.dq[i];
             const bool pl = a.plastic && a.plastic[i];
             if (!pl && a.bits != 32) {
                 const float rs = a.row_scale[a.src[i]];
                 w = (a.bits == 16 ? __uint_as_float((uint32_t)f32_to_bf16_rne(w / rs) << 16)
                                   : fp8_value(f32_to_fp8e4m3(w / rs))) * rs;
             }
-            const float q = rintf((pl ? fmaxf(fabsf(w), a.w_plastic) : fabsf(w)) * a.scale[a.seg ? a.seg[t] : 0]);
-            v = q < 0x1p31f ? (unsigned long long)q : (q == q ? 1ull << 31 : 0ull);
-            key = ((uint32_t)t << 2) | (pl ? 2u : (w > 0.f ? 0u : 1u));
-        }
-        const bool all = wave_all_equal(key);
-        if (all)
+            const float sc = a.scale[a.seg ? a.seg[t] : 0];
+            const float hi = pl ? fmaxf(w, fmaxf(a.w_top, a.w_low)) : w, lo = pl ? fminf(w, fminf(a.w_top, a.w_low)) : w;
+            const float q[2] = {rintf(hi * sc), rintf(-lo * sc)};
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) v += (unsigned long long)__shfl_xor((long long)v, o);
-        if (key != 0xFFFFFFFFu && v && (!all || (threadIdx.x & 63u) == 0u)) {
-            const size_t t = key >> 2;
-            if ((key & 1u) == 0u) atomicAdd(&a.sums[t], v);
-            if ((key & 3u) != 0u) atomicAdd(&a.sums[(size_t)a.n + t], v);
+            for (int e = 0; e < 2; ++e)                      // (not a number: 0)
+                if (q[e] > 0.f) v[e] = q[e] < 0x1p31f ? (unsigned long long)q[e] : 1ull << 31;
+            key = (uint32_t)t;
+        }
+        const bool all = wave_all_equal(key) && wave_all_equal(d);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            if (all)
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) v[e] += (unsigned long long)__shfl_xor((long long)v[e], o);
+            if (key != 0xFFFFFFFFu && v[e] && (!all || (threadIdx.x & 63u) == 0u))
+                atomicAdd(&a.sums[((size_t)d * 2u + (size_t)e) * (size_t)a.n + key], v[e]);
         }
     }
 }

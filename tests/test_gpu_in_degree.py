@@ -165,3 +165,19 @@ def test_scales_that_held_stay():
     deg = np.bincount(tar, minlength=n).max()
     assert s.info()["fix_scale_exc"] == 2.0**np.floor(np.log2(2147483520.0 / (deg * float(np.float32(3e-5)))))
     s.close()
+
+
+@pytest.mark.parametrize("wf", [N.WF_F32, N.WF_BF16])
+def test_a_volley_of_plastic_inputs(wf):
+    """All inputs plastic, delays of 1 to 2 ms in 11 steps: what arrives at once when every
+    source fires in one step fits, at the largest weights, for every target and delay."""
+    w, k, n = 1e-6, 640, 300
+    net = _driven(k, w, n=n, plastic=1)
+    net["projs"][0]["dmax"] = 2e-3
+    sc = np.array(W.stdp_consts(w), dtype=np.float32)
+    s = N.Simulator.generated(**net, weight_format=wf, propagation=N.PROP_TILED, stdp=True, stdpconst=sc)
+    _, col, dl, _ = s.csr()
+    most = np.bincount((col.astype(np.int64) - 700) * 32 + dl, minlength=32 * n).max()
+    assert 60 < most < 150
+    assert most * round(float(sc[4]) * s.info()["fix_scale_exc"]) <= 2**31 - 1
+    s.close()
