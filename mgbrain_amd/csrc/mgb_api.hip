@@ -106,7 +106,6 @@ struct mgb_sim {
     uint64_t* seg_obase = nullptr;     // [nseg+1]
     uint64_t n_offs = 0, n_keys = 0;
     uint32_t* tcnt = nullptr;          // [3][nseg]
-    int64_t* tbase = nullptr;          // [3][nseg] (one segment: the control block's words)
     int tkind = kTClass16;             // synapse word kind of the fused kernel
     uint32_t* tperm = nullptr;         // fused STDP: CSR slot of each tile-order position (~0u: padding)
     uint64_t n_tslots = 0;             // length of the (padded) tile-order arrays
@@ -1234,12 +1233,6 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
     if (s->tiled) {
         MGB_TRY(dalloc_n(s, &s->tcnt, 3 * (size_t)s->nseg));
         MGB_HIP_TRY(hipMemsetAsync(s->tcnt, 0, 12 * (size_t)s->nseg, st));
-        if (s->nseg == 1) {
-            s->tbase = reinterpret_cast<int64_t*>(reinterpret_cast<uint8_t*>(s->ctl) + offsetof(Ctl, tbase));
-        } else {
-            MGB_TRY(dalloc_n(s, &s->tbase, 3 * (size_t)s->nseg));
-            MGB_HIP_TRY(hipMemsetAsync(s->tbase, 0, 24 * (size_t)s->nseg, st));
-        }
     }
     // record
     s->rec_cap = o ? std::max<int64_t>(o->record_capacity, 0) : 0;
@@ -1426,7 +1419,6 @@ TiledArgs tiled_args(const mgb_sim* s) {
     a.nseg = s->nseg; a.window = s->window;
     a.tile_lo = s->tile_lo; a.tile_seg = s->tile_seg; a.seg_lo = s->seg_lo;
     a.seg_tile0 = s->seg_tile0; a.seg_obase = s->seg_obase; a.tcnt = s->tcnt;
-    a.tbase = s->tbase;
     a.type = s->type; a.cset = s->cset; a.tbl = s->tbl; a.stream = s->stream_idx;
     a.rate = s->rate; a.V = s->V; a.Ie = s->Ie; a.Ii = s->Ii;
     a.refr = s->refr; a.last = s->last; a.cnt = s->cnt;
@@ -1508,6 +1500,7 @@ mgb_status issue_windows(mgb_sim* s, int32_t nsteps, bool finalize, bool capturi
     if (s->tiled) {
         const TiledArgs ta = tiled_args(s);
         const int32_t nfull = nsteps / s->window;
+        int32_t prev = 0;                      // steps of the window before
         if (s->persist && nfull >= 2) {
             // the run's whole windows in one launch
             SpanGuard g1{s, kSpanProp, prof, nfull};
@@ -1517,11 +1510,13 @@ mgb_status issue_windows(mgb_sim* s, int32_t nsteps, bool finalize, bool capturi
             s->launches += 2;
             off = nfull * s->window;
             wk = nfull;
+            prev = s->window;
         }
         while (off < nsteps) {
             const int32_t nst = std::min(s->window, nsteps - off);
             // fused STDP: the flush kernel after every second window and after the last
             TiledArgs tw = ta;
+            tw.prev_len = prev;
             tw.flush_next = stdp_kind(s->tkind) && ((wk & 1) != 0 || off + nst >= nsteps) ? 1 : 0;
             SpanGuard g1{s, kSpanProp, prof};
             MGB_TRY(g1.begin());
@@ -1537,10 +1532,11 @@ mgb_status issue_windows(mgb_sim* s, int32_t nsteps, bool finalize, bool capturi
             }
             off += nst;
             ++wk;
+            prev = nst;
         }
         if (finalize) {
-            MGB_HIP_TRY(launch_finalize_tiled(s->ctl, nsteps, wk, s->persist ? s->bar_err : nullptr, s->mir_dev,
-                                              s->stream));
+            MGB_HIP_TRY(launch_finalize_tiled(s->ctl, nsteps, wk, prev, s->persist ? s->bar_err : nullptr,
+                                              s->mir_dev, s->stream));
             s->launches += 1;
         }
         return MGB_OK;
@@ -2442,12 +2438,6 @@ mgb_status mgb_checkpoint_load(mgb_sim* s, const void* buf, int64_t bytes) {
         off += g.bytes;
     }
     MGB_HIP_TRY(hipMemcpy(&s->mir->ctl, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
-    if (s->tiled && s->nseg > 1) {
-        // the lists' start steps, the same in every segment between runs
-        std::vector<int64_t> tb(3 * (size_t)s->nseg);
-        for (int b = 0; b < 3; ++b) std::fill_n(tb.begin() + (size_t)b * s->nseg, s->nseg, s->mir->ctl.tbase[b]);
-        MGB_HIP_TRY(hipMemcpy(s->tbase, tb.data(), 8 * tb.size(), hipMemcpyHostToDevice));
-    }
     // the persistent waits' flags hold window indices of the run before (epochs)
     if (s->bar) MGB_HIP_TRY(hipMemset(s->bar, 0, 4 * (size_t)s->G * kBarStride));
     return MGB_OK;

@@ -50,9 +50,9 @@ struct Ctl {
     uint64_t rec_cnt;       // spikes recorded (may exceed capacity)
     uint64_t se;            // synaptic events
     // fused tiled path: three spike lists (write k%3, read (k-1)%3, clear (k+1)%3);
-    // their per-segment counters and start steps live in TiledArgs::tcnt and tbase
-    int64_t tbase[3];       // first step of the window that wrote each list (segment 0's, for
-                            // checkpoints: between runs all segments' are the same)
+    // their per-segment counters live in TiledArgs::tcnt
+    int64_t tbase[3];       // first step of the window that wrote the list of a run's last
+                            // window (mgb_lists.h)
 };
 
 
@@ -190,7 +190,6 @@ struct TiledArgs {
     const int32_t* seg_tile0;   // [nseg+1] first tile of each segment
     const uint64_t* seg_obase;  // [nseg+1] first offset entry of each segment
     uint32_t* tcnt;             // [3][nseg] entries in each segment's spike lists
-    int64_t* tbase;             // [3][nseg] first step of the window that wrote each (mgb_lists.h)
     const uint8_t* type;
     const uint8_t* cset;
     const uint16_t* tbl;
@@ -222,6 +221,7 @@ struct TiledArgs {
     Ctl* ctl;
     uint32_t* win_buf;
     uint32_t win_stride;
+    int32_t prev_len;       // steps of the window before the launch (0: the run's first launch)
     uint64_t* rec;
     uint64_t rec_cap;
     // kTStdp / kTStdpB.  Window k reads its neurons' last spike steps from last3 buffer
@@ -340,9 +340,9 @@ hipError_t set_tiled_pw_lds_limit(const TiledArgs& a);
 // window index goes back (a restored checkpoint).
 hipError_t launch_tiled_persistent(const TiledArgs& a, int32_t off, int32_t wk, int32_t nsteps, int32_t nwin,
                                    int block, hipStream_t st);
-// err: the persistent waits' error word (or null)
-hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, HostMirror* m,
-                                 hipStream_t st);
+// last: steps of the last window; err: the persistent waits' error word (or null)
+hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, int32_t last, const uint32_t* err,
+                                 HostMirror* m, hipStream_t st);
 hipError_t set_tiled_lds_limit(int kind, size_t bytes);
 // kTStdp: brings the plastic in-synapses of the neurons the fused kernel listed
 // in window base_window + wk up to date (flush of deferred dendrite updates).

@@ -613,8 +613,8 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
 // `epoch` in its flag, words kBarStride apart per tile (a cache line each), even epochs in
 // one and odd ones in another, and waits until the flag of this parity of every
 // workgroup of its segment (tiles [ct0, ct1)) holds `epoch`, one flag per thread.
-// Workgroups of other segments share no list and no list's start step (mgb_lists.h) with it
-// and may be any number of windows ahead or behind.  One of its own segment can be one window ahead -- its tile may have
+// Workgroups of other segments share no list with it, write no word that it reads
+// (mgb_lists.h) and may be any number of windows ahead or behind.  One of its own segment can be one window ahead -- its tile may have
 // little to do -- and have published epoch + 1 before this one reads its flag (two ahead
 // it cannot be): with one word for both parities, what else the flag holds
 // (grid_exchange) would be the next window's.  A poll is one load, back to back with the
@@ -1101,7 +1101,7 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
         uint32_t E, ent0;
         if (kw == 0) {
             const size_t ws = a.win_stride;
-            sprev = list_start(a.tbase, q, nseg, bprev);
+            sprev = window_before(ctl->tbase, bprev, s0, a.prev_len);
             const uint32_t n0 = tcnt[0], n1 = tcnt[nseg], n2 = tcnt[2 * nseg];
             const uint32_t l0 = a.win_buf[lbase + li], l1 = a.win_buf[ws + lbase + li];
             const uint32_t l2 = a.win_buf[2 * ws + lbase + li];
@@ -1141,10 +1141,6 @@ __global__ __launch_bounds__(1024) void k_tiled(TiledArgs a, int32_t off, int32_
             else tcnt[bnext * nseg] = 0u;
         }
         if (kPl && full && g == 0 && tid == 0) a.fcnt[(kwin + 1) & 1] = 0u;
-        if (full && lt == 0 && tid == 0) {
-            set_list_start(a.tbase, q, nseg, bcur, s0);
-            if (g == 0) ctl->tbase[bcur] = s0;          // (for checkpoints)
-        }
         if (tid == 0) {
             sh->se = 0ull;
             sh->n = 0u;
@@ -1918,8 +1914,10 @@ __global__ __launch_bounds__(256) void k_stdp_flush(TiledArgs a, int32_t off, in
 
 // End of a run: the step and window counters move on, and the control block and the
 // persistent waits' error word go to the host (pinned memory the host reads after the run).
-__global__ void k_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, HostMirror* m) {
+__global__ void k_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, int32_t last, const uint32_t* err,
+                                 HostMirror* m) {
     if (threadIdx.x == 0) {
+        end_run(ctl->tbase, ctl->base_step, ctl->base_window, steps, windows, last);
         ctl->base_step += steps;
         ctl->base_window += windows;
         if (err) __hip_atomic_store(&m->err, *err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -2131,9 +2129,10 @@ hipError_t launch_stdp_flush(const TiledArgs& a, int32_t off, int32_t wk, hipStr
     return hipGetLastError();
 }
 
-hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, const uint32_t* err, HostMirror* m,
-                                 hipStream_t st) {
-    hipLaunchKernelGGL(k_finalize_tiled, dim3(1), dim3(64), 0, st, ctl, steps, windows, err, m);
+hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, int32_t last, const uint32_t* err,
+                                 HostMirror* m, hipStream_t st) {
+    if (windows < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_finalize_tiled, dim3(1), dim3(64), 0, st, ctl, steps, windows, last, err, m);
     return hipGetLastError();
 }
 

@@ -1,14 +1,12 @@
-// mgb_lists.h -- start steps of the fused path's spike lists, shared by the kernels, the
-// host and a CPU model of a launch.
+// mgb_lists.h -- which window wrote a spike list of the fused path, shared by the kernels
+// and a CPU model of a run's launches.
 //
-// A window's propagation needs the first step of the window before it, whose list it
-// reads.  Inside a persistent launch that is the launch's own window length; in a launch's
-// first window it is the word that the previous launch left.  The words are [3][nseg], one
-// per list and segment: a segment's workgroups wait only for each other between windows, so
-// another segment can be any number of windows ahead while one of this segment has yet to
-// start, and would have written over a word they shared (window k + 2 goes to the list of
-// window k - 1).  In its own segment no workgroup is more than one window ahead of the
-// last, and window k + 1 writes neither list k nor list k - 1.
+// A window's propagation needs the first step of the window before it, whose list it reads:
+// the window's own length inside a persistent launch, the length that the host gives with
+// each later launch of a run, and in a run's first launch a word (one per list) that the
+// run before left.  Only the end of a run writes these words.  No launch does: a segment's
+// workgroups wait only for each other between windows, so that another segment can be any
+// number of windows ahead while one of this segment has yet to read them.
 #pragma once
 #include <stdint.h>
 
@@ -16,16 +14,20 @@
 
 namespace mgb {
 
-// First step of the window that wrote list b (0, 1, 2) of segment q.  All three words load,
+// First step of the window before the one that starts at s0, whose list is b (0, 1, 2), in
+// the first window of a launch: prev_len steps earlier, or (0) by the words.  All three load,
 // then b picks one: b comes from a load of its own.
-MGB_HD int64_t list_start(const int64_t* tbase, int32_t q, int32_t nseg, int b) {
-    const int64_t s0 = tbase[q], s1 = tbase[nseg + q], s2 = tbase[2 * nseg + q];
-    return b == 0 ? s0 : (b == 1 ? s1 : s2);
+MGB_HD int64_t window_before(const int64_t* tbase, int b, int64_t s0, int32_t prev_len) {
+    if (prev_len) return s0 - prev_len;
+    const int64_t t0 = tbase[0], t1 = tbase[1], t2 = tbase[2];
+    return b == 0 ? t0 : (b == 1 ? t1 : t2);
 }
 
-// (by one workgroup of segment q)
-MGB_HD void set_list_start(int64_t* tbase, int32_t q, int32_t nseg, int b, int64_t step) {
-    tbase[b * nseg + q] = step;
+// End of a run of `steps` steps in `windows` windows (at least one) from base_step and
+// base_window on, whose last window had `last` steps.
+MGB_HD void end_run(int64_t* tbase, int64_t base_step, int64_t base_window, int32_t steps, int32_t windows,
+                    int32_t last) {
+    tbase[(base_window + windows - 1) % 3] = base_step + steps - last;
 }
 
 }  // namespace mgb
