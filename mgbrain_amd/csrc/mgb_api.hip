@@ -139,7 +139,7 @@ struct mgb_sim {
     HostMirror* mir_dev = nullptr;     // its address on the device (the run's last kernel writes it)
     bool err_pending = false;          // mir->err is due with the stream's completion
     // read-back of large arrays: two pinned buffers (kStageBytes each, copy_out) and the
-    // device workspace that sorts spike records, kept from the first such call on
+    // device workspace that sorts spike records (read_records_sorted)
     uint8_t* stage[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     bool stage_on = false, stage_off = false;   // they are there; they could not be had
@@ -2197,6 +2197,18 @@ mgb_status copy_out(mgb_sim* s, void* dst, const void* src, size_t bytes) {
 
 // Spike records from this many on are sorted on the device.
 constexpr uint64_t kDeviceSortMin = 2048;
+// A sort's workspace (about 24 bytes a record) up to this size is kept for the next read, a
+// larger one given back: a second of 110,000 neurons at 28 Hz takes 95 MB, and its two
+// allocations would be a few tenths of a millisecond of 52.
+constexpr size_t kSortKeep = size_t(256) << 20;
+
+void free_sort_space(mgb_sim* s) {
+    if (!s->rd_ws) return;
+    dfree(s, s->rd_ws);
+    s->bytes -= (int64_t)s->rd_ws_bytes;
+    s->rd_ws = nullptr;
+    s->rd_ws_bytes = 0;
+}
 
 // The first w of the `have` records in order of (step, id): radix-sorted on the device by
 // the id's bits, then the step's (the record itself stays as it is), and split into the
@@ -2211,13 +2223,8 @@ mgb_status read_records_sorted(mgb_sim* s, uint64_t have, uint64_t w, int32_t* s
     const size_t keys = (8 * (size_t)have + 255) & ~(size_t)255, temp = std::max(t1, t2);
     const size_t need = 2 * keys + temp;
     if (need > s->rd_ws_bytes) {
-        if (s->rd_ws) {
-            dfree(s, s->rd_ws);
-            s->bytes -= (int64_t)s->rd_ws_bytes;
-            s->rd_ws = nullptr;
-            s->rd_ws_bytes = 0;
-        }
-        const size_t room = need + need / 4;
+        free_sort_space(s);
+        const size_t room = (need + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
         if (dalloc_n(s, &s->rd_ws, room) != MGB_OK) {
             (void)hipGetLastError();
             return MGB_OK;
@@ -2234,6 +2241,7 @@ mgb_status read_records_sorted(mgb_sim* s, uint64_t have, uint64_t w, int32_t* s
     MGB_HIP_TRY(hipStreamSynchronize(s->stream));
     MGB_TRY(copy_out(s, steps, col, 4 * w));
     MGB_TRY(copy_out(s, ids, col + w, 4 * w));
+    if (s->rd_ws_bytes > kSortKeep) free_sort_space(s);
     *done = true;
     return MGB_OK;
 }

@@ -67,3 +67,24 @@ def test_weights_across_the_pinned_buffers(wf, extra):
     for _ in range(2):
         assert np.array_equal(g.weights(), want)
     g.close()
+
+
+def test_a_large_read_gives_its_workspace_back():
+    """Records are sorted in device memory: up to 256 MiB of it is kept for the next read."""
+    print("case: 20000 Poisson neurons at 0.05 a step, reads of 0.1, 12 and 0.1 million records", flush=True)
+    g = N.Simulator.generated([dict(num=20000, type=N.POISSON, rate=0.05)], [], M.config1().lifconst, seed=1,
+                              record_capacity=12_500_000)
+    at = [g.info()["device_bytes"]]
+    for n in (100, 11900, 0):
+        if n:
+            g.run(n)
+        else:
+            g.clear_spikes()
+            g.run(100)
+        steps, ids = g.spikes()
+        key = steps.astype(np.int64) << 32 | ids
+        assert np.all(key[1:] > key[:-1]) and len(ids) == g.info()["spikes_recorded"]
+        at.append(g.info()["device_bytes"])
+    print(at, flush=True)
+    assert at[0] <= at[1] <= at[0] + (8 << 20) and at[2] == at[0] and at[3] == at[1]
+    g.close()
