@@ -113,7 +113,7 @@ struct mgb_sim {
     uint16_t* seg_of = nullptr;        // segment of each neuron (with seg_scale)
     int32_t *hist = nullptr, *tf = nullptr, *cntf = nullptr;   // fused STDP: deferred dendrite updates
     int32_t* flist = nullptr;          // fused STDP: [2][npad][2] neurons to flush
-    uint32_t* fcnt = nullptr;          // [2]
+    uint32_t* fcnt = nullptr;          // [2], and their copy while weights are read
     int32_t stdp_isi = 1;              // fused STDP: shortest inter-spike interval of plastic synapses' ends
     uint32_t* syn_t = nullptr;
     uint16_t* syn16 = nullptr;         // kTClass16 words in tile order (padded sub-rows)
@@ -1186,7 +1186,7 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
         MGB_HIP_TRY(hipMemsetAsync(s->tf, 0xFF, 4 * np, st));     // -1: no update deferred yet
         MGB_HIP_TRY(hipMemsetAsync(s->cntf, 0, 4 * np, st));
         MGB_TRY(dalloc_n(s, &s->flist, 2 * 2 * np));
-        MGB_TRY(dalloc_n(s, &s->fcnt, 2));
+        MGB_TRY(dalloc_n(s, &s->fcnt, 4));
         MGB_HIP_TRY(hipMemsetAsync(s->fcnt, 0, 8, st));
     }
     MGB_HIP_TRY(hipMemsetAsync(s->cnt, 0, 4 * np, st));
@@ -2497,10 +2497,11 @@ hipError_t current_weights_into(mgb_sim* s, float* tmp) {
     ta.w_t = tmp;
     ta.apply_only = 1;
     hipError_t e = hipMemcpyAsync(tmp, s->w_t, S * 4, hipMemcpyDeviceToDevice, s->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(s->fcnt + 2, s->fcnt, 8, hipMemcpyDeviceToDevice, s->stream);
     if (e == hipSuccess) e = launch_tiled(ta, 0, 0, 1, s->tblock, s->stream);
     if (e == hipSuccess) e = launch_stdp_flush(ta, 0, 0, s->stream);
-    // the list this used is empty before the next window appends to it
-    if (e == hipSuccess) e = hipMemsetAsync(s->fcnt, 0, 8, s->stream);
+    // the list this used is as it was before the next window appends to it
+    if (e == hipSuccess) e = hipMemcpyAsync(s->fcnt, s->fcnt + 2, 8, hipMemcpyDeviceToDevice, s->stream);
     if (e == hipSuccess) e = scatter_weights(s->tperm, tmp, (uint64_t)S, s->w32, s->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
     return e;
@@ -2550,6 +2551,46 @@ mgb_status scratch_on(int device, float** out) {
 
 }  // namespace
 
+namespace {
+
+// BF16 / FP8: the weights as the kernels decode them, a part at a time in device memory of
+// the call's own (what the simulator stores stays as it is: with STDP on the direct path
+// the FP32 words are part of a checkpoint).
+mgb_status read_decoded(mgb_sim* s, float* weight) {
+    const size_t S = (size_t)s->S;
+    size_t part = std::min(S, size_t(1) << 24);
+    float* dec = nullptr;
+    hipError_t e = hipMalloc(&dec, 4 * part);
+    if (e != hipSuccess && part > (size_t(1) << 20)) {
+        (void)hipGetLastError();
+        part = size_t(1) << 20;
+        e = hipMalloc(&dec, 4 * part);
+    }
+    if (e != hipSuccess) {
+        set_error("hipMalloc(%zu) for the weight read-back failed: %s", 4 * part, hipGetErrorString(e));
+        return e == hipErrorOutOfMemory ? MGB_ERR_OOM : MGB_ERR_HIP;
+    }
+    mgb_status st = MGB_OK;
+    for (size_t k = 0; k < S && st == MGB_OK; k += part) {
+        const size_t len = std::min(part, S - k);
+        e = wide_weights(s->row_ptr, s->n, s->dly, s->w32, s->wide_kind == kWideBF16 ? s->w16 : nullptr,
+                         s->wide_kind == kWideFP8 ? s->w8 : nullptr, s->row_scale, (int64_t)k, (int64_t)(k + len), dec,
+                         s->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
+        if (e != hipSuccess) {
+            set_error("weight read-back: %s", hipGetErrorString(e));
+            st = MGB_ERR_HIP;
+        } else {
+            st = copy_out(s, weight + k, dec, 4 * len);
+        }
+    }
+    (void)hipStreamSynchronize(s->stream);
+    (void)hipFree(dec);
+    return st;
+}
+
+}  // namespace
+
 mgb_status mgb_read_csr(mgb_sim* s, int64_t* row_ptr, int32_t* col, int32_t* delay, float* weight) {
     if (!s) {
         set_error("null handle");
@@ -2580,13 +2621,8 @@ mgb_status mgb_read_csr(mgb_sim* s, int64_t* row_ptr, int32_t* col, int32_t* del
     }
     if (weight && S) {
         if (s->tiled && stdp_kind(s->tkind)) MGB_TRY(current_weights(s));
-        // BF16 / FP8: decoded on the device in place (the FP32 copy of a static synapse is
-        // read by nothing else)
-        if (s->wide_kind != kWideF32)
-            MGB_HIP_TRY(wide_weights(s->row_ptr, s->n, s->dly, s->w32, s->wide_kind == kWideBF16 ? s->w16 : nullptr,
-                                     s->wide_kind == kWideFP8 ? s->w8 : nullptr, s->row_scale, s->w32, s->stream));
-        MGB_HIP_TRY(hipStreamSynchronize(s->stream));
-        MGB_TRY(copy_out(s, weight, s->w32, 4 * S));
+        if (s->wide_kind == kWideF32) MGB_TRY(copy_out(s, weight, s->w32, 4 * S));
+        else MGB_TRY(read_decoded(s, weight));
     }
     return MGB_OK;
 }
@@ -2632,7 +2668,8 @@ mgb_status mgb_read_weights_noalloc(mgb_sim* s, float* out) {
         from = scr;
     } else if (decode) {
         MGB_HIP_TRY(wide_weights(s->row_ptr, s->n, s->dly, s->w32, s->wide_kind == kWideBF16 ? s->w16 : nullptr,
-                                 s->wide_kind == kWideFP8 ? s->w8 : nullptr, s->row_scale, scr, s->stream));
+                                 s->wide_kind == kWideFP8 ? s->w8 : nullptr, s->row_scale, 0, (int64_t)S, scr,
+                                 s->stream));
         from = scr;
     }
     MGB_HIP_TRY(hipMemcpyAsync(out, from, 4 * S, hipMemcpyDeviceToHost, s->stream));

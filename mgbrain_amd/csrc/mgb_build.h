@@ -134,8 +134,8 @@ hipError_t tile_plastic(const int32_t* tile_lo, int32_t G, const int64_t* in_ptr
 hipError_t class_weights(const uint32_t* syn, const uint16_t* tbl, const float* tbl_w, uint64_t S, float* out,
                          hipStream_t st);
 hipError_t wide_weights(const int64_t* row_ptr, int32_t n, const uint8_t* dly, const float* w32,
-                        const uint16_t* w16, const uint8_t* w8, const float* row_scale, float* out,
-                        hipStream_t st);
+                        const uint16_t* w16, const uint8_t* w8, const float* row_scale, int64_t k0, int64_t k1,
+                        float* out, hipStream_t st);
 hipError_t plastic_isi(const int64_t* in_ptr, const int32_t* in_src, const int32_t* isi, int32_t n, uint64_t np,
                        int32_t* out, hipStream_t st);
 hipError_t tile_offsets(const uint32_t* sorted_keys, const int64_t* row_ptr, const TileTabs& tt,

@@ -290,20 +290,29 @@ __device__ __forceinline__ float fp8_value(uint8_t b) {
 }
 
 // BF16 / FP8 formats: the weight of every CSR slot (plastic slots: their FP32
-// weight; others: the stored code times the source row's scale).  One wave per
-// source row.
+// weight; others: the stored code times the source row's scale), slots [k0, k1) to out[0..].
+// One wave per source row.
 __global__ void k_wide_weights(const int64_t* row_ptr, int32_t n, const uint8_t* dly, const float* w32,
-                               const uint16_t* w16, const uint8_t* w8, const float* row_scale, float* out) {
+                               const uint16_t* w16, const uint8_t* w8, const float* row_scale, int64_t k0, int64_t k1,
+                               float* out) {
     const int32_t lane = (int32_t)(threadIdx.x & 63u);
     const int32_t waves = (int32_t)(gridDim.x * (blockDim.x >> 6));
-    for (int32_t i = (int32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6); i < n; i += waves) {
+    int32_t first = 0, hi = n - 1;             // the last row that starts at k0 or before
+    while (first < hi) {
+        const int32_t mid = first + (hi - first + 1) / 2;
+        if (row_ptr[mid] <= k0) first = mid;
+        else hi = mid - 1;
+    }
+    for (int64_t i = first + (int64_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6); i < n; i += waves) {
+        const int64_t beg = row_ptr[i] > k0 ? row_ptr[i] : k0, end = row_ptr[i + 1] < k1 ? row_ptr[i + 1] : k1;
+        if (row_ptr[i] >= k1) break;
         const float rs = row_scale[i];
-        for (int64_t k = row_ptr[i] + lane; k < row_ptr[i + 1]; k += 64) {
+        for (int64_t k = beg + lane; k < end; k += 64) {
             float v;
             if (dly[k] & 128u) v = w32[k];
             else if (w16) v = __uint_as_float((uint32_t)w16[k] << 16) * rs;
             else v = fp8_value(w8[k]) * rs;
-            out[k] = v;
+            out[k - k0] = v;
         }
     }
 }
@@ -671,11 +680,11 @@ hipError_t class_weights(const uint32_t* syn, const uint16_t* tbl, const float* 
 }
 
 hipError_t wide_weights(const int64_t* row_ptr, int32_t n, const uint8_t* dly, const float* w32,
-                        const uint16_t* w16, const uint8_t* w8, const float* row_scale, float* out,
-                        hipStream_t st) {
-    if (n <= 0) return hipSuccess;
+                        const uint16_t* w16, const uint8_t* w8, const float* row_scale, int64_t k0, int64_t k1,
+                        float* out, hipStream_t st) {
+    if (n <= 0 || k1 <= k0) return hipSuccess;
     hipLaunchKernelGGL(k_wide_weights, dim3(blocks_for((uint64_t)n * 64u, 256)), dim3(256), 0, st, row_ptr, n,
-                       dly, w32, w16, w8, row_scale, out);
+                       dly, w32, w16, w8, row_scale, k0, k1, out);
     return hipGetLastError();
 }
 

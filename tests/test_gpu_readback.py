@@ -88,3 +88,47 @@ def test_a_large_read_gives_its_workspace_back():
     print(at, flush=True)
     assert at[0] <= at[1] <= at[0] + (8 << 20) and at[2] == at[0] and at[3] == at[1]
     g.close()
+
+
+@pytest.mark.parametrize("prop,wf", [(N.PROP_DIRECT, N.WF_BF16), (N.PROP_DIRECT, N.WF_FP8), (N.PROP_DIRECT, N.WF_F32),
+                                     (N.PROP_TILED, N.WF_BF16)])
+def test_reading_weights_changes_nothing(prop, wf):
+    """With STDP a checkpoint is the same bytes before and after a read, as are the run's next
+    steps."""
+    print(f"case: E->E STDP, propagation={prop}, weight_format={wf}: checkpoint, weights, checkpoint", flush=True)
+    net = M.config2(scale=0.02, K=200, poisson_rate=0.3, stdp=True)
+    syn = H.host_synapses(net, seed=6)
+    # weights that neither BF16 nor FP8 holds exactly
+    syn.weight = (syn.weight * (1.0 + 0.01 * (np.arange(syn.n) % 7))).astype(np.float32)
+    g = H.gpu_from_list(net, syn, seed=6, stdp=True, stdpconst=M.stdp_consts_config4(J=1e-4), weight_format=wf,
+                        propagation=prop)
+    g.run(203)
+    before = g.checkpoint()
+    w = g.weights()
+    assert bytes(before) == bytes(g.checkpoint())
+    assert np.array_equal(w, g.weights()) and np.array_equal(w, g.csr()[3])
+    g.close()
+
+
+@pytest.mark.parametrize("wf", [N.WF_BF16, N.WF_FP8])
+def test_decoded_weights_in_parts(wf):
+    """2^24 + 4321 synapses: two parts, the border inside a row, empty rows and one of a single
+    synapse beside it."""
+    s = (1 << 24) + 4321
+    n = 3000
+    print(f"case: {s} synapses, weight_format={wf}", flush=True)
+    rng = np.random.default_rng(9)
+    src, tar = np.sort(rng.integers(0, n, s, dtype=np.int32)), rng.integers(0, n, s, dtype=np.int32)
+    src[(src >= 1200) & (src < 1300)] = 1300         # empty rows
+    at = src[1 << 24]
+    src[src == at - 1] = at                          # one before the border, and one after
+    last = src[-1]
+    src[-1] = n - 1
+    src[-2:-1] = last
+    w = rng.choice(np.float32([1.0, 0.25, -0.5, -1.0, 0.125]), s)   # (448 times these: E4M3 values)
+    w[np.unique(src, return_index=True)[1]] = 1.0    # row maximum 1
+    g = N.Simulator.from_arrays([N.LIF] * n, [0.0] * n, M.config1().lifconst, src, tar, w, np.full(s, np.float32(1e-3)),
+                                weight_format=wf)
+    want = w[np.argsort(src, kind="stable")]
+    assert np.array_equal(g.weights(), want)
+    g.close()
