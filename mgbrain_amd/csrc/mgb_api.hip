@@ -380,7 +380,6 @@ mgb_status choose_tiles(mgb_sim* s, const mgb_opts* o, int32_t n, int32_t D, con
     int lds_max = 65536;
     (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, s->device);
     lds_max = std::min(lds_max, 160 * 1024);
-    // the kernel's static LDS (block scan sums, event counter) shares the limit
     // (per target: the difference over 4 targets, which no alignment rounds; STDP keeps at
     // least one entry of each table in LDS)
     const int lut1 = stdp_kind(s->tkind) ? 1 : 0;
@@ -1287,6 +1286,7 @@ mgb_status setup_state(mgb_sim* s, const HostNeurons& h, const mgb_opts* o) {
         s->spin_limit = us * (uint64_t)khz / 1000ull;
     }
     if (s->tiled) {
+        MGB_HIP_TRY(check_tiled_lds(s->tkind, s->chunk));
         update_persist(s);
         if (s->tblock_auto && s->tblock > 512 && !stdp_kind(s->tkind) && s->persist_req != MGB_PERSIST_OFF) {
             // Two workgroups of 512 may fit on a CU where one of more does: 512 where only
@@ -2076,6 +2076,7 @@ mgb_status mgb_set_launch(mgb_sim* s, int32_t block, int32_t chunk) {
         return MGB_ERR_INVALID;
     }
     MGB_TRY(mgb_sync(s));
+    if (s->tiled && chunk > 0) MGB_HIP_TRY(check_tiled_lds(s->tkind, chunk));
     if (block > 0) {
         if (s->tiled) s->tblock = block;
         else s->prop_block = block;

@@ -344,6 +344,8 @@ hipError_t launch_tiled_persistent(const TiledArgs& a, int32_t off, int32_t wk, 
 hipError_t launch_finalize_tiled(Ctl* ctl, int32_t steps, int32_t windows, int32_t last, const uint32_t* err,
                                  HostMirror* m, hipStream_t st);
 hipError_t set_tiled_lds_limit(int kind, size_t bytes);
+// An error if a form of the fused kernel has LDS of its own.
+hipError_t check_tiled_lds(int kind, int chunk);
 // kTStdp: brings the plastic in-synapses of the neurons the fused kernel listed
 // in window base_window + wk up to date (flush of deferred dendrite updates).
 hipError_t launch_stdp_flush(const TiledArgs& a, int32_t off, int32_t wk, hipStream_t st);

@@ -2112,15 +2112,22 @@ hipError_t set_tiled_lds_limit(int kind, size_t bytes) {
             const void* f = tiled_fn_of(kind, chunk, pw != 0, pw == 2);
             if (!f) continue;
             const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-            if (e == hipSuccess) continue;
-            // the persistent form's own static LDS may not leave room for these tiles: it
-            // is then never resident, and never launched
-            if (pw) {
-                (void)hipGetLastError();
-                continue;
-            }
-            return e;
+            if (e != hipSuccess) return e;
         }
+    return hipSuccess;
+}
+
+// Propagation takes a synapse's byte offset in the ring slice for its LDS address, so the
+// launch's LDS has to begin at 0: a __shared__ variable anywhere in the kernel would move it.
+hipError_t check_tiled_lds(int kind, int chunk) {
+    for (int pw = 0; pw < 3; ++pw) {
+        const void* f = tiled_fn_of(kind, chunk, pw != 0, pw == 2);
+        if (!f) continue;
+        hipFuncAttributes fa;
+        const hipError_t e = hipFuncGetAttributes(&fa, f);
+        if (e != hipSuccess) return e;
+        if (fa.sharedSizeBytes != 0) return hipErrorInvalidDeviceFunction;
+    }
     return hipSuccess;
 }
 
