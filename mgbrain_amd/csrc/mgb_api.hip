@@ -369,7 +369,7 @@ uint64_t host_u64(const void* p) {
 
 // Tile shape of the fused path.  Tiles never straddle a segment boundary and
 // never mix neuron types (one update path per tile).  Within a segment they are
-// balanced by weight — a neuron weighs its in-degree (StatArgs::in_bal) plus half the
+// balanced by weight — a neuron weighs its in-degree (StatArgs::indeg, low halves) plus half the
 // mean in-degree of the neurons that have one (its own update) — so tiles of neurons
 // without input (Poisson) are larger and the others share the synapses evenly.
 // A segment of Nq neurons gets at most max(ceil(Nq / B), its type runs) tiles
@@ -763,15 +763,15 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     Scratch X;
     // ---- statistics + delay quantisation --------------------------------------
     uint8_t* dq = nullptr;
-    uint32_t *flags = nullptr, *wcls = nullptr, *in_bal = nullptr, *in_more = nullptr, *in_pl = nullptr, *absmax = nullptr;
+    uint32_t *flags = nullptr, *wcls = nullptr, *in_pl = nullptr, *absmax = nullptr;
+    uint2* indeg = nullptr;
     int32_t* mm = nullptr;
     unsigned long long* npl = nullptr;
     MGB_TRY(X.get(&dq, S));
     MGB_TRY(X.get(&flags, 1));
     MGB_TRY(X.get(&mm, 2));
     MGB_TRY(X.get(&wcls, 2 * (size_t)n));
-    MGB_TRY(X.get(&in_bal, 2 * (size_t)n));
-    MGB_TRY(X.get(&in_more, 2 * (size_t)n));
+    MGB_TRY(X.get(&indeg, 2 * (size_t)n));
     MGB_TRY(X.get(&in_pl, (size_t)n));
     MGB_TRY(X.get(&npl, 1));
     std::vector<uint16_t> run_of;
@@ -787,8 +787,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_HIP_TRY(hipMemsetAsync(flags, 0, 4, st));
     MGB_HIP_TRY(hipMemcpyAsync(mm, mm_init, 8, hipMemcpyHostToDevice, st));
     MGB_HIP_TRY(hipMemsetAsync(wcls, 0xFF, 8 * (size_t)n, st));
-    MGB_HIP_TRY(hipMemsetAsync(in_bal, 0, 8 * (size_t)n, st));
-    MGB_HIP_TRY(hipMemsetAsync(in_more, 0, 8 * (size_t)n, st));
+    MGB_HIP_TRY(hipMemsetAsync(indeg, 0, 16 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(in_pl, 0, 4 * (size_t)n, st));
     MGB_HIP_TRY(hipMemsetAsync(absmax, 0, 4 * std::max<size_t>(nruns, 1), st));
     MGB_HIP_TRY(hipMemsetAsync(npl, 0, 8, st));
@@ -799,7 +798,7 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         a.plastic = h.stdp ? L.plastic : nullptr;
         a.seg = seg_dev;                                   // null for one run: absmax[0]
         a.dq = dq; a.flags = flags; a.min_d = mm; a.max_d = mm + 1;
-        a.wcls = wcls; a.in_bal = in_bal; a.in_more = in_more; a.in_pl = in_pl; a.absmax = absmax; a.n_plastic = npl;
+        a.wcls = wcls; a.indeg = indeg; a.in_pl = in_pl; a.absmax = absmax; a.n_plastic = npl;
         MGB_HIP_TRY(run_stats(a, st));
     }
     uint32_t hflags = 0;
@@ -812,10 +811,13 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
     MGB_HIP_TRY(hipMemcpyAsync(&hnpl, npl, 8, hipMemcpyDeviceToHost, st));
     std::vector<uint32_t> h_wcls(2 * (size_t)n), h_bal(2 * (size_t)n), h_indeg(2 * (size_t)n);
     MGB_HIP_TRY(hipMemcpyAsync(h_wcls.data(), wcls, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
-    MGB_HIP_TRY(hipMemcpyAsync(h_bal.data(), in_bal, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
-    MGB_HIP_TRY(hipMemcpyAsync(h_indeg.data(), in_more, 8 * (size_t)n, hipMemcpyDeviceToHost, st));
+    std::vector<uint2> h_in(2 * (size_t)n);
+    MGB_HIP_TRY(hipMemcpyAsync(h_in.data(), indeg, 16 * (size_t)n, hipMemcpyDeviceToHost, st));
     MGB_HIP_TRY(hipStreamSynchronize(st));
-    for (size_t k = 0; k < h_indeg.size(); ++k) h_indeg[k] += h_bal[k];
+    for (size_t k = 0; k < h_in.size(); ++k) {
+        h_bal[k] = h_in[k].x;
+        h_indeg[k] = h_in[k].x + h_in[k].y;
+    }
     if (hflags & kFlagBadId) {
         set_error("a synapse references a neuron id outside [0, %d)", n);
         return MGB_ERR_INVALID;
@@ -977,8 +979,8 @@ mgb_status build_network(mgb_sim* s, const HostNeurons& h, const DevList& L, int
         MGB_HIP_TRY(hipStreamSynchronize(st));
     } else {
         // Fixed-point scale per segment: a power of two with in-degree * max |w| < 2^31, the
-        // in-degree by its part in_bal (for lists that are not in target order the whole of
-        // it: a batched network gets the scale it has alone).  Where that could let a
+        // in-degree by its first part (StatArgs::indeg; for lists that are not in target
+        // order the whole of it: a batched network gets the scale it has alone).  Where that could let a
         // target's inputs of one sign leave int32, fit_scales below lowers it
         const std::vector<int32_t>& slo = s->h_seg_lo;
         const size_t nseg = slo.size() - 1;

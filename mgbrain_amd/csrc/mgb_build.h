@@ -26,11 +26,11 @@ struct StatArgs {
     int32_t* min_d;
     int32_t* max_d;
     uint32_t* wcls;         // [2][n] class weight bits per target
-    // [2][n] in-degree per target and class, in two parts: in_bal counts a wave of 64 synapses
-    // of one target and class (target-major lists) as one, in_more has its other 63.  Tile
-    // boundaries, which saved checkpoints rest on, balance by the first part alone
-    uint32_t* in_bal;
-    uint32_t* in_more;
+    // [2][n] in-degree per target and class, in two parts of a word (one atomic for both): the
+    // low half counts a wave of 64 synapses of one target and class (target-major lists) as
+    // one, the high half has its other 63.  Tile boundaries, which saved checkpoints rest on,
+    // balance by the first part alone
+    uint2* indeg;
     uint32_t* in_pl;        // [n] plastic in-degree
     uint32_t* absmax;       // max |w| (float bits)
     unsigned long long* n_plastic;

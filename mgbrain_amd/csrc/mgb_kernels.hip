@@ -49,17 +49,14 @@ __device__ __forceinline__ float fp8e4m3_to_f32(uint8_t b) {
     return __uint_as_float(s | ((e + 120u) << 23) | (m << 20));
 }
 
-// s mod D and k mod 3 of a step or window index (>= 0) in 32-bit arithmetic: the 64-bit
-// remainder is a sequence of well over a hundred instructions, and every workgroup
-// needs these before its first load of a window.
+// s mod D of a step (>= 0) in 32-bit arithmetic: the 64-bit remainder is a sequence of well
+// over a hundred instructions, and every workgroup needs it before its first load of a
+// window.
 __device__ __forceinline__ int32_t mod_ring(int64_t s, int32_t D) {
     const uint32_t hi = (uint32_t)((uint64_t)s >> 32), lo = (uint32_t)s, d = (uint32_t)D;
     if (hi == 0u) return (int32_t)(lo % d);
     const uint32_t r32 = (0xFFFFFFFFu % d + 1u) % d;       // 2^32 mod D (D <= 128: no overflow below)
     return (int32_t)(((hi % d) * r32 + lo % d) % d);
-}
-__device__ __forceinline__ int mod3(int64_t k) {           // 2^32 = 1 mod 3
-    return (int)(((uint32_t)((uint64_t)k >> 32) % 3u + (uint32_t)k % 3u) % 3u);
 }
 
 // Inclusive prefix sum over the wave, in data-parallel moves: rows of 16 lanes, then the

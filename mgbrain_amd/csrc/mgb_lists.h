@@ -14,6 +14,12 @@
 
 namespace mgb {
 
+// The list of window k (>= 0): k mod 3 in 32-bit arithmetic (2^32 = 1 mod 3; the 64-bit
+// remainder takes well over a hundred instructions on the device).
+MGB_HD int mod3(int64_t k) {
+    return (int)(((uint32_t)((uint64_t)k >> 32) % 3u + (uint32_t)k % 3u) % 3u);
+}
+
 // First step of the window before the one that starts at s0, whose list is b (0, 1, 2), in
 // the first window of a launch: prev_len steps earlier, or (0) by the words.  All three load,
 // then b picks one: b comes from a load of its own.
@@ -27,7 +33,7 @@ MGB_HD int64_t window_before(const int64_t* tbase, int b, int64_t s0, int32_t pr
 // base_window on, whose last window had `last` steps.
 MGB_HD void end_run(int64_t* tbase, int64_t base_step, int64_t base_window, int32_t steps, int32_t windows,
                     int32_t last) {
-    tbase[(base_window + windows - 1) % 3] = base_step + steps - last;
+    tbase[mod3(base_window + windows - 1)] = base_step + steps - last;
 }
 
 }  // namespace mgb

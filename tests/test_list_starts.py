@@ -28,7 +28,7 @@ static int runs(const std::vector<int>& lengths, int window, bool persistent, co
         auto launch = [&](int nwin, int nst) {
             for (int q : order) {
                 const int64_t s0 = base + off;
-                wrong += mgb::window_before(tb, (int)((win + wk + 2) % 3), s0, prev) != s0 - before;
+                wrong += mgb::window_before(tb, mgb::mod3(win + wk + 2), s0, prev) != s0 - before;
 #ifdef SHARED
                 if (q == 0)
                     for (int k = 0; k < nwin; ++k) tb[(win + wk + k) % 3] = s0 + (int64_t)k * nst;
@@ -48,6 +48,9 @@ static int runs(const std::vector<int>& lengths, int window, bool persistent, co
 }
 int main() {
     int wrong = 0, n = 0;
+    for (int64_t k = 0; k < 1000; ++k)
+        for (int64_t at : {(int64_t)0, ((int64_t)1 << 32) - 500, ((int64_t)1 << 40) + 7, (int64_t)0x7FFFFFFFFFFFF000})
+            wrong += mgb::mod3(at + k) != (int)((at + k) % 3);
     for (int nseg = 1; nseg <= 4; ++nseg) {
         std::vector<int> order(nseg);
         std::iota(order.begin(), order.end(), 0);
