@@ -162,8 +162,7 @@ __global__ void k_tile_keys(const int32_t* src, const int32_t* tar, const float*
     }
 }
 
-// 16-bit CLASS words (tiles of at most 1024 targets): tile-local target |
-// delay-1 << 10 | inhibitory << 15, from the 32-bit words in tile order.
+// Spike records (step << 32 | id) into their two columns.
 __global__ void k_split_records(const uint64_t* r, uint64_t n, int32_t* steps, int32_t* ids) {
     for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
          k += (uint64_t)gridDim.x * blockDim.x) {
@@ -173,6 +172,8 @@ __global__ void k_split_records(const uint64_t* r, uint64_t n, int32_t* steps, i
     }
 }
 
+// 16-bit CLASS words (tiles of tn <= 1024 targets): (delay - 1) * tn + tile-local target, the
+// synapse's place in the ring slice, | inhibitory << 15; from the 32-bit words in tile order.
 __global__ void k_class16(const uint32_t* w32, uint64_t S, TileTabs tt, uint16_t* out) {
     for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < S;
          k += (uint64_t)gridDim.x * blockDim.x) {
