@@ -152,6 +152,7 @@ struct mgb_sim {
     int region = 0;                    // persistent launches: spikes with the flags (TiledArgs::region)
     uint64_t tile_hash = 0;            // FNV-1a of the tile boundaries (the ring slices' layout)
     uint64_t scale_hash = 0;           // of the fixed-point scales that fit_scales lowered (0: none)
+    std::vector<int32_t> scale_drop;   // [nseg] bits it lowered them by (empty: none)
     // host mirrors for read-back
     std::vector<float> class_w;        // [n_tbl][2]
     std::vector<uint16_t> h_tbl;       // [n]
@@ -693,8 +694,8 @@ std::vector<int32_t> stream_runs(const HostNeurons& h, std::vector<uint16_t>& ru
 // ever have, keep the scale that holds what arrives when all sources fire in one step: the
 // whole of a neuron's inputs, of any delay, would take 2 to 4 bits more (and their results
 // with them), for sums that only sources timed to cancel the delays could reach.  A scale
-// that is lowered joins the layout that a checkpoint has to match, its ring
-// words being multiples of 1 / scale.
+// that is lowered joins the layout that a checkpoint has to match, its ring words being
+// multiples of 1 / scale (ckpt_rescale takes those of the scale before).
 mgb_status fit_scales(mgb_sim* s, const HostNeurons& h, const DevList& L, const uint8_t* dq,
                       const std::vector<uint32_t>& indeg, const std::vector<float>& w_seg, const uint16_t* seg, std::vector<float2>& sc) {
     const size_t n = (size_t)h.n, nseg = sc.size();
@@ -740,6 +741,8 @@ mgb_status fit_scales(mgb_sim* s, const HostNeurons& h, const DevList& L, const 
             const int by = std::max(1, (int)std::ceil(std::log2((double)m / kMax)));
             const int e = std::max(-100, std::ilogb(sc[q].x) - by);
             sc[q] = make_float2(std::ldexp(1.0f, e), std::ldexp(1.0f, -e));
+            s->scale_drop.resize(nseg, 0);
+            s->scale_drop[q] += std::ilogb(now[q]) - e;
             s->scale_hash = (s->scale_hash ^ (((uint64_t)q << 32) | (uint32_t)(e + 128))) * 1099511628211ull + 1ull;
             fits = false;
         }
@@ -2385,6 +2388,28 @@ CkptHeader ckpt_header(const mgb_sim* s, uint64_t n_rec) {
     return h;
 }
 
+// Ring words saved before the scales of fit_scales were lowered (by a build that did not),
+// in the units of now: divided by 2^drop, to the nearest.
+void ckpt_rescale(const mgb_sim* s, const void* ring, int32_t* w) {
+    auto to_units = [](int32_t v, int32_t drop) {
+        return drop ? (int32_t)(((int64_t)v + (1ll << (drop - 1))) >> drop) : v;
+    };
+    const size_t nseg = s->scale_drop.size();
+    for (size_t q = 0; q < nseg; ++q) {
+        const int32_t drop = s->scale_drop[q];
+        if (ring == s->ring_t) {
+            const size_t k0 = (size_t)s->h_seg_tile0[q] * s->ring_slab, k1 = (size_t)s->h_seg_tile0[q + 1] * s->ring_slab;
+            for (size_t k = k0; k < k1; ++k) w[k] = to_units(w[k], drop);
+        } else {
+            for (int32_t d = 0; d < s->D; ++d)
+                for (int32_t i = s->h_seg_lo[q]; i < s->h_seg_lo[q + 1]; ++i) {
+                    int32_t& x = w[(size_t)d * (size_t)s->npad + (size_t)i];
+                    x = to_units(x, drop);
+                }
+        }
+    }
+}
+
 mgb_status ckpt_records(mgb_sim* s, uint64_t* n_rec) {
     const Ctl c = s->mir->ctl;
     *n_rec = std::min<uint64_t>(c.rec_cnt, (uint64_t)s->rec_cap);
@@ -2446,10 +2471,12 @@ mgb_status mgb_checkpoint_load(mgb_sim* s, const void* buf, int64_t bytes) {
         return MGB_ERR_CAPACITY;
     }
     const CkptHeader want = ckpt_header(s, (uint64_t)h.n_rec);
+    const bool old_units = s->scale_hash != 0 && h.tiling == s->tile_hash;
     if (h.n != want.n || h.npad != want.npad || h.D != want.D || h.window != want.window ||
         h.tiled != want.tiled || h.tkind != want.tkind || h.B != want.B || h.G != want.G ||
         h.nseg != want.nseg || h.mode != want.mode || h.wide_kind != want.wide_kind ||
-        h.stdp != want.stdp || h.S != want.S || h.payload != want.payload || h.tiling != want.tiling) {
+        h.stdp != want.stdp || h.S != want.S || h.payload != want.payload ||
+        (h.tiling != want.tiling && !old_units)) {
         set_error("checkpoint layout differs from this simulator (build it from the same network and "
                   "options)");
         return MGB_ERR_INVALID;
@@ -2462,7 +2489,14 @@ mgb_status mgb_checkpoint_load(mgb_sim* s, const void* buf, int64_t bytes) {
     const uint8_t* in = static_cast<const uint8_t*>(buf);
     size_t off = sizeof(h);
     for (const CkptSeg& g : ckpt_segments(s, (uint64_t)h.n_rec)) {
-        if (g.bytes) MGB_HIP_TRY(hipMemcpy(g.p, in + off, g.bytes, hipMemcpyHostToDevice));
+        if (old_units && g.p && (g.p == s->ring_t || g.p == s->ring_e || g.p == s->ring_i)) {
+            std::vector<int32_t> w(g.bytes / 4);
+            std::memcpy(w.data(), in + off, g.bytes);
+            ckpt_rescale(s, g.p, w.data());
+            MGB_HIP_TRY(hipMemcpy(g.p, w.data(), g.bytes, hipMemcpyHostToDevice));
+        } else if (g.bytes) {
+            MGB_HIP_TRY(hipMemcpy(g.p, in + off, g.bytes, hipMemcpyHostToDevice));
+        }
         off += g.bytes;
     }
     MGB_HIP_TRY(hipMemcpy(&s->mir->ctl, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));

@@ -181,3 +181,48 @@ def test_a_volley_of_plastic_inputs(wf):
     assert 60 < most < 150
     assert most * round(float(sc[4]) * s.info()["fix_scale_exc"]) <= 2**31 - 1
     s.close()
+
+
+@pytest.mark.parametrize("prop", [N.PROP_TILED, N.PROP_DIRECT])
+def test_checkpoint_from_before_the_scale_was_lowered(prop):
+    """A checkpoint whose pending inputs are in the units of in_bal * max |w| (in_bal: 10 for
+    the 10 waves of 640 synapses) loads, its ring words brought to the units of now."""
+    k, w = 640, float(np.float32(1.7e-6))
+    net = _driven(k, w)
+    net["pops"][0]["rate"] = 0.002                             # few enough for the old units
+    make = lambda: N.Simulator.generated(**net, weight_format=N.WF_F32, propagation=prop)
+    a, b, c = make(), make(), make()
+    drop = int(np.floor(np.log2(2147483520.0 / (10 * w)))) - int(np.log2(a.info()["fix_scale_exc"]))
+    _say(f"case: propagation={prop}, scale lowered by {drop} bits")
+    assert drop >= 5
+    a.run(133)
+    blob = np.frombuffer(bytes(a.checkpoint()), np.uint8).copy()
+    head = blob[8:60].view(np.int32)
+    n, npad, D, window, tiled, G = (int(head[i]) for i in (1, 2, 3, 4, 5, 8))
+    assert n == 1000 and tiled == (prop == N.PROP_TILED)
+    at = 96 + 24 * npad + 72 + 4 * (3 if tiled else 2) * npad * window
+    if tiled:
+        slab = (D * int(head[7]) + 3) // 4 * 4                  # (LIFB neurons: one ring)
+        words = G * slab
+        h = 1469598103934665603
+        for v in a.tiles():
+            h = (h ^ int(v)) * 1099511628211 % 2**64
+    else:
+        words, h = 2 * D * npad, 0
+    ring = blob[at:at + 4 * words].view(np.int32)
+    assert np.count_nonzero(ring) > 1000 and np.abs(ring.astype(np.int64)).max() < 2**31 >> drop
+    ring <<= drop
+    old = blob[88:96].view(np.uint64)
+    assert int(old[0]) != h
+    old[0] = h
+    b.restore(blob.tobytes())
+    with pytest.raises(N.MGBError):                             # (neither tiling)
+        old[0] = h ^ 1
+        c.restore(blob.tobytes())
+    a.run(200)
+    b.run(200)
+    assert a.state(N.F_V)[700:].min() > 1e-4
+    assert np.array_equal(a.state(N.F_V).view(np.uint32), b.state(N.F_V).view(np.uint32))
+    assert np.array_equal(a.fire_counts(), b.fire_counts())
+    for s in (a, b, c):
+        s.close()
