@@ -701,7 +701,8 @@ mgb_status fit_scales(mgb_sim* s, const HostNeurons& h, const DevList& L, const 
     const size_t n = (size_t)h.n, nseg = sc.size();
     const std::vector<int32_t>& lo = s->h_seg_lo;
     constexpr double kMax = 2147483647.0;
-    bool safe = h.fp8_scale.empty();       // (a caller's FP8 scale may round far above max |w|)
+    // (a caller's FP8 scale may round far above max |w|)
+    bool safe = s->wide_kind != kWideFP8 || h.fp8_scale.empty();
     for (size_t q = 0; q < nseg && safe; ++q) {
         uint32_t deg = 0;
         for (int32_t t = lo[q]; t < lo[q + 1]; ++t) deg = std::max(deg, indeg[t] + indeg[n + t]);

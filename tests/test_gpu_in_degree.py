@@ -226,3 +226,25 @@ def test_checkpoint_from_before_the_scale_was_lowered(prop):
     assert np.array_equal(a.fire_counts(), b.fire_counts())
     for s in (a, b, c):
         s.close()
+
+
+@pytest.mark.parametrize("prop", [N.PROP_TILED, N.PROP_DIRECT])
+def test_fp8_scales_whose_codes_round_up(prop):
+    """A caller's FP8 scale of w / 0.00110: the code is 2^-9, 1.78 times the weight.  The scale
+    of in-degree * max |w| holds 1.06 times it; w is such that little is left of int32."""
+    _say(f"case: 1000 inputs in every step, codes above the weights, propagation={prop}")
+    k, d = 1000, np.float32(1e-3)
+    w = np.float32(0.98 * 2.0**31 / 1.0625 / k / 2.0**40)
+    scale = np.float32(w / np.float32(0.0011))
+    src, tar = np.repeat(np.arange(k), 2), np.tile([k, k + 1], k)       # (in source order)
+    s = N.Simulator.from_arrays([N.POISSON] * k + [N.LIFB] * 2, [1.0] * k + [0.0] * 2, W.lifb_consts(), src, tar,
+                                np.full(2 * k, w), np.full(2 * k, d), weight_format=N.WF_FP8, propagation=prop,
+                                fp8_scale=np.full(k + 2, scale))
+    code = float(np.float32(2.0**-9) * scale)
+    assert np.all(s.weights() == np.float32(code)) and code > 1.7 * float(w)
+    at = s.info()["fix_scale_exc"]
+    assert at == 2.0**39 and k * round(code * at) <= 2**31 - 1
+    s.run(14)
+    want = _v_after(k * code, 4)
+    assert np.abs(s.state(N.F_V)[k:] - want).max() <= 4 * (0.5 * k / at + 4 * 2.0**-24 * want)
+    s.close()
