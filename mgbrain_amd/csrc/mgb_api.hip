@@ -1386,7 +1386,8 @@ void update_persist(mgb_sim* s) {
     // Spikes that pass with the wait's flags (grid_exchange) wherever a tile's mostly fit
     // there: without Poisson tiles whose rates alone say that they do not (80,000
     // conductance neurons 8.71 -> 8.40 us a window, 20,000 in BF16 8.16 -> 7.50, 5,000 7.3 -> 6.8;
-    // with busy Poisson tiles, 5,000 and 11,000 neurons 8.0 -> 8.7 and 9.0 -> 9.9, by lists).  16-bit
+    // with busy Poisson tiles, 5,000 and 11,000 neurons 8.0 -> 8.7 and 9.0 -> 9.9, by lists; busy
+    // integrating neurons, whose rates are not known here, lose the same).  16-bit
     // CLASS words also when asked for, and in networks of windows of many spikes, where
     // regions beat lists by themselves.  One thread per tile scans the regions' counts, and the
     // LDS holds them beside the tile's data with every workgroup still resident
