@@ -128,7 +128,8 @@ def test_decoded_weights_in_parts(wf):
     w = rng.choice(np.float32([1.0, 0.25, -0.5, -1.0, 0.125]), s)   # (448 times these: E4M3 values)
     w[np.unique(src, return_index=True)[1]] = 1.0    # row maximum 1
     g = N.Simulator.from_arrays([N.LIF] * n, [0.0] * n, M.config1().lifconst, src, tar, w, np.full(s, np.float32(1e-3)),
-                                weight_format=wf)
+                                weight_format=wf, propagation=N.PROP_DIRECT, stdp=True, plastic=(tar % 7 == 0),
+                                stdpconst=M.stdp_consts_config4(J=1e-4))
     want = w[np.argsort(src, kind="stable")]
     assert np.array_equal(g.weights(), want)
     g.close()
